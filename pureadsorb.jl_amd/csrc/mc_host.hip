@@ -28,7 +28,7 @@ struct pa_state {
     std::vector<double> const_p, const_q;  // exchange constant term, eV (src/moves.jl:728-773)
     std::vector<int> acc_at_audit;         // accepted moves per system at the last audit
     int64_t samp_stride = 0;               // production samples per system of the last GCMC run
-    DevAlloc d_guest_off, d_occ, d_refpos, d_quat, d_host_e, d_Sk, d_dS, d_skabs, d_sk_off, d_energy, d_energy_abs,
+    DevAlloc d_guest_off, d_occ, d_refpos, d_quat, d_host_e, d_Sk, d_skabs, d_sk_off, d_energy, d_energy_abs,
         d_seed, d_counter, d_acc, d_att, d_step_t, d_step_r, d_fug, d_cp, d_cq, d_samp_e, d_samp_n, d_maxocc,
         d_caphit, d_trace;
     // NVT driver: fractional atom table, insertion constant per system, move-launch snapshots,
@@ -36,6 +36,10 @@ struct pa_state {
     DevAlloc d_atomf64, d_atype_s, d_chunk, d_chunk_off, d_lines, d_rounds, d_round_off, d_perm, d_coff,
         d_half_perp, d_ct, d_snap_pos, d_snap_quat, d_snap_sk, d_snap_occ, d_item_off, d_cw_dU, d_pose_pos,
         d_pose_quat;
+    // the k-vectors' order on the device (KRuns): position of every k-vector within its framework's
+    // slice, and the runs
+    std::vector<int> kpos;
+    DevAlloc d_run, d_run_off, d_kbase, d_kblk_off, d_kw;
     // the audit's device rebuild: per-axis power tables, structure factor, per-slot host-guest
     // energies, per-system sums
     DevAlloc d_aud_tab, d_aud_sk, d_aud_he, d_aud_sums;
@@ -61,6 +65,7 @@ struct pa_state {
 namespace {
 
 int ensure_chain_tables(pa_state *st);
+int build_k_runs(pa_state *st);
 
 // Entry points that read the guest slots (or launch kernels over them) refuse a state whose
 // occupancy a test put above a capacity.
@@ -277,8 +282,8 @@ McArgs base_mc(pa_state *st)
     a.atomf = st->d_atomf64.as<double4>();
     a.atypef = st->d_atype_s.as<int>();
     a.upper = b->upper_all ? 1 : 0;
-    a.k64 = b->d_k64.as<double4>();
-    a.kn = b->d_kn.as<int4>();
+    a.kr = KRuns{st->d_run.as<int4>(), st->d_run_off.as<int>(), st->d_kbase.as<int>(), st->d_kblk_off.as<int>(),
+                 st->d_kw.as<double>()};
     a.ktab_w = 0;
     for (const FwDesc &D : b->desc) a.ktab_w = std::max(a.ktab_w, D.kn_max[0] + D.kn_max[1] + D.kn_max[2] + 3);
     a.pair64 = b->d_pair64.as<double2>();
@@ -294,7 +299,6 @@ McArgs base_mc(pa_state *st)
     a.quat = st->d_quat.as<double4>();
     a.host_e = st->d_host_e.as<double>();
     a.Sk = st->d_Sk.as<double2>();
-    a.dS = st->d_dS.as<double2>();
     a.sk_abs = st->d_skabs.as<double>();
     a.sk_off = st->d_sk_off.as<int>();
     a.energy = st->d_energy.as<double>();
@@ -405,6 +409,7 @@ extern "C" int pa_state_create(pa_batch *b, const pa_guest *guest, const int32_t
     S->const_p.resize(nsys);
     S->const_q.resize(nsys);
     const double kT = KB * T;
+    if (int e = build_k_runs(S.get())) return e;
     // systems are independent: built on the host threads, each keeping its status and message
     auto build_system = [&](int n) -> int {
         const int u = b->fw_of[n];
@@ -447,7 +452,7 @@ extern "C" int pa_state_create(pa_batch *b, const pa_guest *guest, const int32_t
         }
         std::vector<double2> sk;
         rebuild_sk(b, u, pos, quat, S->guest_off[n], ncounts[n], sk);
-        std::copy(sk.begin(), sk.end(), Sk.begin() + S->sk_off[n]);
+        for (size_t k = 0; k < sk.size(); ++k) Sk[S->sk_off[n] + S->kpos[F.k_off + k]] = sk[k];
         std::vector<double> he;
         int st = total_energy_h(b, u, pos, quat, S->guest_off[n], ncounts[n], sk, &energy[n], &he);
         if (st) return st;
@@ -474,8 +479,7 @@ extern "C" int pa_state_create(pa_batch *b, const pa_guest *guest, const int32_t
     HIP_TRY(upload(S->d_quat, quat));
     HIP_TRY(upload(S->d_host_e, host_e));
     HIP_TRY(upload(S->d_Sk, Sk));
-    HIP_TRY(S->d_dS.ensure(sizeof(double2) * MC_SPEC * std::max<size_t>(Sk.size(), 1)));
-    HIP_TRY(upload(S->d_skabs, std::vector<double>(Sk.size(), 0.0)));
+    HIP_TRY(upload(S->d_skabs, std::vector<double>(nsys, 0.0)));
     HIP_TRY(upload(S->d_energy, energy));
     HIP_TRY(upload(S->d_energy_abs, std::vector<double>(nsys, 0.0)));
     HIP_TRY(upload(S->d_seed, S->seed));
@@ -640,7 +644,13 @@ extern "C" int pa_state_sk(const pa_state *st, int32_t sys, double *sk)
     if (sys < 0 || sys >= st->nsys) return fail(PA_ERR_ARG, "system index %d out of range 0..%d", sys, st->nsys - 1);
     const int nk = st->sk_off[sys + 1] - st->sk_off[sys];
     if (nk == 0) return ok();
-    HIP_TRY(hipMemcpy(sk, st->d_Sk.as<double2>() + st->sk_off[sys], sizeof(double2) * nk, hipMemcpyDeviceToHost));
+    std::vector<double2> v(nk);
+    HIP_TRY(hipMemcpy(v.data(), st->d_Sk.as<double2>() + st->sk_off[sys], sizeof(double2) * nk, hipMemcpyDeviceToHost));
+    const int *kpos = st->kpos.data() + st->b->desc[st->b->fw_of[sys]].k_off;
+    for (int k = 0; k < nk; ++k) {
+        sk[2 * k] = v[kpos[k]].x;
+        sk[2 * k + 1] = v[kpos[k]].y;
+    }
     return ok();
 }
 
@@ -741,7 +751,7 @@ extern "C" int pa_audit_energy(pa_state *st, double *discrepancy)
     HIP_TRY(download(Erun, st->d_energy, nsys));
     HIP_TRY(download(Eabs, st->d_energy_abs, nsys));
     HIP_TRY(download(skrun, st->d_Sk, std::max(1, nsk)));
-    HIP_TRY(download(skabs, st->d_skabs, std::max(1, nsk)));
+    HIP_TRY(download(skabs, st->d_skabs, nsys));
     HIP_TRY(download(acc, st->d_acc, (size_t)nsys * NMOVES));
     const double eps = DBL_EPSILON;
     auto tol = [&](double abs_accum, double mag, double nm) {
@@ -757,11 +767,12 @@ extern "C" int pa_audit_energy(pa_state *st, double *discrepancy)
         const FwDesc &F = b->desc[u];
         const double nterms = (double)occ[n] * NS;
         for (int k = 0; k < F.nk; ++k) {
-            const int j = st->sk_off[n] + k;
-            const double2 r = skrun[j], w = skr[j], h = b->S64_h[F.k_off + k];
+            // the rebuild is in the k tables' order, the running values by position
+            const double2 r = skrun[st->sk_off[n] + st->kpos[F.k_off + k]], w = skr[st->sk_off[n] + k],
+                          h = b->S64_h[F.k_off + k];
             const double mag = nterms * (std::hypot(h.x, h.y) + occ[n] * qabs);
             const double d = std::hypot(r.x - w.x, r.y - w.y);
-            const double tk = tol(skabs[j], mag, nmoves);
+            const double tk = tol(skabs[n], mag, nmoves);
             if (!(d <= tk))
                 return fail(PA_ERR_ARG,
                             "energy audit failed for system %d (Float64): structure factor at k-vector %d disagrees with "
@@ -787,8 +798,8 @@ extern "C" int pa_audit_energy(pa_state *st, double *discrepancy)
                         "energy audit failed for system %d (Float64): accumulated=%.17g, recomputed=%.17g, "
                         "discrepancy=%.17g exceeds tolerance %.17g over %.0f accepted move(s) since the last audit",
                         n + 1, Erun[n], E, d, te, nmoves);
-        std::copy(skr.begin() + st->sk_off[n], skr.begin() + st->sk_off[n + 1], skrun.begin() + st->sk_off[n]);
-        std::fill(skabs.begin() + st->sk_off[n], skabs.begin() + st->sk_off[n + 1], 0.0);
+        for (int k = 0; k < F.nk; ++k) skrun[st->sk_off[n] + st->kpos[F.k_off + k]] = skr[st->sk_off[n] + k];
+        skabs[n] = 0.0;
         Erun[n] = E;
         Eabs[n] = 0.0;
         st->acc_at_audit[n] = nacc;
@@ -815,7 +826,8 @@ extern "C" int pa_state_set_value(pa_state *st, int32_t field, int32_t sys, int6
         const int nk = st->sk_off[sys + 1] - st->sk_off[sys];
         if (index < 0 || index >= nk) return fail(PA_ERR_ARG, "k-vector index %lld out of range 0..%d", (long long)index, nk - 1);
         const double2 v = make_double2(re, im);
-        HIP_TRY(hipMemcpy(st->d_Sk.as<double2>() + st->sk_off[sys] + index, &v, sizeof(double2), hipMemcpyHostToDevice));
+        const int at = st->kpos[st->b->desc[st->b->fw_of[sys]].k_off + (int)index];
+        HIP_TRY(hipMemcpy(st->d_Sk.as<double2>() + st->sk_off[sys] + at, &v, sizeof(double2), hipMemcpyHostToDevice));
         return ok();
     }
     case PA_FIELD_HOST_ENERGY: {
@@ -1094,6 +1106,56 @@ uint32_t spread3(uint32_t v)
     return v;
 }
 
+// The order in which the device keeps and visits the k-vectors of a chain (KRuns): the runs of
+// consecutive n3 at fixed (n1, n2) in k-table order, longest first.
+int build_k_runs(pa_state *st)
+{
+    const pa_batch *b = st->b;
+    const size_t nkt = std::max<size_t>(b->k64_h.size(), 1);
+    std::vector<int4> run;
+    std::vector<int> run_off(1, 0), base, blk_off(1, 0);
+    std::vector<double> kw(nkt, 0.0);
+    st->kpos.assign(nkt, 0);
+    for (int u = 0; u < b->nfw; ++u) {
+        const FwDesc &F = b->desc[u];
+        const int4 *kn = b->kn_h.data() + F.k_off;
+        std::vector<int2> fl;  // first k-vector, length
+        for (int k = 0; k < F.nk; ++k) {
+            if (k > 0 && kn[k].x == kn[k - 1].x && kn[k].y == kn[k - 1].y && kn[k].z == kn[k - 1].z + 1) ++fl.back().y;
+            else fl.push_back(make_int2(k, 1));
+        }
+        std::stable_sort(fl.begin(), fl.end(), [](const int2 &x, const int2 &y) { return x.y > y.y; });
+        int pos = 0;
+        for (size_t r0 = 0; r0 < fl.size(); r0 += 64) {
+            base.push_back(pos);
+            const size_t r1 = std::min(fl.size(), r0 + 64);
+            auto put = [&](size_t r, int off) {
+                st->kpos[F.k_off + fl[r].x + (fl[r].y - 1) / 2 + off] = pos;
+                kw[F.k_off + pos] = b->k64_h[F.k_off + fl[r].x + (fl[r].y - 1) / 2 + off].w;
+                ++pos;
+            };
+            for (size_t r = r0; r < r1; ++r) {
+                const int4 n = kn[fl[r].x];
+                run.push_back(make_int4(n.x, n.y, n.z + (fl[r].y - 1) / 2, fl[r].y));
+                put(r, 0);
+            }
+            for (int j = 1; 2 * j <= fl[r0].y; ++j) {
+                for (size_t r = r0; r < r1 && 2 * j <= fl[r].y; ++r) put(r, j);
+                for (size_t r = r0; r < r1 && 2 * j + 1 <= fl[r].y; ++r) put(r, -j);
+            }
+        }
+        if (pos != F.nk) return fail(PA_ERR_INTERNAL, "framework %d: %d of %d k-vectors placed", u + 1, pos, F.nk);
+        run_off.push_back((int)run.size());
+        blk_off.push_back((int)base.size());
+    }
+    HIP_TRY(upload(st->d_run, run));
+    HIP_TRY(upload(st->d_run_off, run_off));
+    HIP_TRY(upload(st->d_kbase, base));
+    HIP_TRY(upload(st->d_kblk_off, blk_off));
+    HIP_TRY(upload(st->d_kw, kw));
+    return PA_OK;
+}
+
 // Tables of the chain-insertion kernel, built once per state: every framework's atoms in
 // Morton order of a ~4 Å cell grid, cut into chunks of 64 with a centre and a radius that
 // bounds every atom's nearest-image distance to the centre; the k-vectors cut into runs of
@@ -1201,7 +1263,14 @@ int ensure_chain_tables(pa_state *st)
     HIP_TRY(upload(st->d_lines, lines));
     HIP_TRY(upload(st->d_rounds, rounds));
     HIP_TRY(upload(st->d_round_off, round_off));
-    HIP_TRY(upload(st->d_perm, perm));
+    // by position, as the running structure factors are stored
+    std::vector<int> perm_pos(perm.size(), 0);
+    for (int u = 0; u < b->nfw; ++u)
+        for (int k = 0; k < b->desc[u].nk; ++k) {
+            const int k0 = b->desc[u].k_off;
+            perm_pos[k0 + st->kpos[k0 + k]] = perm[k0 + k];
+        }
+    HIP_TRY(upload(st->d_perm, perm_pos));
     std::vector<int> coff(st->nsys + 1, 0);
     for (int n = 0; n < st->nsys; ++n) coff[n + 1] = coff[n] + fsize[b->fw_of[n]];
     st->ctot = coff[st->nsys];

@@ -11,11 +11,11 @@
 //   * the guest-guest real-space change over (other guest, site, site) triples
 //     (guest_guest_move_delta / guest_pair_realspace_energy_range, src/guest.jl:112-156),
 //   * the reciprocal change over the k-vectors against the running structure factor
-//     (_reciprocal_move_delta_k, src/guest.jl:228-238), keeping each lane's dS(k) for the
-//     update on acceptance;
+//     (_reciprocal_move_delta_k, src/guest.jl:228-238), evaluated again for the update on
+//     acceptance;
 // reduces them through LDS, and every work-item takes the same Metropolis decision
-// (src/moves.jl:198-246). Work-item 0 commits poses and occupancy; each lane applies its own
-// k-vectors' dS to the running structure factor. Everything is FP64.
+// (src/moves.jl:198-246). Work-item 0 commits poses and occupancy; the workgroup applies the
+// changes to the running structure factor. Everything is FP64.
 #include "pa_device.hpp"
 
 namespace pa {
@@ -70,10 +70,13 @@ __global__ __launch_bounds__(MC_WG) void mc_chain_kernel(McArgs a)
     const int n = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const FwDesc &F = a.fw[a.fw_of[n]];
     const int gr0 = a.guest_off[n], cap = a.guest_off[n + 1] - gr0, nslots = a.guest_off[a.nsys];
-    const double4 *ks = a.k64 + F.k_off;
+    const int u = a.fw_of[n];
+    const double *kw = a.kr.kw + F.k_off;
+    const int4 *runs = a.kr.run + a.kr.run_off[u];
+    const int *kbase = a.kr.base + a.kr.blk_off[u];
+    const int nruns = a.kr.run_off[u + 1] - a.kr.run_off[u], nkblk = a.kr.blk_off[u + 1] - a.kr.blk_off[u];
     double2 *Sk = a.Sk + a.sk_off[n];
-    double2 *dS = a.dS + (size_t)MC_SPEC * a.sk_off[n];   // MC_SPEC slices of nk
-    double *skabs = a.sk_abs + a.sk_off[n];
+    double skabs = a.sk_abs[n];
     const int nk = F.nk, natoms = F.natoms;
     const GuestDev &G = a.guest;
     const double alpha = F.alpha;
@@ -107,7 +110,63 @@ __global__ __launch_bounds__(MC_WG) void mc_chain_kernel(McArgs a)
     const int gi = tid / MC_GW, gt = tid - gi * MC_GW;
     const int m0 = F.kn_max[0] + 1, m1 = F.kn_max[1] + 1, tw = m0 + m1 + F.kn_max[2] + 1;
     double2 *mytab = ktab + (size_t)gi * 2 * NS * tw;
-    double2 *mydS = dS + (size_t)gi * nk;
+
+    // Visits the k-vectors' structure-factor changes of one attempt (its phase tables at `tab`):
+    // use(active, position, Re dS, Im dS), the blocks of 64 runs dealt to `nw` wavefronts in
+    // snake order (they get shorter), this one being `w`. One complex product of table entries per
+    // run and site starts it; a pair of k-vectors m +- j then takes 4 fused multiply-adds per
+    // site and pose for both. Per k-vector that is 12 FP64 instructions for a 3-site guest's
+    // old and new pose, where two complex products per site and k-vector took about 120.
+    auto visit_k = [&](const double2 *tab, bool ho, bool hn, int w, int nw, auto &&use) {
+        for (int r = 0; r * nw < nkblk; ++r) {
+            const int blk = r * nw + ((r & 1) ? nw - 1 - w : w);
+            if (blk >= nkblk) continue;
+            const int ri = blk * 64 + lane;
+            const int4 run = ri < nruns ? runs[ri] : make_int4(0, 0, 0, 0);
+            const int L = run.w;
+            int pos = __builtin_amdgcn_readfirstlane(kbase[blk]);
+            double er[2][NS], ei[2][NS], sre = 0.0, sim = 0.0;
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+                if (!(p ? hn : ho)) continue;
+#pragma unroll
+                for (int s = 0; s < NS; ++s) {
+                    const double2 *tb = tab + (p * NS + s) * tw;
+                    const double2 cc = cis_from_axes(tb[abs(run.x)], tb[m0 + abs(run.y)], tb[m0 + m1 + abs(run.z)],
+                                                     run.x, run.y, run.z);
+                    const double q = p ? G.q[s] : -G.q[s];
+                    er[p][s] = q * cc.x;
+                    ei[p][s] = q * cc.y;
+                    sre += er[p][s];
+                    sim += ei[p][s];
+                }
+            }
+            use(L >= 1, pos + lane, sre, sim);
+            pos += __popcll(__builtin_amdgcn_ballot_w64(L >= 1));
+            const double2 *tz = tab + m0 + m1;
+            for (int j = 1;; ++j) {
+                const int np = __popcll(__builtin_amdgcn_ballot_w64(L >= 2 * j));
+                if (np == 0) break;
+                const int nm = __popcll(__builtin_amdgcn_ballot_w64(L >= 2 * j + 1));
+                double A = 0.0, B = 0.0, C = 0.0, D = 0.0;
+#pragma unroll
+                for (int p = 0; p < 2; ++p) {
+                    if (!(p ? hn : ho)) continue;
+#pragma unroll
+                    for (int s = 0; s < NS; ++s) {
+                        const double2 z = tz[(p * NS + s) * tw + j];
+                        A = __builtin_fma(er[p][s], z.x, A);
+                        B = __builtin_fma(ei[p][s], z.y, B);
+                        C = __builtin_fma(er[p][s], z.y, C);
+                        D = __builtin_fma(ei[p][s], z.x, D);
+                    }
+                }
+                use(lane < np, pos + lane, A - B, C + D);
+                use(lane < nm, pos + np + lane, A + B, D - C);
+                pos += np + nm;
+            }
+        }
+    };
 
     // cycle mode: a cycle of chain n is max(occupancy at its start, min_cycle) attempts, and its
     // sample is taken at its end. Called before every attempt; false once the run is over.
@@ -136,9 +195,8 @@ __global__ __launch_bounds__(MC_WG) void mc_chain_kernel(McArgs a)
         return true;
     };
 
-    // writes the pending snapshots: every work-item copies the structure-factor entries it
-    // updates itself on a commit (k = tid mod MC_WG) and a share of the guests, which work-item 0
-    // last wrote before a barrier
+    // writes the pending snapshots: the structure factor and the guests were last written before
+    // a barrier
     auto flush_snapshots = [&]() {
         for (int p = 0; p < npend; ++p) {
             const int64_t cs = pend[p];
@@ -146,7 +204,7 @@ __global__ __launch_bounds__(MC_WG) void mc_chain_kernel(McArgs a)
             double2 *dsk = S.csk + cs * S.ctot + S.coff[n];
             const int *perm = S.perm + F.k_off;
             for (int k = tid; k < nk; k += MC_WG) {
-                const double w = ks[k].w;
+                const double w = kw[k];
                 const double2 v = Sk[k];
                 dsk[perm[k]] = make_double2(w * v.x, w * v.y);
             }
@@ -309,46 +367,15 @@ __global__ __launch_bounds__(MC_WG) void mc_chain_kernel(McArgs a)
                     mytab[e] = axis_power(F.invA, pose ? ns[t] : os[t], d, m);
                 }
             __syncthreads();
-            const int4 *kn = a.kn + F.k_off;
-            if (active) {
-                // one chain's attempt is latency-bound: the next k-vector's loads are issued
-                // before the current one is evaluated
-                double kw_next = 0.0;
-                int4 nn_next = make_int4(0, 0, 0, 0);
-                double2 S_next = make_double2(0.0, 0.0);
-                if (gt < nk) {
-                    kw_next = ks[gt].w;
-                    nn_next = kn[gt];
-                    S_next = Sk[gt];
-                }
-#pragma unroll 1
-                for (int k = gt; k < nk; k += MC_GW) {
-                    const double kw = kw_next;
-                    const int4 nn = nn_next;
-                    const double2 S = S_next;
-                    if (k + MC_GW < nk) {
-                        kw_next = ks[k + MC_GW].w;
-                        nn_next = kn[k + MC_GW];
-                        S_next = Sk[k + MC_GW];
-                    }
-                    const int ax = abs(nn.x), ay = abs(nn.y), az = abs(nn.z);
-                    double sre = 0.0, sim = 0.0;
-#pragma unroll
-                    for (int pose = 0; pose < 2; ++pose) {
-                        if (pose == 1 ? !has_new : !has_old) continue;
-                        const double sg = pose == 1 ? 1.0 : -1.0;
-#pragma unroll
-                        for (int s = 0; s < NS; ++s) {
-                            const double2 *tb = mytab + (pose * NS + s) * tw;
-                            const double2 cc = cis_from_axes(tb[ax], tb[m0 + ay], tb[m0 + m1 + az], nn.x, nn.y, nn.z);
-                            sre += sg * G.q[s] * cc.x;
-                            sim += sg * G.q[s] * cc.y;
-                        }
-                    }
-                    mydS[k] = make_double2(sre, sim);
-                    rsum += kw * (2.0 * (S.x * sre + S.y * sim) + (sre * sre + sim * sim));
-                }
-            }
+            if (active)
+                visit_k(mytab, has_old, has_new, wid - gi * MC_GNW, MC_GNW,
+                        [&](bool on, int p, double sre, double sim) {
+                            const int k = on ? p : 0;
+                            const double2 S = Sk[k];
+                            const double w = on ? kw[k] : 0.0;
+                            rsum = __builtin_fma(w, __builtin_fma(sre, __builtin_fma(2.0, S.x, sre),
+                                                                  sim * __builtin_fma(2.0, S.y, sim)), rsum);
+                        });
         }
         hsum = wave_sum_d(hsum);
         gsum = wave_sum_d(gsum);
@@ -441,26 +468,17 @@ __global__ __launch_bounds__(MC_WG) void mc_chain_kernel(McArgs a)
             Eabs += fabs(dU);
             ++acc[ty - 1];
             if (G.charged) {
-                const double2 *fdS = dS + (size_t)first * nk;
-                double2 dd_next = make_double2(0.0, 0.0), S_next = make_double2(0.0, 0.0);
-                double sa_next = 0.0;
-                if (tid < nk) {
-                    dd_next = fdS[tid];
-                    S_next = Sk[tid];
-                    sa_next = skabs[tid];
-                }
-                for (int k = tid; k < nk; k += MC_WG) {
-                    const double2 dd = dd_next, S = S_next;
-                    const double sa = sa_next;
-                    if (k + MC_WG < nk) {  // other entries than the ones written below
-                        dd_next = fdS[k + MC_WG];
-                        S_next = Sk[k + MC_WG];
-                        sa_next = skabs[k + MC_WG];
-                    }
-                    Sk[k] = make_double2(S.x + dd.x, S.y + dd.y);
-                    skabs[k] = sa + ds_bound;
-                }
+                // the accepted attempt's changes, evaluated again from its tables (cheaper than
+                // writing and reading every attempt's)
+                visit_k(ktab + (size_t)first * 2 * NS * tw, ty != MOVE_INSERTION, ty != MOVE_DELETION, wid, MC_NW,
+                        [&](bool on, int p, double sre, double sim) {
+                            if (on) {
+                                const double2 S = Sk[p];
+                                Sk[p] = make_double2(S.x + sre, S.y + sim);
+                            }
+                        });
             }
+            skabs += ds_bound;
         }
         ctr += (uint64_t)done;
         __syncthreads();  // committed poses, red[] and the group records reused by the next round
@@ -499,6 +517,7 @@ __global__ __launch_bounds__(MC_WG) void mc_chain_kernel(McArgs a)
         a.occupancy[n] = occ;
         a.energy[n] = E;
         a.energy_abs[n] = Eabs;
+        a.sk_abs[n] = skabs;
         a.rng_counter[n] = ctr;
         for (int t = 0; t < NMOVES; ++t) {
             a.accepted[n * NMOVES + t] = acc[t];

@@ -217,19 +217,19 @@ __global__ __launch_bounds__(CW_WG, (NS <= 3 ? 4 : 1)) void chain_widom_kernel(C
 // Snapshot slot `slot` of every system's live state (after an audit, or for insertions at
 // caller poses): one workgroup per system.
 __global__ __launch_bounds__(256) void chain_snapshot_kernel(ChainSnap S, int64_t slot, const FwDesc *fw,
-                                                            const int *fw_of, const double4 *k64, const int *guest_off,
+                                                            const int *fw_of, const double *kw_all, const int *guest_off,
                                                             const int *sk_off, const int *occupancy,
                                                             const double4 *refpos, const double4 *quat,
                                                             const double2 *Sk)
 {
     const int n = blockIdx.x, tid = threadIdx.x;
     const FwDesc &F = fw[fw_of[n]];
-    const double4 *ks = k64 + F.k_off;
+    const double *kw = kw_all + F.k_off;
     const double2 *sk = Sk + sk_off[n];
     const int *perm = S.perm + F.k_off;
     double2 *dsk = S.csk + slot * S.ctot + S.coff[n];
     for (int k = tid; k < F.nk; k += 256) {
-        const double w = ks[k].w;
+        const double w = kw[k];
         const double2 v = sk[k];
         dsk[perm[k]] = make_double2(w * v.x, w * v.y);
     }
@@ -243,7 +243,7 @@ __global__ __launch_bounds__(256) void chain_snapshot_kernel(ChainSnap S, int64_
 
 hipError_t launch_chain_snapshot(const ChainSnap &S, int64_t slot, const McArgs &m, hipStream_t st)
 {
-    hipLaunchKernelGGL(chain_snapshot_kernel, dim3((unsigned)S.nsys), dim3(256), 0, st, S, slot, m.fw, m.fw_of, m.k64,
+    hipLaunchKernelGGL(chain_snapshot_kernel, dim3((unsigned)S.nsys), dim3(256), 0, st, S, slot, m.fw, m.fw_of, m.kr.kw,
                        m.guest_off, m.sk_off, m.occupancy, m.refpos, m.quat, m.Sk);
     return hipGetLastError();
 }

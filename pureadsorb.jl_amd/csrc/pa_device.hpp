@@ -220,13 +220,47 @@ __device__ inline double cw_r2(const double A[9], double f0, double f1, double f
     return cw_r2_t<false>(A, f0, f1, f2);
 }
 
-// LJ inside rc_lj plus qq_ke erfc(alpha r)/r inside rc_ew (site_pair_energy with one division
-// for 1/r shared by both terms).
+// 1/x and 1/sqrt(x) of a positive normal x: the hardware's approximation (about 2^-24) and two
+// Newton steps with fused residuals, which leave at most an ulp or two. The compiler's own FP64
+// division and square root add the scaling and fix-up for zeros, subnormals and infinities that
+// squared distances inside a cutoff never are (r2 = 0 still gives a non-finite pair energy).
+__device__ inline double rcp64(double x)
+{
+    double y = __builtin_amdgcn_rcp(x);
+    y = __builtin_fma(__builtin_fma(-x, y, 1.0), y, y);
+    return __builtin_fma(__builtin_fma(-x, y, 1.0), y, y);
+}
+
+__device__ inline double rsqrt64(double x)
+{
+    double y = __builtin_amdgcn_rsq(x);
+    y = __builtin_fma(__builtin_fma(-x * y, y, 1.0), 0.5 * y, y);
+    return __builtin_fma(__builtin_fma(-x * y, y, 1.0), 0.5 * y, y);
+}
+
+// exp(x) for x in [-700, 1]: x = n ln2 + r with |r| <= ln2 / 2, the Taylor series of exp(r) to
+// r^13 (remainder below 5e-18 of the value), scaled by 2^n.
+__device__ inline double exp64_small(double x)
+{
+    const double n = __builtin_rint(x * 1.4426950408889634);
+    const double r = __builtin_fma(-n, 1.9082149292705877e-10, __builtin_fma(-n, 0.6931471803691238, x));
+    constexpr double C[14] = {1.0, 1.0, 1.0 / 2, 1.0 / 6, 1.0 / 24, 1.0 / 120, 1.0 / 720, 1.0 / 5040, 1.0 / 40320,
+                              1.0 / 362880, 1.0 / 3628800, 1.0 / 39916800, 1.0 / 479001600, 1.0 / 6227020800.0};
+    double p = C[13];
+#pragma unroll
+    for (int k = 12; k >= 0; --k) p = __builtin_fma(p, r, C[k]);
+    return __builtin_amdgcn_ldexp(p, (int)n);
+}
+
+// LJ inside rc_lj plus qq_ke erfc(alpha r)/r inside rc_ew. The value of pair_erfc_f64 through the
+// same series as an ordinary polynomial (16 fused steps instead of 32 operations), one
+// reciprocal square root for r and 1/r and one reciprocal for t: about 65 FP64 instructions
+// where the Clenshaw form with the library's divisions, square root and exp takes about 250.
+// An attempt of one chain evaluates some 1,100 pairs on four wavefronts.
 __device__ inline double cw_pair(double r2, double sg, double ep, double qq_ke, double alpha, double rc_lj2,
                                  double rc_ew2)
 {
-    const double r = __builtin_sqrt(r2);
-    const double ir = 1.0 / r;
+    const double ir = rsqrt64(r2);
     double e = 0.0;
     if (r2 < rc_lj2) {
         const double s = sg * ir;
@@ -234,7 +268,13 @@ __device__ inline double cw_pair(double r2, double sg, double ep, double qq_ke, 
         x = x * x * x;
         e = 4.0 * ep * __builtin_fma(x, x, -x);
     }
-    if (r2 < rc_ew2) e = __builtin_fma(qq_ke * pair_erfc_f64_t<true>(alpha * r), ir, e);
+    if (r2 < rc_ew2) {
+        const double z = alpha * (r2 * ir);
+        const double t = 2.0 * rcp64(2.0 + z);
+        constexpr double XA = 4.0 / (1.0 - PAIR_ERFC_XLO), XB = -2.0 * (1.0 + PAIR_ERFC_XLO) / (1.0 - PAIR_ERFC_XLO) - 1.0;
+        const double p = pair_erfc_poly64(__builtin_fma(XA, t, XB));
+        e = __builtin_fma(qq_ke * (t * exp64_small(__builtin_fma(-z, z, p))), ir, e);
+    }
     return e;
 }
 
@@ -266,15 +306,20 @@ __host__ __device__ inline double site_pair_energy(double r2, double sg, double 
 }
 
 // e^{i k.r} of a guest site for k = 2 pi A^-T n at the Cartesian point r = A f, as the product
-// over axes of e^{2 pi i n_d f_d}. axis_power gives e^{2 pi i m f_d} (m >= 0); cis_from_axes
-// multiplies the three, conjugating the axes with negative n_d. The move path's kernel (from
-// per-attempt LDS tables) and the host's structure-factor rebuild evaluate both identically.
+// over axes of e^{2 pi i n_d f_d}. axis_power gives e^{2 pi i m f_d} (m >= 0), the phase m f_d
+// reduced to one revolution with its rounding error carried along, so that a product of two
+// powers agrees with the power of the sum to an ulp or two (the move kernel multiplies powers
+// where the audit's rebuild takes one); cis_from_axes multiplies the three, conjugating the axes
+// with negative n_d. The host's and the audit's structure-factor rebuilds evaluate both
+// identically.
 __host__ __device__ inline double2 axis_power(const double *invA, const double r[3], int d, int m)
 {
 #pragma clang fp contract(off)
-    const double f = invA[d] * r[0] + invA[d + 3] * r[1] + invA[d + 6] * r[2];
+    double f = invA[d] * r[0] + invA[d + 3] * r[1] + invA[d + 6] * r[2];
+    f -= __builtin_rint(f);
+    const double p = (double)m * f, lo = __builtin_fma((double)m, f, -p);
     double sn, cs;
-    sincospi(2.0 * ((double)m * f), &sn, &cs);
+    sincospi(2.0 * ((p - __builtin_rint(p)) + lo), &sn, &cs);
     return make_double2(cs, sn);
 }
 
@@ -286,24 +331,39 @@ __host__ __device__ inline double2 cis_from_axes(double2 e0, double2 e1, double2
     return make_double2(pr * e2.x - pi * i2, pr * i2 + pi * e2.x);
 }
 
+// The k-vectors of a framework as runs of consecutive n3 at fixed (n1, n2), longest first, cut
+// into blocks of 64 runs, one run per lane. A run of length L is walked from its middle outwards:
+// step 0 is n3 = m, step j takes m + j (while 2j <= L) and m - j (while 2j + 1 <= L), so that both
+// share the products of e^{2 pi i (n1 f1 + n2 f2 + m f3)} and e^{2 pi i j f3}. Lengths descend,
+// so the runs still active at a step are the block's first lanes, and the k-vectors are stored in
+// the order in which they are visited (block, step, +/-, lane) without gaps.
+struct KRuns {
+    const int4 *run;           // n1, n2, m, length; framework u's at [run_off[u], run_off[u + 1])
+    const int *run_off;        // nfw + 1
+    const int *base;           // per block of 64 runs: position of its first k-vector
+    const int *blk_off;        // nfw + 1
+    const double *kw;          // kprefactor by position (slices as the k tables)
+};
+
 // Move types of the move path: the reference's three NVT moves (src/moves.jl:69-71) and the two
 // exchange moves.
 constexpr int MOVE_TRANSLATION = 1, MOVE_ROTATION = 2, MOVE_REINSERTION = 3, MOVE_INSERTION = 4, MOVE_DELETION = 5;
 constexpr int NMOVES = 5;
 // attempts of one chain the move kernel evaluates together (speculatively, against the state at
-// the start of the round); the pending structure-factor changes take MC_SPEC slices per chain
+// the start of the round)
 constexpr int MC_SPEC = 2;
 
 // Snapshots of the chains' states for the test insertions (nvt_kernels.hip). Slot c holds, per
 // system n: occupancy at occ[c * nsys + n]; guests at pos/quat[c * nslots + guest_off[n] + i];
 // the weighted structure factor c_k = kprefactor_k * S_k of every k-vector at
-// csk[c * ctot + coff[n] + perm[F.k_off + k]], the order in which the insertion kernel's lanes
-// read it (runs of consecutive n3 interleaved across the 64 lanes).
+// csk[c * ctot + coff[n] + perm[F.k_off + p]] for the k-vector at position p (KRuns), the order
+// in which the insertion kernel's lanes read it (runs of consecutive n3 interleaved across the
+// 64 lanes).
 struct ChainSnap {
     int nsys, nslots;
     int64_t ctot;
     const int *coff;           // per system: first entry of its slice of csk
-    const int *perm;           // per k-vector of the batch: position within its framework's slice
+    const int *perm;           // per k-vector position of the batch: place within its framework's slice
     int *occ;
     double4 *pos, *quat;
     double2 *csk;
@@ -319,8 +379,7 @@ struct McArgs {
     const int *atype;
     const double4 *atomf;       // fractional x, y, z and charge (the test-insertion tables' order)
     const int *atypef;          // compact types in the same order
-    const double4 *k64;         // kx, ky, kz, kprefactor
-    const int4 *kn;             // n of k = 2 pi A^-T n, same order as k64
+    KRuns kr;                   // the k-vectors; Sk is stored in their order
     int ktab_w;                 // max over frameworks of kn_max[0] + kn_max[1] + kn_max[2] + 3
     const double2 *pair64;      // [site][type]: sigma, epsilon
     int ntypes_c;
@@ -334,9 +393,8 @@ struct McArgs {
     double4 *refpos;            // per slot: x, y, z (Å), 0
     double4 *quat;              // per slot: x, y, z, w
     double *host_e;             // per slot: cached host-guest real-space energy
-    double2 *Sk;                // per system k slice: host + every guest
-    double2 *dS;                // scratch, same layout: the pending move's structure-factor change
-    double *sk_abs;             // per k: accumulated rounding scale
+    double2 *Sk;                // per system k slice, by position: host + every guest
+    double *sk_abs;             // per system: accumulated rounding scale of every S_k
     const int *sk_off;          // nsys + 1
     double *energy, *energy_abs;
     const uint64_t *rng_seed;

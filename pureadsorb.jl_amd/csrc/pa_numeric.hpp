@@ -232,40 +232,67 @@ __host__ __device__ inline uint32_t to_fixed(double f)
 constexpr double PAIR_ERFC_XMAX = 4.0;
 constexpr double PAIR_ERFC_XLO = 2.0 * (2.0 / (2.0 + PAIR_ERFC_XMAX)) - 1.0;
 
-// FUSED = true evaluates the recurrence with fma (one rounding per step instead of two); the
-// move path and the Widom FP64 path use FUSED = false.
-template <bool FUSED>
-__host__ __device__ inline double pair_erfc_f64_t(double z)
+// Coefficient of T_j in the Float64 series.
+__host__ __device__ constexpr inline double pair_erfc_f64_t(int j)
+{
+    constexpr double c[17] = {-0.888894912038317, 0.4479385778277769, -0.00021608983881297707,
+                              -0.003410058708799526, 8.555152981629436e-5, 5.532830637302869e-5,
+                              -5.2098383667087075e-6, -8.380063246741613e-7, 1.9764068422519322e-7,
+                              1.7838566371819855e-9, -5.26989861621132e-9, 5.378177355603348e-10,
+                              7.748359588558286e-11, -2.3770397709020423e-11, 8.934868696420547e-13,
+                              5.207576546902621e-13, -9.42604840757663e-14};
+    return c[j];
+}
+
+// The Clenshaw form with the library's division and exp, every rounding step of the reference's
+// formula.
+__host__ __device__ inline double pair_erfc_f64(double z)
 {
 #pragma clang fp contract(off)
-    const double c[17] = {-0.888894912038317, 0.4479385778277769, -0.00021608983881297707,
-                          -0.003410058708799526, 8.555152981629436e-5, 5.532830637302869e-5,
-                          -5.2098383667087075e-6, -8.380063246741613e-7, 1.9764068422519322e-7,
-                          1.7838566371819855e-9, -5.26989861621132e-9, 5.378177355603348e-10,
-                          7.748359588558286e-11, -2.3770397709020423e-11, 8.934868696420547e-13,
-                          5.207576546902621e-13, -9.42604840757663e-14};
     double t = 2.0 / (2.0 + z);
     double xi = 2.0 * (2.0 * t - 1.0 - PAIR_ERFC_XLO) / (1.0 - PAIR_ERFC_XLO) - 1.0;
     double d = 0.0, dd = 0.0;
-    if (FUSED) {
-        const double x2 = 2.0 * xi;
-#pragma unroll
-        for (int j = 16; j >= 1; --j) {
-            double tmp = d;
-            d = __builtin_fma(x2, d, c[j] - dd);
-            dd = tmp;
-        }
-        return t * exp(__builtin_fma(xi, d, c[0] / 2.0 - dd) - z * z);
-    }
     for (int j = 16; j >= 1; --j) {
         double tmp = d;
-        d = 2.0 * xi * d - dd + c[j];
+        d = 2.0 * xi * d - dd + pair_erfc_f64_t(j);
         dd = tmp;
     }
-    return t * exp(xi * d - dd + c[0] / 2.0 - z * z);
+    return t * exp(xi * d - dd + pair_erfc_f64_t(0) / 2.0 - z * z);
 }
 
-__host__ __device__ inline double pair_erfc_f64(double z) { return pair_erfc_f64_t<false>(z); }
+// Coefficient k of the same series c0/2 + sum_{j=1..16} c_j T_j(xi) as an ordinary polynomial
+// (T_{j+1} = 2 xi T_j - T_{j-1}, expanded at compile time).
+__host__ __device__ constexpr double pair_erfc_mono64(int k)
+{
+    double a[17] = {}, b[17] = {};
+    a[0] = 1.0;
+    b[1] = 1.0;
+    double v = 0.5 * pair_erfc_f64_t(0) * a[k] + pair_erfc_f64_t(1) * b[k];
+    for (int j = 2; j < 17; ++j) {
+        double n[17] = {};
+        for (int i = 0; i < 17; ++i) n[i] = (i > 0 ? 2.0 * b[i - 1] : 0.0) - a[i];
+        for (int i = 0; i < 17; ++i) {
+            a[i] = b[i];
+            b[i] = n[i];
+        }
+        v += pair_erfc_f64_t(j) * b[k];
+    }
+    return v;
+}
+
+template <int K>
+struct PairErfcMono64 {
+    static constexpr double v = pair_erfc_mono64(K);
+};
+
+// log(erfc(z)/t) + z^2 at xi by Horner's rule: 16 fused steps. The coefficients fall off fast
+// enough that no digits are lost: it stays within 3e-16 of the Clenshaw form over [-1, 1].
+template <int K = 0>
+__host__ __device__ inline double pair_erfc_poly64(double xi)
+{
+    if constexpr (K == 16) return PairErfcMono64<16>::v;
+    else return __builtin_fma(pair_erfc_poly64<K + 1>(xi), xi, PairErfcMono64<K>::v);
+}
 
 // The reference's Float32 coefficient set (src/ewald.jl:120-123).
 __host__ __device__ constexpr float pair_erfc_c32(int j)
