@@ -28,12 +28,12 @@ struct pa_state {
     std::vector<double> const_p, const_q;  // exchange constant term, eV (src/moves.jl:728-773)
     std::vector<int> acc_at_audit;         // accepted moves per system at the last audit
     int64_t samp_stride = 0;               // production samples per system of the last GCMC run
-    DevAlloc d_guest_off, d_occ, d_refpos, d_quat, d_host_e, d_Sk, d_skabs, d_sk_off, d_energy, d_energy_abs,
-        d_seed, d_counter, d_acc, d_att, d_step_t, d_step_r, d_fug, d_cp, d_cq, d_samp_e, d_samp_n, d_maxocc,
+    DevAlloc d_guest_off, d_occ, d_refpos, d_quat, d_host_e, d_gsite, d_Sk, d_skabs, d_sk_off, d_energy, d_energy_abs,
+        d_seed, d_counter, d_acc, d_att, d_step_t, d_step_r, d_log_fugV, d_logn, d_cp, d_cq, d_samp_e, d_samp_n, d_maxocc,
         d_caphit, d_trace;
     // NVT driver: fractional atom table, insertion constant per system, move-launch snapshots,
     // test-insertion scratch, and the per-cycle records of the last run (nsys x nvt_np)
-    DevAlloc d_atomf64, d_atype_s, d_chunk, d_chunk_off, d_lines, d_rounds, d_round_off, d_perm, d_coff,
+    DevAlloc d_chunk, d_chunk_off, d_lines, d_rounds, d_round_off, d_perm, d_coff,
         d_half_perp, d_ct, d_snap_pos, d_snap_quat, d_snap_sk, d_snap_occ, d_item_off, d_cw_dU, d_pose_pos,
         d_pose_quat;
     // the k-vectors' order on the device (KRuns): position of every k-vector within its framework's
@@ -279,8 +279,7 @@ McArgs base_mc(pa_state *st)
     a.fw_of = b->d_fw_of.as<int>();
     a.atom64 = b->d_atom64.as<double4>();
     a.atype = b->d_atype.as<int>();
-    a.atomf = st->d_atomf64.as<double4>();
-    a.atypef = st->d_atype_s.as<int>();
+    a.near = near_lists(b);
     a.upper = b->upper_all ? 1 : 0;
     a.kr = KRuns{st->d_run.as<int4>(), st->d_run_off.as<int>(), st->d_kbase.as<int>(), st->d_kblk_off.as<int>(),
                  st->d_kw.as<double>()};
@@ -298,6 +297,7 @@ McArgs base_mc(pa_state *st)
     a.refpos = st->d_refpos.as<double4>();
     a.quat = st->d_quat.as<double4>();
     a.host_e = st->d_host_e.as<double>();
+    a.gsite = st->d_gsite.as<double4>();
     a.Sk = st->d_Sk.as<double2>();
     a.sk_abs = st->d_skabs.as<double>();
     a.sk_off = st->d_sk_off.as<int>();
@@ -309,7 +309,8 @@ McArgs base_mc(pa_state *st)
     a.attempted = st->d_att.as<int>();
     a.step_trans = st->d_step_t.as<double>();
     a.step_rot = st->d_step_r.as<double>();
-    a.fug = st->d_fug.as<double>();
+    a.log_fugV = st->d_log_fugV.as<double>();
+    a.logn = st->d_logn.as<double>();
     a.const_p = st->d_cp.as<double>();
     a.const_q = st->d_cq.as<double>();
     a.max_occ = st->d_maxocc.as<int>();
@@ -478,6 +479,7 @@ extern "C" int pa_state_create(pa_batch *b, const pa_guest *guest, const int32_t
     HIP_TRY(upload(S->d_refpos, pos));
     HIP_TRY(upload(S->d_quat, quat));
     HIP_TRY(upload(S->d_host_e, host_e));
+    HIP_TRY(S->d_gsite.ensure(sizeof(double4) * (size_t)nslots * NS));
     HIP_TRY(upload(S->d_Sk, Sk));
     HIP_TRY(upload(S->d_skabs, std::vector<double>(nsys, 0.0)));
     HIP_TRY(upload(S->d_energy, energy));
@@ -493,7 +495,13 @@ extern "C" int pa_state_create(pa_batch *b, const pa_guest *guest, const int32_t
     std::vector<double> zd(nsys, 0.0);
     HIP_TRY(upload(S->d_step_t, zd));
     HIP_TRY(upload(S->d_step_r, zd));
-    HIP_TRY(upload(S->d_fug, zd));
+    HIP_TRY(upload(S->d_log_fugV, zd));
+    // log(occupancy + 1) of the exchange moves' acceptance, for every occupancy a chain can have
+    int capmax = 0;
+    for (int n = 0; n < nsys; ++n) capmax = std::max(capmax, S->guest_off[n + 1] - S->guest_off[n]);
+    std::vector<double> logn(capmax + 1);
+    for (int i = 0; i <= capmax; ++i) logn[i] = std::log((double)i + 1.0);
+    HIP_TRY(upload(S->d_logn, logn));
     S->acc_at_audit.assign(nsys, 0);
     int s_tab = ensure_chain_tables(S.get());
     if (s_tab) return s_tab;
@@ -502,6 +510,12 @@ extern "C" int pa_state_create(pa_batch *b, const pa_guest *guest, const int32_t
 }
 
 extern "C" void pa_state_destroy(pa_state *st) { delete st; }
+
+// log(f V) of system n's exchange moves, f in Pa (Pa -> eV/Å^3, src/constants.jl:10).
+static double log_fugacity_volume(const pa_state *st, int n, double fugacity_pa)
+{
+    return std::log(fugacity_pa * PASCAL_EV * st->b->desc[st->b->fw_of[n]].volume);
+}
 
 // Runs `nmoves` attempts of one move type on every chain (mode 0 of the chain kernel).
 static int run_moves(pa_state *st, int movetype, int64_t nmoves, const double *step_trans, const double *step_rot,
@@ -527,9 +541,9 @@ static int run_moves(pa_state *st, int movetype, int64_t nmoves, const double *s
         std::vector<double> f(st->nsys);
         for (int n = 0; n < st->nsys; ++n) {
             if (!(fugacity_pa[n] > 0)) return fail(PA_ERR_ARG, "fugacity[%d] = %g Pa must be positive", n, fugacity_pa[n]);
-            f[n] = fugacity_pa[n] * PASCAL_EV;  // Pa -> eV/Å^3 (src/constants.jl:10)
+            f[n] = log_fugacity_volume(st, n, fugacity_pa[n]);
         }
-        HIP_TRY(upload(st->d_fug, f));
+        HIP_TRY(upload(st->d_log_fugV, f));
     }
     if (nmoves == 0) return ok();
     McArgs a = base_mc(st);
@@ -537,6 +551,7 @@ static int run_moves(pa_state *st, int movetype, int64_t nmoves, const double *s
     a.movetype = movetype;
     a.nmoves = nmoves;
     a.kT = KB * T;
+    a.log_kT = std::log(a.kT);
     if (trace) {
         HIP_TRY(st->d_trace.ensure(sizeof(double4) * (size_t)st->nsys * nmoves));
         a.trace = st->d_trace.as<double4>();
@@ -973,13 +988,14 @@ extern "C" int pa_gcmc_run(pa_state *st, const pa_gcmc_params *p, pa_gcmc_result
         std::vector<double> f(nsys);
         for (int n = 0; n < nsys; ++n) {
             if (!(p->fugacity_pa[n] > 0)) return fail(PA_ERR_ARG, "fugacity[%d] = %g Pa must be positive", n, p->fugacity_pa[n]);
-            f[n] = p->fugacity_pa[n] * PASCAL_EV;
+            f[n] = log_fugacity_volume(st, n, p->fugacity_pa[n]);
         }
-        HIP_TRY(upload(st->d_fug, f));
+        HIP_TRY(upload(st->d_log_fugV, f));
     }
     McArgs a = base_mc(st);
     a.mode = 1;
     a.kT = KB * p->T;
+    a.log_kT = std::log(a.kT);
     double c = 0.0;
     for (int t = 0; t < NMOVES; ++t) {
         c += pr[t] / tot;
@@ -1095,17 +1111,6 @@ double insertion_constant_term(const pa_batch *b, int u, int Ng)
     return base + guest_tail_h(b, u, N + 1) - guest_tail_h(b, u, N) + net_h(b, u, N + 1) - net_h(b, u, N);
 }
 
-// Spreads the low 10 bits of v to every third bit (Morton interleave).
-uint32_t spread3(uint32_t v)
-{
-    v &= 0x3FF;
-    v = (v | (v << 16)) & 0x030000FF;
-    v = (v | (v << 8)) & 0x0300F00F;
-    v = (v | (v << 4)) & 0x030C30C3;
-    v = (v | (v << 2)) & 0x09249249;
-    return v;
-}
-
 // The order in which the device keeps and visits the k-vectors of a chain (KRuns): the runs of
 // consecutive n3 at fixed (n1, n2) in k-table order, longest first.
 int build_k_runs(pa_state *st)
@@ -1157,16 +1162,18 @@ int build_k_runs(pa_state *st)
 }
 
 // Tables of the chain-insertion kernel, built once per state: every framework's atoms in
-// Morton order of a ~4 Å cell grid, cut into chunks of 64 with a centre and a radius that
+// Morton order, cut into chunks of 64 with a centre and a radius that
 // bounds every atom's nearest-image distance to the centre; the k-vectors cut into runs of
 // consecutive n3 at fixed (n1, n2), longest first; half the smallest perpendicular width.
 int ensure_chain_tables(pa_state *st)
 {
     pa_batch *b = st->b;
-    if (st->d_atomf64.p) return PA_OK;
-    const size_t na = std::max<size_t>(b->atom64_h.size(), 1);
-    std::vector<double4> af(na, make_double4(0, 0, 0, 0));
-    std::vector<int> at(na, 0), chunk_off(1, 0), round_off(1, 0), perm(std::max<size_t>(b->k64_h.size(), 1), 0),
+    if (st->d_half_perp.p) return PA_OK;
+    if (int e = ensure_near_lists(b)) return e;
+    std::vector<double4> af;
+    std::vector<int> at;
+    if (int e = near_atoms(b, af, at)) return e;
+    std::vector<int> chunk_off(1, 0), round_off(1, 0), perm(std::max<size_t>(b->k64_h.size(), 1), 0),
         fsize(b->nfw, 0);
     std::vector<double4> chunks;
     std::vector<int2> lines, rounds;
@@ -1174,29 +1181,7 @@ int ensure_chain_tables(pa_state *st)
     for (int u = 0; u < b->nfw; ++u) {
         const FwDesc &F = b->desc[u];
         const FwHost &h = b->info[u];
-        const std::vector<double> &fr = b->fgh[u].frac;
         const int n = F.natoms;
-        if ((int)fr.size() != 3 * n) return fail(PA_ERR_INTERNAL, "framework %d: fractional table missing", u + 1);
-        int nc[3];
-        for (int d = 0; d < 3; ++d) nc[d] = std::max(1, std::min(1024, (int)std::floor(h.perp[d] / 4.0)));
-        std::vector<uint64_t> key(n);
-        std::vector<double> f(3 * (size_t)n);
-        for (int j = 0; j < n; ++j) {
-            uint32_t c[3];
-            for (int d = 0; d < 3; ++d) {
-                const double x = fr[3 * j + d] - std::floor(fr[3 * j + d]);
-                f[3 * j + d] = x;
-                c[d] = (uint32_t)std::min(nc[d] - 1, (int)(x * nc[d]));
-            }
-            const uint64_t m = spread3(c[0]) | (spread3(c[1]) << 1) | (spread3(c[2]) << 2);
-            key[j] = (m << 32) | (uint32_t)j;
-        }
-        std::sort(key.begin(), key.end());
-        for (int i = 0; i < n; ++i) {
-            const int j = (int)(key[i] & 0xFFFFFFFFu);
-            af[F.atom_off + i] = make_double4(f[3 * j], f[3 * j + 1], f[3 * j + 2], b->atom64_h[F.atom_off + j].w);
-            at[F.atom_off + i] = b->atype_h[F.atom_off + j];
-        }
         for (int c0 = 0; c0 < n; c0 += 64) {
             const int c1 = std::min(n, c0 + 64);
             const double4 r0 = af[F.atom_off + c0];
@@ -1257,7 +1242,6 @@ int ensure_chain_tables(pa_state *st)
     }
     const double rcmax = std::max(b->rc_lj, b->gdev.charged ? b->rc_ew : 0.0);
     st->cull_extra = rcmax + b->r_guest + 1e-6;
-    HIP_TRY(upload(st->d_atype_s, at));
     HIP_TRY(upload(st->d_chunk, chunks));
     HIP_TRY(upload(st->d_chunk_off, chunk_off));
     HIP_TRY(upload(st->d_lines, lines));
@@ -1276,7 +1260,6 @@ int ensure_chain_tables(pa_state *st)
     st->ctot = coff[st->nsys];
     HIP_TRY(upload(st->d_coff, coff));
     HIP_TRY(upload(st->d_half_perp, halfw));
-    HIP_TRY(upload(st->d_atomf64, af));
     return PA_OK;
 }
 
@@ -1301,8 +1284,8 @@ ChainWidomArgs base_chain_widom(pa_state *st)
     ChainWidomArgs a{};
     a.fw = b->d_fw.as<FwDesc>();
     a.fw_of = b->d_fw_of.as<int>();
-    a.atomf64 = st->d_atomf64.as<double4>();
-    a.atype = st->d_atype_s.as<int>();
+    a.atomf64 = b->d_nearf.as<double4>();
+    a.atype = b->d_neart.as<int>();
     a.chunk = st->d_chunk.as<double4>();
     a.chunk_off = st->d_chunk_off.as<int>();
     a.lines = st->d_lines.as<int2>();
@@ -1479,6 +1462,7 @@ extern "C" int pa_nvt_run(pa_state *st, const pa_guest *guest, const pa_nvt_para
     McArgs a = base_mc(st);
     a.mode = 1;
     a.kT = kT;
+    a.log_kT = std::log(kT);
     const double pr[NMOVES] = {1.0, 1.0, 1.0, 0.0, 0.0};
     double c = 0.0;
     for (int t = 0; t < NMOVES; ++t) {

@@ -107,7 +107,7 @@ __global__ __launch_bounds__(CW_WG, (NS <= 3 ? 4 : 1)) void chain_widom_kernel(C
                 const unsigned i = (head + lane) & (CW_RING - 1);
                 const int code = qcode[i];
                 const double2 p = a.pair64[code];
-                e += cw_pair(qr2[i], p.x, p.y, qqq[i], F.alpha, a.rc_lj2, a.rc_ew2);
+                e += cw_pair(qr2[i], p.x * p.x, 4.0 * p.y, qqq[i], F.alpha, a.rc_lj2, a.rc_ew2);
             }
             head = __builtin_amdgcn_readfirstlane(head + n);
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -206,7 +206,7 @@ __global__ __launch_bounds__(CW_WG, (NS <= 3 ? 4 : 1)) void chain_widom_kernel(C
         const double r2 = cw_r2_t<UPPER>(F.A, sf[sa][0] - fb[0], sf[sa][1] - fb[1], sf[sa][2] - fb[2]);
         if (r2 < a.rc_lj2 || r2 < a.rc_ew2) {
             const double2 p = a.pair64[sa * a.ntypes_c + G.type[sb]];
-            e += cw_pair(r2, p.x, p.y, KE * G.q[sa] * G.q[sb], F.alpha, a.rc_lj2, a.rc_ew2);
+            e += cw_pair(r2, p.x * p.x, 4.0 * p.y, KE * G.q[sa] * G.q[sb], F.alpha, a.rc_lj2, a.rc_ew2);
         }
     }
 

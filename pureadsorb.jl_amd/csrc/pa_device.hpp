@@ -1,6 +1,8 @@
 // pa_device.hpp -- device-side data layout shared by the host library and the kernels.
 #pragma once
 
+#include <utility>
+
 #include "pa_numeric.hpp"
 
 namespace pa {
@@ -238,18 +240,56 @@ __device__ inline double rsqrt64(double x)
     return __builtin_fma(__builtin_fma(-x * y, y, 1.0), 0.5 * y, y);
 }
 
+// The FP64 polynomials' coefficients in constant memory: FP64 instructions take no literals, so
+// written as constants they are moved into registers once, outside every loop (60 doubles, 120
+// registers). pair_coefs() hides the table's address at each use, and they come by scalar loads.
+// exp(r) = sum r^k / k!, the erfc series' 17 coefficients, sincospi's 9 and 10.
+struct PairCoefs {
+    double exp_c[14], erfc_c[17], sin_c[9], cos_c[10];
+};
+typedef __attribute__((address_space(4))) const PairCoefs *PairCoefPtr;
+
+template <int... K>
+constexpr PairCoefs make_pair_coefs(std::integer_sequence<int, K...>)
+{
+    return PairCoefs{{1.0, 1.0, 1.0 / 2, 1.0 / 6, 1.0 / 24, 1.0 / 120, 1.0 / 720, 1.0 / 5040, 1.0 / 40320, 1.0 / 362880,
+                      1.0 / 3628800, 1.0 / 39916800, 1.0 / 479001600, 1.0 / 6227020800.0},
+                     {pair_erfc_mono64(K)...},
+                     {SINCOSPI_S[0], SINCOSPI_S[1], SINCOSPI_S[2], SINCOSPI_S[3], SINCOSPI_S[4], SINCOSPI_S[5],
+                      SINCOSPI_S[6], SINCOSPI_S[7], SINCOSPI_S[8]},
+                     {SINCOSPI_C[0], SINCOSPI_C[1], SINCOSPI_C[2], SINCOSPI_C[3], SINCOSPI_C[4], SINCOSPI_C[5],
+                      SINCOSPI_C[6], SINCOSPI_C[7], SINCOSPI_C[8], SINCOSPI_C[9]}};
+}
+static __constant__ const PairCoefs PAIR_COEFS = make_pair_coefs(std::make_integer_sequence<int, 17>{});
+
+__device__ inline PairCoefPtr pair_coefs()
+{
+    PairCoefPtr p = (PairCoefPtr)&PAIR_COEFS;
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
+// sum_{k=0..N} c_k x^k as two Horner chains in x^2, even and odd powers: half the dependent steps
+// of one chain, which is what a wavefront alone on its SIMD waits for.
+template <int N, class P>
+__device__ inline double poly_even_odd(double x, const P &c)
+{
+    const double y = x * x;
+    double e = c[N & ~1], o = c[(N - 1) | 1];
+#pragma unroll
+    for (int k = (N & ~1) - 2; k >= 0; k -= 2) e = __builtin_fma(e, y, c[k]);
+#pragma unroll
+    for (int k = ((N - 1) | 1) - 2; k >= 0; k -= 2) o = __builtin_fma(o, y, c[k]);
+    return __builtin_fma(o, x, e);
+}
+
 // exp(x) for x in [-700, 1]: x = n ln2 + r with |r| <= ln2 / 2, the Taylor series of exp(r) to
 // r^13 (remainder below 5e-18 of the value), scaled by 2^n.
-__device__ inline double exp64_small(double x)
+__device__ inline double exp64_small(double x, PairCoefPtr C)
 {
     const double n = __builtin_rint(x * 1.4426950408889634);
     const double r = __builtin_fma(-n, 1.9082149292705877e-10, __builtin_fma(-n, 0.6931471803691238, x));
-    constexpr double C[14] = {1.0, 1.0, 1.0 / 2, 1.0 / 6, 1.0 / 24, 1.0 / 120, 1.0 / 720, 1.0 / 5040, 1.0 / 40320,
-                              1.0 / 362880, 1.0 / 3628800, 1.0 / 39916800, 1.0 / 479001600, 1.0 / 6227020800.0};
-    double p = C[13];
-#pragma unroll
-    for (int k = 12; k >= 0; --k) p = __builtin_fma(p, r, C[k]);
-    return __builtin_amdgcn_ldexp(p, (int)n);
+    return __builtin_amdgcn_ldexp(poly_even_odd<13>(r, C->exp_c), (int)n);
 }
 
 // LJ inside rc_lj plus qq_ke erfc(alpha r)/r inside rc_ew. The value of pair_erfc_f64 through the
@@ -257,23 +297,30 @@ __device__ inline double exp64_small(double x)
 // reciprocal square root for r and 1/r and one reciprocal for t: about 65 FP64 instructions
 // where the Clenshaw form with the library's divisions, square root and exp takes about 250.
 // An attempt of one chain evaluates some 1,100 pairs on four wavefronts.
-__device__ inline double cw_pair(double r2, double sg, double ep, double qq_ke, double alpha, double rc_lj2,
+// sg2 = sigma^2, ep4 = 4 epsilon. EXACT_LJ: the LJ term in site_pair_energy's own operations, so
+// that a pair of overlapping guests (1e6 eV and more are allowed) has the same bits here and in
+// the rebuilds that the running energy is audited against.
+template <bool EXACT_LJ = false>
+__device__ inline double cw_pair(double r2, double sg2, double ep4, double qq_ke, double alpha, double rc_lj2,
                                  double rc_ew2)
 {
     const double ir = rsqrt64(r2);
     double e = 0.0;
     if (r2 < rc_lj2) {
-        const double s = sg * ir;
-        double x = s * s;
+#pragma clang fp contract(off)
+        double x = EXACT_LJ ? sg2 / r2 : sg2 * (ir * ir);
         x = x * x * x;
-        e = 4.0 * ep * __builtin_fma(x, x, -x);
+        e = ep4 * (EXACT_LJ ? x * x - x : __builtin_fma(x, x, -x));
     }
     if (r2 < rc_ew2) {
         const double z = alpha * (r2 * ir);
         const double t = 2.0 * rcp64(2.0 + z);
         constexpr double XA = 4.0 / (1.0 - PAIR_ERFC_XLO), XB = -2.0 * (1.0 + PAIR_ERFC_XLO) / (1.0 - PAIR_ERFC_XLO) - 1.0;
-        const double p = pair_erfc_poly64(__builtin_fma(XA, t, XB));
-        e = __builtin_fma(qq_ke * (t * exp64_small(__builtin_fma(-z, z, p))), ir, e);
+        const double xi = __builtin_fma(XA, t, XB);
+        // log(erfc(z)/t) + z^2
+        const PairCoefPtr C = pair_coefs();
+        const double p = poly_even_odd<16>(xi, C->erfc_c);
+        e = __builtin_fma(qq_ke * (t * exp64_small(__builtin_fma(-z, z, p), C)), ir, e);
     }
     return e;
 }
@@ -312,15 +359,34 @@ __host__ __device__ inline double site_pair_energy(double r2, double sg, double 
 // where the audit's rebuild takes one); cis_from_axes multiplies the three, conjugating the axes
 // with negative n_d. The host's and the audit's structure-factor rebuilds evaluate both
 // identically.
+__host__ __device__ inline double axis_phase(double f, int m)
+{
+#pragma clang fp contract(off)
+    f -= __builtin_rint(f);
+    const double p = (double)m * f, lo = __builtin_fma((double)m, f, -p);
+    return 2.0 * ((p - __builtin_rint(p)) + lo);
+}
+
+__host__ __device__ inline double2 axis_power(double f, int m)
+{
+    double sn, cs;
+    sincospi(axis_phase(f, m), &sn, &cs);
+    return make_double2(cs, sn);
+}
+
+// The same with the series' coefficients from constant memory (pair_coefs), same operations.
+__device__ inline double2 axis_power_const(double f, int m)
+{
+    const PairCoefPtr C = pair_coefs();
+    double sn, cs;
+    sincospi_coefs(axis_phase(f, m), C->sin_c, C->cos_c, &sn, &cs);
+    return make_double2(cs, sn);
+}
+
 __host__ __device__ inline double2 axis_power(const double *invA, const double r[3], int d, int m)
 {
 #pragma clang fp contract(off)
-    double f = invA[d] * r[0] + invA[d + 3] * r[1] + invA[d + 6] * r[2];
-    f -= __builtin_rint(f);
-    const double p = (double)m * f, lo = __builtin_fma((double)m, f, -p);
-    double sn, cs;
-    sincospi(2.0 * ((p - __builtin_rint(p)) + lo), &sn, &cs);
-    return make_double2(cs, sn);
+    return axis_power(invA[d] * r[0] + invA[d + 3] * r[1] + invA[d + 6] * r[2], m);
 }
 
 __host__ __device__ inline double2 cis_from_axes(double2 e0, double2 e1, double2 e2, int nx, int ny, int nz)
@@ -345,13 +411,39 @@ struct KRuns {
     const double *kw;          // kprefactor by position (slices as the k tables)
 };
 
+// Lists of the atoms near a point (near_lists.hip): bins of framework u's cell, and per bin the
+// atoms that a guest with its reference point in the bin can have inside the cutoff. An entry is
+// the atom's index (Morton order, framework-relative) and above it its compact type.
+constexpr int NEAR_TYPE_SHIFT = 26;
+constexpr uint32_t NEAR_INDEX = (1u << NEAR_TYPE_SHIFT) - 1u;
+struct NearDesc {
+    int nb[3];
+    int bin_off;               // first bin of the framework in `start`
+    double r2;                 // squared list radius, Å^2
+    double reach[3];           // list radius over the perpendicular widths
+};
+struct NearLists {
+    const double4 *atomf;      // fractional x, y, z in [0, 1) and charge, Morton order
+    const NearDesc *desc;
+    const int *start;          // per bin, one past the last included
+    const uint32_t *ent;
+};
+
+// The bin of a point with fractional coordinates f.
+__device__ inline int near_bin(const NearDesc &D, const double f[3])
+{
+    int c[3];
+    for (int d = 0; d < 3; ++d) {
+        const double x = f[d] - __builtin_floor(f[d]);
+        c[d] = min(D.nb[d] - 1, (int)(x * D.nb[d]));
+    }
+    return D.bin_off + c[0] + D.nb[0] * (c[1] + D.nb[1] * c[2]);
+}
+
 // Move types of the move path: the reference's three NVT moves (src/moves.jl:69-71) and the two
 // exchange moves.
 constexpr int MOVE_TRANSLATION = 1, MOVE_ROTATION = 2, MOVE_REINSERTION = 3, MOVE_INSERTION = 4, MOVE_DELETION = 5;
 constexpr int NMOVES = 5;
-// attempts of one chain the move kernel evaluates together (speculatively, against the state at
-// the start of the round)
-constexpr int MC_SPEC = 2;
 
 // Snapshots of the chains' states for the test insertions (nvt_kernels.hip). Slot c holds, per
 // system n: occupancy at occ[c * nsys + n]; guests at pos/quat[c * nslots + guest_off[n] + i];
@@ -377,8 +469,7 @@ struct McArgs {
     const int *fw_of;
     const double4 *atom64;
     const int *atype;
-    const double4 *atomf;       // fractional x, y, z and charge (the test-insertion tables' order)
-    const int *atypef;          // compact types in the same order
+    NearLists near;             // the framework atoms near a pose
     KRuns kr;                   // the k-vectors; Sk is stored in their order
     int ktab_w;                 // max over frameworks of kn_max[0] + kn_max[1] + kn_max[2] + 3
     const double2 *pair64;      // [site][type]: sigma, epsilon
@@ -393,6 +484,7 @@ struct McArgs {
     double4 *refpos;            // per slot: x, y, z (Å), 0
     double4 *quat;              // per slot: x, y, z, w
     double *host_e;             // per slot: cached host-guest real-space energy
+    double4 *gsite;             // scratch, per slot and site: Cartesian positions of the live guests' sites
     double2 *Sk;                // per system k slice, by position: host + every guest
     double *sk_abs;             // per system: accumulated rounding scale of every S_k
     const int *sk_off;          // nsys + 1
@@ -407,7 +499,9 @@ struct McArgs {
     int64_t ncycles, min_cycle;
     double pcum[NMOVES];        // mode 1: cumulative probabilities of the move types
     const double *step_trans, *step_rot;   // per chain
-    const double *fug;          // per chain, eV/Å^3
+    const double *log_fugV;     // per chain: log of fugacity (eV/Å^3) times volume
+    const double *logn;         // log 1, log 2, ... up to the largest capacity + 1
+    double log_kT;
     const double *const_p, *const_q;       // exchange constant term p + q N (src/moves.jl:728-773)
     double kT;
     int upper;                  // every framework's A has A[1] == A[2] == A[5] == 0

@@ -219,6 +219,9 @@ struct pa_batch {
     std::vector<int> atype_h;
     pa::DevAlloc d_corefx, d_coreidx, d_cell_start, d_rho2, d_cand, d_ncand, d_nbr_start, d_nbr_atoms, d_passes;
     pa::DevAlloc d_binfx, d_bintype;  // the atoms in Morton order, for the mixed path's list build
+    // FP64 paths: lists of the atoms near a point, built on first use (near_lists.hip)
+    pa::DevAlloc d_nearf, d_neart, d_near_desc, d_near_start, d_near_ent;
+    bool near_ready = false;
     // gradient scratch
     pa::PinnedAlloc h_acc_q;  // gradient path: the per-atom charge accumulators read back
     pa::PinnedAlloc h_tiles;  // Widom calls: the Boltzmann tile sums read back
@@ -242,4 +245,9 @@ struct pa_batch {
 namespace pa {
 // Squared phase-0 rejection radii of system s at kT, NS x ntypes_c (build_rejection_tables).
 int rejection_radii(const pa_batch *b, int s, double kT, double eps_f, double *rho2, double *rmax2);
+// The batch's near lists (near_lists.hip): builds them once; their device form; the Morton-ordered
+// atoms they index.
+int ensure_near_lists(pa_batch *b);
+NearLists near_lists(const pa_batch *b);
+int near_atoms(const pa_batch *b, std::vector<double4> &af, std::vector<int> &at);
 }  // namespace pa

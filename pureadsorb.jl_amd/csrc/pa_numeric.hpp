@@ -46,23 +46,28 @@ __host__ __device__ inline double unit_f64(uint64_t raw) { return (double)(raw >
 // sin(pi x), cos(pi x): exact reduction by the nearest half-integer, then Taylor series of
 // sin(pi r), cos(pi r) for |r| <= 1/4 in Horner form with fused multiply-adds. The
 // coefficients are (-1)^k pi^(2k+1)/(2k+1)! and (-1)^k pi^(2k)/(2k)! rounded to double.
-__host__ __device__ inline void sincospi(double x, double *s_out, double *c_out)
+constexpr double SINCOSPI_S[9] = {0x1.921fb54442d18p+1, -0x1.4abbce625be53p+2, 0x1.466bc6775aae2p+1,
+                                  -0x1.32d2cce62bd86p-1, 0x1.50783487ee782p-4, -0x1.e3074fde8871fp-8,
+                                  0x1.e8f434d018d63p-12, -0x1.6fadb9f155744p-16, 0x1.aaec32af93359p-21};
+constexpr double SINCOSPI_C[10] = {0x1.0000000000000p+0, -0x1.3bd3cc9be45dep+2, 0x1.03c1f081b5ac4p+2,
+                                   -0x1.55d3c7e3cbffap+0, 0x1.e1f506891babbp-3, -0x1.a6d1f2a204a8cp-6,
+                                   0x1.f9d38a3763cc3p-10, -0x1.b6e24f44b128fp-14, 0x1.20c62c2f2d7f5p-18,
+                                   -0x1.2a0c591af8314p-23};
+
+// S, Cc: the two series' coefficients, wherever the caller keeps them.
+template <class P, class Q>
+__host__ __device__ inline void sincospi_coefs(double x, const P &S, const Q &Cc, double *s_out, double *c_out)
 {
 #pragma clang fp contract(off)
-    const double S[9] = {0x1.921fb54442d18p+1, -0x1.4abbce625be53p+2, 0x1.466bc6775aae2p+1,
-                         -0x1.32d2cce62bd86p-1, 0x1.50783487ee782p-4, -0x1.e3074fde8871fp-8,
-                         0x1.e8f434d018d63p-12, -0x1.6fadb9f155744p-16, 0x1.aaec32af93359p-21};
-    const double Cc[10] = {0x1.0000000000000p+0, -0x1.3bd3cc9be45dep+2, 0x1.03c1f081b5ac4p+2,
-                           -0x1.55d3c7e3cbffap+0, 0x1.e1f506891babbp-3, -0x1.a6d1f2a204a8cp-6,
-                           0x1.f9d38a3763cc3p-10, -0x1.b6e24f44b128fp-14, 0x1.20c62c2f2d7f5p-18,
-                           -0x1.2a0c591af8314p-23};
     double n = __builtin_rint(2.0 * x);
     double r = x - 0.5 * n;
     double r2 = r * r;
     double ps = S[8];
+#pragma unroll
     for (int k = 7; k >= 0; --k) ps = __builtin_fma(ps, r2, S[k]);
     double s = r * ps;
     double pc = Cc[9];
+#pragma unroll
     for (int k = 8; k >= 0; --k) pc = __builtin_fma(pc, r2, Cc[k]);
     double c = pc;
     int q = (int)((int64_t)n & 3);
@@ -73,6 +78,11 @@ __host__ __device__ inline void sincospi(double x, double *s_out, double *c_out)
     else { so = -c; co = s; }
     *s_out = so;
     *c_out = co;
+}
+
+__host__ __device__ inline void sincospi(double x, double *s_out, double *c_out)
+{
+    sincospi_coefs(x, SINCOSPI_S, SINCOSPI_C, s_out, c_out);
 }
 
 // Shoemake (1992) uniform unit quaternion, (x, y, z, w) order (src/rng.jl:126-129).
@@ -261,7 +271,9 @@ __host__ __device__ inline double pair_erfc_f64(double z)
 }
 
 // Coefficient k of the same series c0/2 + sum_{j=1..16} c_j T_j(xi) as an ordinary polynomial
-// (T_{j+1} = 2 xi T_j - T_{j-1}, expanded at compile time).
+// (T_{j+1} = 2 xi T_j - T_{j-1}, expanded at compile time). By Horner's rule it takes 16 fused
+// steps; the coefficients fall off fast enough that no digits are lost (1.1e-16 from the series in
+// extended precision over [-1, 1], the Clenshaw form 1.4e-16).
 __host__ __device__ constexpr double pair_erfc_mono64(int k)
 {
     double a[17] = {}, b[17] = {};
@@ -278,20 +290,6 @@ __host__ __device__ constexpr double pair_erfc_mono64(int k)
         v += pair_erfc_f64_t(j) * b[k];
     }
     return v;
-}
-
-template <int K>
-struct PairErfcMono64 {
-    static constexpr double v = pair_erfc_mono64(K);
-};
-
-// log(erfc(z)/t) + z^2 at xi by Horner's rule: 16 fused steps. The coefficients fall off fast
-// enough that no digits are lost: it stays within 3e-16 of the Clenshaw form over [-1, 1].
-template <int K = 0>
-__host__ __device__ inline double pair_erfc_poly64(double xi)
-{
-    if constexpr (K == 16) return PairErfcMono64<16>::v;
-    else return __builtin_fma(pair_erfc_poly64<K + 1>(xi), xi, PairErfcMono64<K>::v);
 }
 
 // The reference's Float32 coefficient set (src/ewald.jl:120-123).
