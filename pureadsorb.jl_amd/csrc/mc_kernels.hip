@@ -25,26 +25,6 @@ namespace pa {
 constexpr int MC_RING = 256;           // per-wavefront ring of in-cutoff pairs: up to 63 pending and 3 x 64 new
 constexpr int MC_BATCH = 64;           // attempts whose random part is drawn at once
 
-// Sum over the wavefront, in lane 63 (DPP shifts within rows of 16 lanes, then row broadcasts).
-template <int CTRL, int ROWS>
-__device__ inline double dpp_add(double v)
-{
-    const uint64_t b = __double_as_longlong(v);
-    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xf, true);
-    const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, ROWS, 0xf, true);
-    return v + __longlong_as_double(((uint64_t)hi << 32) | lo);
-}
-
-__device__ inline double wave_sum63(double v)
-{
-    v = dpp_add<0x111, 0xf>(v);  // row_shr:1
-    v = dpp_add<0x112, 0xf>(v);  // row_shr:2
-    v = dpp_add<0x114, 0xf>(v);  // row_shr:4
-    v = dpp_add<0x118, 0xf>(v);  // row_shr:8
-    v = dpp_add<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
-    return dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
-}
-
 // Minimum-image squared distance between two points of the cell, minimum_image's operations.
 // UPPER drops the products with the exact zeros of an upper-triangular cell and its inverse,
 // which leaves every bit unchanged.

@@ -46,22 +46,27 @@ __global__ __launch_bounds__(256) void near_kernel(NearBuild a)
     const double c0 = (bx + 0.5) / D.nb[0], c1 = (by + 0.5) / D.nb[1], c2 = (bz + 0.5) / D.nb[2];
     int total = 0;
     const int at0 = FILL ? a.start[b] : 0;
+    // filled in two sweeps: the atoms close to the bin come first, so that a caller that tests for
+    // overlaps finds them among the first entries
+    for (int cls = 0; cls < (FILL ? 2 : 1); ++cls)
     for (int j0 = 0; j0 < F.natoms; j0 += 64) {
         const int j = j0 + lane;
         bool in = false;
+        double best = INFINITY;
         if (j < F.natoms) {
             const double4 h = a.atomf[F.atom_off + j];
             double f[3] = {h.x - c0, h.y - c1, h.z - c2};
             for (int d = 0; d < 3; ++d) f[d] -= __builtin_rint(f[d]);
-            for (int s = 0; s < 27 && !in; ++s) {
+            for (int s = 0; s < 27; ++s) {
                 const double g0 = f[0] + (s % 3 - 1), g1 = f[1] + ((s / 3) % 3 - 1), g2 = f[2] + (s / 9 - 1);
                 // an offset's component times the perpendicular width bounds its length from below
                 if (fabs(g0) > D.reach[0] || fabs(g1) > D.reach[1] || fabs(g2) > D.reach[2]) continue;
                 const double x = F.A[0] * g0 + F.A[3] * g1 + F.A[6] * g2;
                 const double y = F.A[1] * g0 + F.A[4] * g1 + F.A[7] * g2;
                 const double z = F.A[2] * g0 + F.A[5] * g1 + F.A[8] * g2;
-                in = x * x + y * y + z * z <= D.r2;
+                best = fmin(best, x * x + y * y + z * z);
             }
+            in = best <= D.r2 && (!FILL || (best <= D.close2) == (cls == 0));
         }
         const uint64_t mask = __builtin_amdgcn_ballot_w64(in);
         if (FILL && in) {
@@ -152,6 +157,7 @@ int ensure_near_lists(pa_batch *b)
                 }
             const double R = rcmax + b->r_guest + rb + 1.0e-6;
             D.r2 = R * R;
+            D.close2 = (rb + b->r_guest + 2.0) * (rb + b->r_guest + 2.0);
             for (int d = 0; d < 3; ++d) D.reach[d] = R / h.perp[d] * (1.0 + 1.0e-9);
             D.bin_off = (int)nbins;
             bin_fw[u] = (int)nbins;

@@ -411,6 +411,71 @@ struct KRuns {
     const double *kw;          // kprefactor by position (slices as the k tables)
 };
 
+// Ring of in-cutoff pairs of one wavefront in LDS: lanes append the pairs they found inside the
+// cutoff (two numbers and a code), full wavefronts evaluate 64 at a time, so that LJ + erfc run
+// on full wavefronts whatever the lanes' own pairs do. Up to 63 pending and 3 x 64 new.
+constexpr int PAIR_RING = 256;
+struct PairRing {
+    double x[PAIR_RING], y[PAIR_RING];
+    int code[PAIR_RING];
+};
+struct PairQueue {
+    PairRing &r;
+    int lane;
+    unsigned head, tail;
+    __device__ PairQueue(PairRing &ring, int l) : r(ring), lane(l), head(0), tail(0) {}
+    __device__ inline unsigned pending() const { return tail - head; }
+    __device__ inline void push(bool in, double x, double y, int code)
+    {
+        const uint64_t mask = __builtin_amdgcn_ballot_w64(in);
+        if (in) {
+            const unsigned below = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+            const unsigned i = (tail + below) & (PAIR_RING - 1);
+            r.x[i] = x;
+            r.y[i] = y;
+            r.code[i] = code;
+        }
+        tail += (unsigned)__popcll(mask);
+    }
+    // evaluates the oldest cnt <= 64 pairs: eval(x, y, code)
+    template <class E>
+    __device__ inline void drain(unsigned cnt, E &&eval)
+    {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if ((unsigned)lane < cnt) {
+            const unsigned i = (head + lane) & (PAIR_RING - 1);
+            eval(r.x[i], r.y[i], r.code[i]);
+        }
+        head += cnt;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+};
+
+// Sum over the wavefront, in lane 63 (DPP shifts within rows of 16 lanes, then row broadcasts).
+template <int CTRL, int ROWS>
+__device__ inline double dpp_add(double v)
+{
+    const uint64_t b = __double_as_longlong(v);
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xf, true);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, ROWS, 0xf, true);
+    return v + __longlong_as_double(((uint64_t)hi << 32) | lo);
+}
+
+__device__ inline double wave_sum63(double v)
+{
+    v = dpp_add<0x111, 0xf>(v);  // row_shr:1
+    v = dpp_add<0x112, 0xf>(v);  // row_shr:2
+    v = dpp_add<0x114, 0xf>(v);  // row_shr:4
+    v = dpp_add<0x118, 0xf>(v);  // row_shr:8
+    v = dpp_add<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+    return dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+}
+
 // Lists of the atoms near a point (near_lists.hip): bins of framework u's cell, and per bin the
 // atoms that a guest with its reference point in the bin can have inside the cutoff. An entry is
 // the atom's index (Morton order, framework-relative) and above it its compact type.
@@ -420,6 +485,7 @@ struct NearDesc {
     int nb[3];
     int bin_off;               // first bin of the framework in `start`
     double r2;                 // squared list radius, Å^2
+    double close2;             // a list's first entries: the atoms within 2 Å of any site in the bin
     double reach[3];           // list radius over the perpendicular widths
 };
 struct NearLists {
@@ -438,6 +504,56 @@ __device__ inline int near_bin(const NearDesc &D, const double f[3])
         c[d] = min(D.nb[d] - 1, (int)(x * D.nb[d]));
     }
     return D.bin_off + c[0] + D.nb[0] * (c[1] + D.nb[1] * c[2]);
+}
+
+// One wavefront's host-guest pairs inside the cutoff, from the near list of `bin`: the guest's sites
+// at fractional coordinates f, pairs queued as (r^2, KE q_site q_atom, site * ntypes_c + type) and
+// evaluated by `eval`. With rho2 (squared radii by the same code) the first 64 entries, which hold
+// the atoms close to the bin, are tested first: true if a site lies inside one, with nothing
+// more evaluated.
+template <int NS, bool UPPER, class E>
+__device__ inline bool near_scan(const NearLists &L, const FwDesc &F, int bin, const double (&f)[NS][3],
+                                 const double *q, int ntypes_c, double rc_max2, const double *rho2, PairQueue &Q,
+                                 E &&eval)
+{
+    const double nan = __builtin_nan("");
+    const double4 *af = L.atomf + F.atom_off;
+    const int e0 = L.start[bin], ne = L.start[bin + 1] - e0, lane = Q.lane;
+    const uint32_t *ent = L.ent + e0;
+    // the next entry and its atom are loaded while the current one is evaluated; a lane past the
+    // list's end takes a NaN position, which is inside nothing
+    uint32_t en = lane < ne ? ent[lane] : 0u;
+    double4 hn = lane < ne ? af[en & NEAR_INDEX] : make_double4(nan, nan, nan, 0.0);
+#pragma unroll 1
+    for (int jb = 0; jb < ne; jb += 64) {
+        const double4 h = hn;
+        const int ht = (int)(en >> NEAR_TYPE_SHIFT), j = jb + lane + 64;
+        hn = make_double4(nan, nan, nan, 0.0);
+        if (j < ne) {
+            en = ent[j];
+            hn = af[en & NEAR_INDEX];
+        }
+        double r2[NS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) r2[s] = cw_r2_t<UPPER>(F.A, f[s][0] - h.x, f[s][1] - h.y, f[s][2] - h.z);
+        if (rho2 && jb == 0) {
+            bool hit = false;
+#pragma unroll
+            for (int s = 0; s < NS; ++s) hit = hit || r2[s] < rho2[s * ntypes_c + ht];
+            if (__builtin_amdgcn_ballot_w64(hit)) return true;
+        }
+        const double qh = KE * h.w;
+#pragma unroll
+        for (int s0 = 0; s0 < NS; s0 += 3) {
+#pragma unroll
+            for (int s = s0; s < (s0 + 3 < NS ? s0 + 3 : NS); ++s)
+                Q.push(r2[s] < rc_max2, r2[s], q[s] * qh, s * ntypes_c + ht);
+#pragma unroll 1
+            while (Q.pending() >= 64) Q.drain(64, eval);
+        }
+    }
+    Q.drain(Q.pending(), eval);
+    return false;
 }
 
 // Move types of the move path: the reference's three NVT moves (src/moves.jl:69-71) and the two

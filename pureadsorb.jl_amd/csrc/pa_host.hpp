@@ -190,6 +190,8 @@ struct pa_batch {
     // and the largest per system
     double rr_kT = -1.0;
     std::vector<double> rr_r2, rr_max2;
+    double rr64_kT = -1.0;  // the same with the FP64 path's rounding allowance
+    std::vector<double> rr64_r2;
     // force field as given, compact type map and per-framework host tables (gradients)
     int nt_ff = 0, ff_tail = 0;
     std::vector<double> ff_sigma, ff_eps;
@@ -220,7 +222,7 @@ struct pa_batch {
     pa::DevAlloc d_corefx, d_coreidx, d_cell_start, d_rho2, d_cand, d_ncand, d_nbr_start, d_nbr_atoms, d_passes;
     pa::DevAlloc d_binfx, d_bintype;  // the atoms in Morton order, for the mixed path's list build
     // FP64 paths: lists of the atoms near a point, built on first use (near_lists.hip)
-    pa::DevAlloc d_nearf, d_neart, d_near_desc, d_near_start, d_near_ent;
+    pa::DevAlloc d_nearf, d_neart, d_near_desc, d_near_start, d_near_ent, d_rho2_64;
     bool near_ready = false;
     // gradient scratch
     pa::PinnedAlloc h_acc_q;  // gradient path: the per-atom charge accumulators read back

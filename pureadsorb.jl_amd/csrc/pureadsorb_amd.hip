@@ -19,6 +19,8 @@
 
 namespace pa {
 hipError_t launch_energy(const WidomArgs &a, int precision, bool upper, hipStream_t st);
+hipError_t launch_near(const WidomArgs &a, const NearLists &L, const double *rho2, bool upper, int tab_w, hipStream_t st);
+int near_tab_max(int ns);
 hipError_t launch_tiles(const double *dU, const int64_t *tile_g0, const int *tile_n, int ntiles, double kT, double4 *out,
                         hipStream_t st);
 hipError_t launch_poses(const FwDesc *fw, const int *fw_of, int sys, uint64_t seed, int64_t j0, int64_t n, double *pos,
@@ -1370,11 +1372,34 @@ static int run_energies(pa_batch *b, const std::vector<int64_t> &seg, int64_t gb
         a.seed = seed;
         a.dU = dU;
         a.out_base = out_base;
+        // two-phase calls (kT > 0) go over the near lists, which the first of them builds; a call
+        // into a fixed scratch region uses them only if they are there. Single energies and
+        // PA_SINGLE_PHASE calls take the plain kernel.
+        int tab_w = 0;
+        for (const FwDesc &D : b->desc) tab_w = std::max(tab_w, D.kn_max[0] + D.kn_max[1] + D.kn_max[2] + 3);
+        bool near = kT > 0.0 && (!b->gdev.charged || tab_w <= near_tab_max(b->nsites));
+        if (near && !b->near_ready) near = !scr.base && ensure_near_lists(b) == PA_OK;
+        double *d_r2 = nullptr;
+        if (near) {
+            const size_t per_sys = (size_t)b->nsites * b->ntypes_c;
+            if (b->rr64_kT != kT) {
+                // a system without a valid radius rejects nothing
+                b->rr64_r2.assign((size_t)nsys * per_sys, 0.0);
+                for (int s = 0; s < nsys; ++s) {
+                    double rmax2 = 0.0;
+                    if (rejection_radii(b, s, kT, DBL_EPSILON, b->rr64_r2.data() + s * per_sys, &rmax2))
+                        std::fill_n(b->rr64_r2.begin() + s * per_sys, per_sys, 0.0);
+                }
+                b->rr64_kT = kT;
+            }
+            SCR_TRY(b, scr.put(b->d_rho2_64, b->rr64_r2, &d_r2));
+        }
         for (int64_t g0 = gb; g0 < ge; g0 += CH) {
             a.g0 = g0;
             a.g1 = std::min(ge, g0 + CH);
             if (timed) HIP_TRY(hipEventRecord(b->kev[2 * *launches], b->stream));
-            HIP_TRY(launch_energy(a, (int)precision, b->upper_all, b->stream));
+            if (near) HIP_TRY(launch_near(a, near_lists(b), d_r2, b->upper_all, tab_w, b->stream));
+            else HIP_TRY(launch_energy(a, (int)precision, b->upper_all, b->stream));
             if (timed) HIP_TRY(hipEventRecord(b->kev[2 * *launches + 1], b->stream));
             ++*launches;
         }
@@ -1702,8 +1727,7 @@ static int widom_core(pa_batch *b, const pa_guest *guest, double T, int64_t nins
     }
     HIP_TRY(hipEventRecord(b->ev[0], b->stream));
     int64_t launches = 0;
-    // the mixed path runs phase 0 (hard-core rejection) unless PA_SINGLE_PHASE; the FP64 plain
-    // path evaluates every insertion
+    // phase 0 (hard-core rejection) unless PA_SINGLE_PHASE
     st = run_energies(b, seg, 0, G, 0, seed, precision, chunk, &launches, kT_phase0, dU);
     if (st) return st;
     HIP_TRY(hipEventRecord(b->ev[1], b->stream));
