@@ -31,10 +31,9 @@ struct pa_state {
     DevAlloc d_guest_off, d_occ, d_refpos, d_quat, d_host_e, d_gsite, d_Sk, d_skabs, d_sk_off, d_energy, d_energy_abs,
         d_seed, d_counter, d_acc, d_att, d_step_t, d_step_r, d_log_fugV, d_logn, d_cp, d_cq, d_samp_e, d_samp_n, d_maxocc,
         d_caphit, d_trace;
-    // NVT driver: fractional atom table, insertion constant per system, move-launch snapshots,
+    // NVT driver: insertion constant per system, move-launch snapshots,
     // test-insertion scratch, and the per-cycle records of the last run (nsys x nvt_np)
-    DevAlloc d_chunk, d_chunk_off, d_lines, d_rounds, d_round_off, d_perm, d_coff,
-        d_half_perp, d_ct, d_snap_pos, d_snap_quat, d_snap_sk, d_snap_occ, d_item_off, d_cw_dU, d_pose_pos,
+    DevAlloc d_coff, d_ct, d_snap_pos, d_snap_quat, d_snap_sk, d_snap_occ, d_item_off, d_cw_dU, d_pose_pos,
         d_pose_quat;
     // the k-vectors' order on the device (KRuns): position of every k-vector within its framework's
     // slice, and the runs
@@ -47,7 +46,6 @@ struct pa_state {
     // reads the guest slots refuses the state until the occupancy is set back
     bool occ_over_capacity = false;
     std::vector<int> occ_live;  // live guests per system when an occupancy was first set over its capacity
-    double cull_extra = 0.0;
     int64_t ctot = 0;       // entries of one snapshot slot's weighted structure factors
     int64_t snap_slots = 0; // slots allocated
     std::vector<double> nvt_E, nvt_sW, nvt_sUW;
@@ -164,8 +162,13 @@ double guest_tail_h(const pa_batch *b, int u, double N)
     const std::vector<double> &cnt = b->fgh[u].counts;
     const double rc = b->rc_lj;
     double acc = 0.0;
+    // only the guest's types y have a term: the others, all of a force field of some hundred types
+    // but two or three, would add zeros (the whole double loop cost 0.1 ms a call)
+    std::vector<int> gy;
+    for (int y = 0; y < NT; ++y)
+        if (g[y] != 0.0) gy.push_back(y);
     for (int x = 0; x < NT; ++x)
-        for (int y = 0; y < NT; ++y) {
+        for (int y : gy) {
             const double e = b->ff_eps[x + NT * y];
             if (e == 0.0) continue;
             const double sg = b->ff_sigma[x + NT * y], r = sg / rc, r3 = r * r * r;
@@ -271,6 +274,20 @@ hipError_t download(std::vector<T> &v, const DevAlloc &d, size_t n)
     return hipMemcpy(v.data(), d.p, sizeof(T) * n, hipMemcpyDeviceToHost);
 }
 
+KRuns k_runs(const pa_state *st)
+{
+    return KRuns{st->d_run.as<int4>(), st->d_run_off.as<int>(), st->d_kbase.as<int>(), st->d_kblk_off.as<int>(),
+                 st->d_kw.as<double>()};
+}
+
+// Entries per site of the widest per-axis phase table.
+int ktab_width(const pa_batch *b)
+{
+    int w = 0;
+    for (const FwDesc &D : b->desc) w = std::max(w, D.kn_max[0] + D.kn_max[1] + D.kn_max[2] + 3);
+    return w;
+}
+
 McArgs base_mc(pa_state *st)
 {
     pa_batch *b = st->b;
@@ -281,10 +298,8 @@ McArgs base_mc(pa_state *st)
     a.atype = b->d_atype.as<int>();
     a.near = near_lists(b);
     a.upper = b->upper_all ? 1 : 0;
-    a.kr = KRuns{st->d_run.as<int4>(), st->d_run_off.as<int>(), st->d_kbase.as<int>(), st->d_kblk_off.as<int>(),
-                 st->d_kw.as<double>()};
-    a.ktab_w = 0;
-    for (const FwDesc &D : b->desc) a.ktab_w = std::max(a.ktab_w, D.kn_max[0] + D.kn_max[1] + D.kn_max[2] + 3);
+    a.kr = k_runs(st);
+    a.ktab_w = ktab_width(b);
     a.pair64 = b->d_pair64.as<double2>();
     a.ntypes_c = b->ntypes_c;
     a.rc_lj2 = b->rc_lj * b->rc_lj;
@@ -1161,105 +1176,14 @@ int build_k_runs(pa_state *st)
     return PA_OK;
 }
 
-// Tables of the chain-insertion kernel, built once per state: every framework's atoms in
-// Morton order, cut into chunks of 64 with a centre and a radius that
-// bounds every atom's nearest-image distance to the centre; the k-vectors cut into runs of
-// consecutive n3 at fixed (n1, n2), longest first; half the smallest perpendicular width.
+// Tables of the move and chain-insertion kernels beyond build_k_runs: the batch's near lists, and
+// each system's slice of a snapshot's structure factors.
 int ensure_chain_tables(pa_state *st)
 {
-    pa_batch *b = st->b;
-    if (st->d_half_perp.p) return PA_OK;
-    if (int e = ensure_near_lists(b)) return e;
-    std::vector<double4> af;
-    std::vector<int> at;
-    if (int e = near_atoms(b, af, at)) return e;
-    std::vector<int> chunk_off(1, 0), round_off(1, 0), perm(std::max<size_t>(b->k64_h.size(), 1), 0),
-        fsize(b->nfw, 0);
-    std::vector<double4> chunks;
-    std::vector<int2> lines, rounds;
-    std::vector<double> halfw(b->nfw);
-    for (int u = 0; u < b->nfw; ++u) {
-        const FwDesc &F = b->desc[u];
-        const FwHost &h = b->info[u];
-        const int n = F.natoms;
-        for (int c0 = 0; c0 < n; c0 += 64) {
-            const int c1 = std::min(n, c0 + 64);
-            const double4 r0 = af[F.atom_off + c0];
-            std::vector<double> uw(3 * (size_t)(c1 - c0));
-            double cen[3] = {0, 0, 0};
-            for (int i = c0; i < c1; ++i) {
-                const double4 p = af[F.atom_off + i];
-                const double d[3] = {p.x - r0.x, p.y - r0.y, p.z - r0.z};
-                for (int e = 0; e < 3; ++e) {
-                    uw[3 * (i - c0) + e] = (e == 0 ? r0.x : e == 1 ? r0.y : r0.z) + (d[e] - std::rint(d[e]));
-                    cen[e] += uw[3 * (i - c0) + e];
-                }
-            }
-            for (int e = 0; e < 3; ++e) cen[e] /= (double)(c1 - c0);
-            double rad = 0.0;
-            for (int i = 0; i < c1 - c0; ++i) {
-                const double d[3] = {uw[3 * i] - cen[0], uw[3 * i + 1] - cen[1], uw[3 * i + 2] - cen[2]};
-                double m[3];
-                matvec(F.A, d, m);
-                rad = std::max(rad, std::sqrt(m[0] * m[0] + m[1] * m[1] + m[2] * m[2]));
-            }
-            chunks.push_back(make_double4(cen[0], cen[1], cen[2], rad * (1.0 + 1e-12) + 1e-9));
-        }
-        chunk_off.push_back((int)chunks.size());
-        // runs of consecutive n3 at fixed (n1, n2), in k-table order, then longest first
-        std::vector<int2> fl;
-        for (int k = 0; k < F.nk; ++k) {
-            const int4 nn = b->kn_h[F.k_off + k];
-            if (k > 0) {
-                const int4 pn = b->kn_h[F.k_off + k - 1];
-                if (nn.x == pn.x && nn.y == pn.y && nn.z == pn.z + 1) {
-                    ++fl.back().y;
-                    continue;
-                }
-            }
-            fl.push_back(make_int2(k, 1));
-        }
-        std::stable_sort(fl.begin(), fl.end(), [](const int2 &x, const int2 &y) { return x.y > y.y; });
-        // rounds of 64 runs (one per lane); step i of lane l in a round sits at base + 64 i + l
-        int base = 0;
-        for (size_t r0 = 0; r0 < fl.size(); r0 += 64) {
-            rounds.push_back(make_int2(base, 0));
-            const int len0 = fl[r0].y;  // longest run of the round
-            for (int l = 0; l < 64; ++l) {
-                const size_t r = r0 + l;
-                if (r < fl.size()) {
-                    lines.push_back(fl[r]);
-                    for (int i = 0; i < fl[r].y; ++i) perm[F.k_off + fl[r].x + i] = base + 64 * i + l;
-                } else {
-                    lines.push_back(make_int2(0, 0));
-                }
-            }
-            base += 64 * len0;
-        }
-        round_off.push_back((int)rounds.size());
-        fsize[u] = base;
-        halfw[u] = 0.5 * std::min({h.perp[0], h.perp[1], h.perp[2]});
-    }
-    const double rcmax = std::max(b->rc_lj, b->gdev.charged ? b->rc_ew : 0.0);
-    st->cull_extra = rcmax + b->r_guest + 1e-6;
-    HIP_TRY(upload(st->d_chunk, chunks));
-    HIP_TRY(upload(st->d_chunk_off, chunk_off));
-    HIP_TRY(upload(st->d_lines, lines));
-    HIP_TRY(upload(st->d_rounds, rounds));
-    HIP_TRY(upload(st->d_round_off, round_off));
-    // by position, as the running structure factors are stored
-    std::vector<int> perm_pos(perm.size(), 0);
-    for (int u = 0; u < b->nfw; ++u)
-        for (int k = 0; k < b->desc[u].nk; ++k) {
-            const int k0 = b->desc[u].k_off;
-            perm_pos[k0 + st->kpos[k0 + k]] = perm[k0 + k];
-        }
-    HIP_TRY(upload(st->d_perm, perm_pos));
-    std::vector<int> coff(st->nsys + 1, 0);
-    for (int n = 0; n < st->nsys; ++n) coff[n + 1] = coff[n] + fsize[b->fw_of[n]];
-    st->ctot = coff[st->nsys];
-    HIP_TRY(upload(st->d_coff, coff));
-    HIP_TRY(upload(st->d_half_perp, halfw));
+    if (st->d_coff.p) return PA_OK;
+    if (int e = ensure_near_lists(st->b)) return e;
+    st->ctot = st->sk_off[st->nsys];
+    HIP_TRY(upload(st->d_coff, st->sk_off));
     return PA_OK;
 }
 
@@ -1270,7 +1194,6 @@ ChainSnap chain_snap(pa_state *st)
     S.nslots = st->guest_off[st->nsys];
     S.ctot = st->ctot;
     S.coff = st->d_coff.as<int>();
-    S.perm = st->d_perm.as<int>();
     S.occ = st->d_snap_occ.as<int>();
     S.pos = st->d_snap_pos.as<double4>();
     S.quat = st->d_snap_quat.as<double4>();
@@ -1284,18 +1207,10 @@ ChainWidomArgs base_chain_widom(pa_state *st)
     ChainWidomArgs a{};
     a.fw = b->d_fw.as<FwDesc>();
     a.fw_of = b->d_fw_of.as<int>();
-    a.atomf64 = b->d_nearf.as<double4>();
-    a.atype = b->d_neart.as<int>();
-    a.chunk = st->d_chunk.as<double4>();
-    a.chunk_off = st->d_chunk_off.as<int>();
-    a.lines = st->d_lines.as<int2>();
-    a.rounds = st->d_rounds.as<int2>();
-    a.round_off = st->d_round_off.as<int>();
-    a.half_perp = st->d_half_perp.as<double>();
-    a.cull_extra = st->cull_extra;
+    a.near = near_lists(b);
+    a.kr = k_runs(st);
+    a.ktab_w = ktab_width(b);
     a.upper = b->upper_all ? 1 : 0;
-    a.k64 = b->d_k64.as<double4>();
-    a.kn = b->d_kn.as<int4>();
     a.pair64 = b->d_pair64.as<double2>();
     a.ntypes_c = b->ntypes_c;
     a.rc_lj2 = b->rc_lj * b->rc_lj;

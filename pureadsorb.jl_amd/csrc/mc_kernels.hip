@@ -347,11 +347,10 @@ __global__ __launch_bounds__(SPEC *GNW * 64) void mc_chain_kernel(McArgs a)
         for (int64_t cs = pend0; cs < pend0 + npend; ++cs) {
             const auto &S = rare()->snap;
             double2 *dsk = S.csk + cs * S.ctot + S.coff[n];
-            const int *perm = S.perm + F.k_off;
             for (int k = tid; k < nk; k += WG) {
                 const double w = kw[k];
                 const double2 v = Sk[k];
-                dsk[perm[k]] = make_double2(w * v.x, w * v.y);
+                dsk[k] = make_double2(w * v.x, w * v.y);
             }
             double4 *dp = S.pos + cs * S.nslots + gr0, *dq = S.quat + cs * S.nslots + gr0;
             for (int i = tid; i < occ; i += WG) {

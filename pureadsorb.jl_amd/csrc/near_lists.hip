@@ -91,7 +91,7 @@ static uint32_t spread3(uint32_t v)
 
 // Every framework's atoms (fractional coordinates in [0, 1), charge; compact type) in Morton
 // order of a ~4 Å cell grid, so that 64 consecutive atoms lie close together.
-int near_atoms(const pa_batch *b, std::vector<double4> &af, std::vector<int> &at)
+static int near_atoms(const pa_batch *b, std::vector<double4> &af, std::vector<int> &at)
 {
     const size_t na = std::max<size_t>(b->atom64_h.size(), 1);
     af.assign(na, make_double4(0, 0, 0, 0));

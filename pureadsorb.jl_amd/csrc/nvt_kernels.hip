@@ -8,210 +8,202 @@
 // (the host adds insertion_constant_term, src/nvt.jl:44-66).
 //
 // One wavefront per insertion:
-//   * host-guest: the framework's atoms are stored in spatially compact chunks of 64 (one atom
-//     per lane); pairs inside the cutoff are compacted through LDS before the LJ + erfc
-//     evaluation. A chunk whose centre lies farther than its radius + guest radius + cutoff from
-//     the insertion's reference point is skipped whole. The distance is a lower bound of the
-//     true nearest-image distance: the rint image is the nearest one whenever it is shorter
-//     than half the smallest perpendicular width, so min(rint distance, half width) never
-//     exceeds the true distance; and with widths >= 2 * cutoff every pair within the cutoff
-//     is found by the per-pair rint image the energy uses.
-//   * reciprocal: k = 2 pi A^-T n is enumerated n1 outer, n2, n3 inner ascending (kvectors,
-//     src/ewald.jl:142-157), so the k-vectors fall into runs of consecutive n3 at fixed
-//     (n1, n2). Each lane takes whole runs (longest first, so the lanes' trip counts match):
-//     one sincospi of 2 pi n.f per site at the start of a run, then one complex multiply by
-//     e^{2 pi i f3} per further k-vector (f = A^-1 r). The snapshot stores kprefactor * S in
-//     the lanes' reading order, so each step is one coalesced load.
-//   * guest-guest: lanes take (guest, site, site) triples.
-// The lanes' partial sums are reduced across the wavefront in a fixed order. The pose is drawn
-// exactly as the Widom path draws it; the energy terms use fused multiply-adds.
+//   * host-guest: the near list of the insertion's bin (near_lists.hip), pairs inside the cutoff
+//     queued in LDS and evaluated 64 at a time;
+//   * reciprocal: the chain's k-vectors in the order of the move kernel (KRuns), one run of
+//     consecutive n3 per lane, walked from its middle. The pair m +- j of a run whose middle has
+//     the phase x = e^{2 pi i (n1 f1 + n2 f2 + m f3)} adds, with z = e^{2 pi i j f3} and the
+//     snapshot's c = kprefactor S,
+//       x_r [z_r (c+_r + c-_r) + z_i (c+_i - c-_i)] + x_i [z_r (c+_i + c-_i) + z_i (c-_r - c+_r)],
+//     so the brackets are summed over j first: 4 fused multiply-adds per site for two k-vectors
+//     (a recurrence with one complex product per k-vector and site took 8 each). Phases come from
+//     per-axis tables in LDS;
+//   * guest-guest: lanes take (guest, site) pairs against every site, through the same queue.
+// The pose is drawn exactly as the Widom path draws it, `per` insertions of a wavefront one per
+// lane; the energy terms use fused multiply-adds. FP64 issue bounds it: CW_TIME_NOTE
 #include "pa_device.hpp"
 
 namespace pa {
 
-constexpr int CW_WG = 256;
-constexpr int CW_NW = CW_WG / 64;
-
-__device__ inline double cw_wave_sum(double v)
-{
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
-constexpr int CW_RING = 128;  // per-wavefront ring of in-cutoff pairs (< 64 pending + one append)
+constexpr int CW_NW = 4;
+constexpr int CW_BATCH = 16;  // insertions of one wavefront
 
 // Guests of up to three sites fit 4 wavefronts per SIMD without spilling; larger guests keep
 // the compiler's own register budget.
 template <int NS, bool UPPER>
-__global__ __launch_bounds__(CW_WG, (NS <= 3 ? 4 : 1)) void chain_widom_kernel(ChainWidomArgs a)
+__global__ __launch_bounds__(64 * CW_NW, (NS <= 3 ? 4 : 1)) void chain_widom_kernel(ChainWidomArgs a, int per)
 {
-    __shared__ double ring_r2[CW_NW][CW_RING], ring_qq[CW_NW][CW_RING];
-    __shared__ int ring_code[CW_NW][CW_RING];
-    const int lane = threadIdx.x & 63;
-    const int64_t item = (int64_t)blockIdx.x * CW_NW + (threadIdx.x >> 6);
-    if (item >= a.nitems) return;  // whole wavefront; the kernel has no barrier
-    int lo = 0, hi = a.nsys - 1;
-    while (lo < hi) {  // system of the item: item_off[s] <= item < item_off[s+1]
-        const int mid = (lo + hi + 1) >> 1;
-        if (a.item_off[mid] <= item) lo = mid; else hi = mid - 1;
-    }
-    const int s = lo;
-    const int64_t local = item - a.item_off[s];
-    const int64_t cl = local / a.nw, t = local - cl * a.nw;
-    const int u = a.fw_of[s];
-    const FwDesc &F = a.fw[u];
+    __shared__ PairRing rings[CW_NW];
+    __shared__ double wf[CW_NW][CW_BATCH][3 * NS];
+    __shared__ int wsys[CW_NW][CW_BATCH], wbin[CW_NW][CW_BATCH];
+    extern __shared__ double2 tabs[];  // per wavefront, with charges: (ktab_w x NS) phases e^{2 pi i m f_d}
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nwv = blockDim.x >> 6;
+    const int64_t first = ((int64_t)blockIdx.x * nwv + wv) * per;
+    if (first >= a.nitems) return;  // whole wavefront; the kernel has no barrier
+    const int cnt = (int)(a.nitems - first < per ? a.nitems - first : per);
     const GuestDev &G = a.guest;
-
-    // the state this insertion sees: the snapshot of its cycle slot
     const ChainSnap &S = a.snap;
-    const int64_t slot = cl < a.snap_n ? cl : a.snap_n - 1;
-    const int gr0 = a.guest_off[s];
-    const int occ = S.occ[slot * S.nsys + s];
-    const double4 *gpos = S.pos + slot * S.nslots + gr0;
-    const double4 *gquat = S.quat + slot * S.nslots + gr0;
-    const double2 *csk = S.csk + slot * S.ctot + S.coff[s];
-
-    double pos[3], q[4];
-    if (a.pose_pos) {
-        for (int d = 0; d < 3; ++d) pos[d] = a.pose_pos[3 * item + d];
-        for (int d = 0; d < 4; ++d) q[d] = a.pose_quat[4 * item + d];
-    } else {
-        double f[3];
-        pose_uniforms(a.widom_seed, s, (a.cyc0 + cl) * a.nw + t, f, q);
-        matvec(F.A, f, pos);
+    if (lane < cnt) {
+        const int64_t item = first + lane;
+        int lo = 0, hi = a.nsys - 1;
+        while (lo < hi) {  // system of the item: item_off[s] <= item < item_off[s+1]
+            const int mid = (lo + hi + 1) >> 1;
+            if (a.item_off[mid] <= item) lo = mid; else hi = mid - 1;
+        }
+        const int u = a.fw_of[lo];
+        const FwDesc &F = a.fw[u];
+        double pos[3], q[4], pf[3];
+        if (a.pose_pos) {
+            for (int d = 0; d < 3; ++d) pos[d] = a.pose_pos[3 * item + d];
+            for (int d = 0; d < 4; ++d) q[d] = a.pose_quat[4 * item + d];
+        } else {
+            double f[3];
+            pose_uniforms(a.widom_seed, lo, a.cyc0 * a.nw + (item - a.item_off[lo]), f, q);
+            matvec(F.A, f, pos);
+        }
+        matvec(F.invA, pos, pf);
+        for (int t = 0; t < NS; ++t) {
+            double r[3], x[3], f[3];
+            rotate(q, G.site[t], r);
+            for (int d = 0; d < 3; ++d) x[d] = pos[d] + r[d];
+            matvec(F.invA, x, f);
+            for (int d = 0; d < 3; ++d) wf[wv][lane][3 * t + d] = f[d];
+        }
+        wsys[wv][lane] = lo;
+        wbin[wv][lane] = near_bin(a.near.desc[u], pf);
     }
-    double pf[3], sc[NS][3], sf[NS][3];
-    matvec(F.invA, pos, pf);
+    auto fence = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    fence();
+    double2 *tab = tabs + (size_t)wv * NS * a.ktab_w;
+    PairQueue Q(rings[wv], lane);
+#pragma unroll 1
+    for (int i = 0; i < cnt; ++i) {
+        const int s = __builtin_amdgcn_readfirstlane(wsys[wv][i]), bin = __builtin_amdgcn_readfirstlane(wbin[wv][i]);
+        const int u = a.fw_of[s];
+        const FwDesc &F = a.fw[u];
+        // the state this insertion sees: the snapshot of its cycle slot
+        const int64_t cl = (first + i - a.item_off[s]) / a.nw;
+        const int64_t slot = cl < a.snap_n ? cl : a.snap_n - 1;
+        const int gr0 = a.guest_off[s], occ = S.occ[slot * S.nsys + s];
+        double f[NS][3];
 #pragma unroll
-    for (int x = 0; x < NS; ++x) {
-        double r[3];
-        rotate(q, G.site[x], r);
-        for (int d = 0; d < 3; ++d) sc[x][d] = pos[d] + r[d];
-        matvec(F.invA, sc[x], sf[x]);
-    }
-    double e = 0.0;
-
-    // (1) host-guest real space, chunk by chunk. The (site, atom) pairs inside the cutoff are
-    // appended to the wavefront's ring in LDS and evaluated 64 at a time, one per lane, so the
-    // LJ + erfc work runs on full wavefronts whatever the lanes' own pairs do.
-    {
-        const int w = threadIdx.x >> 6;
-        double *qr2 = ring_r2[w], *qqq = ring_qq[w];
-        int *qcode = ring_code[w];
-        unsigned head = 0, tail = 0;
-        auto drain = [&](unsigned n) {
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            if ((unsigned)lane < n) {
-                const unsigned i = (head + lane) & (CW_RING - 1);
-                const int code = qcode[i];
-                const double2 p = a.pair64[code];
-                e += cw_pair(qr2[i], p.x * p.x, 4.0 * p.y, qqq[i], F.alpha, a.rc_lj2, a.rc_ew2);
-            }
-            head = __builtin_amdgcn_readfirstlane(head + n);
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        for (int t = 0; t < NS; ++t)
+            for (int d = 0; d < 3; ++d) f[t][d] = wf[wv][i][3 * t + d];
+        double e = 0.0;
+        const double alpha = F.alpha;
+        auto eval = [&](double r2, double qq, int code) {
+            const double2 p = a.pair64[code];
+            e += cw_pair(r2, p.x * p.x, 4.0 * p.y, qq, alpha, a.rc_lj2, a.rc_ew2);
         };
-        const int c0 = a.chunk_off[u], c1 = a.chunk_off[u + 1];
-        const double halfw = a.half_perp[u];
-        const double4 *af = a.atomf64 + F.atom_off;
-        const int *types = a.atype + F.atom_off;
-        const double nan = __builtin_nan("");
+        // (1) host-guest real space
+        near_scan<NS, UPPER>(a.near, F, bin, f, G.q, a.ntypes_c, a.rc_max2, nullptr, Q, eval);
+        // (2) guest-guest real space
+        const double4 *gpos = S.pos + slot * S.nslots + gr0, *gquat = S.quat + slot * S.nslots + gr0;
 #pragma unroll 1
-        for (int c = c0; c < c1; ++c) {
-            const double4 cc = a.chunk[c];
-            const double dist = fmin(__builtin_sqrt(cw_r2_t<UPPER>(F.A, pf[0] - cc.x, pf[1] - cc.y, pf[2] - cc.z)), halfw);
-            // the same value in every lane (one insertion per wavefront): a uniform branch
-            if (__builtin_amdgcn_readfirstlane((int)(dist > cc.w + a.cull_extra))) continue;
-            const int j = (c - c0) * 64 + lane;
-            // lanes past the last atom take a NaN position, whose r2 fails every cutoff test
-            const double4 h = j < F.natoms ? af[j] : make_double4(nan, nan, nan, 0.0);
-            const int ht = j < F.natoms ? types[j] : 0;
+        for (int xb = 0; xb < occ * NS; xb += 64) {
+            const int x = xb + lane, jj = x / NS, sb = x - jj * NS;
+            const double nan = __builtin_nan("");
+            double fb[3] = {nan, nan, nan};
+            if (x < occ * NS) {
+                const double4 p4 = gpos[jj], q4 = gquat[jj];
+                const double qj[4] = {q4.x, q4.y, q4.z, q4.w};
+                double r[3];
+                rotate(qj, G.site[sb], r);
+                const double pb[3] = {p4.x + r[0], p4.y + r[1], p4.z + r[2]};
+                matvec(F.invA, pb, fb);
+            }
+            const double qb = KE * G.q[sb];
+            const int tb = G.type[sb];
 #pragma unroll
-            for (int x = 0; x < NS; ++x) {
-                const double r2 = cw_r2_t<UPPER>(F.A, sf[x][0] - h.x, sf[x][1] - h.y, sf[x][2] - h.z);
-                const bool in = r2 < a.rc_max2;
-                const uint64_t mask = __builtin_amdgcn_ballot_w64(in);
-                if (in) {
-                    const unsigned below = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
-                                                                     __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-                    const unsigned i = (tail + below) & (CW_RING - 1);
-                    qr2[i] = r2;
-                    qqq[i] = KE * G.q[x] * h.w;
-                    qcode[i] = x * a.ntypes_c + ht;
+            for (int s0 = 0; s0 < NS; s0 += 3) {
+#pragma unroll
+                for (int sa = s0; sa < (s0 + 3 < NS ? s0 + 3 : NS); ++sa) {
+                    const double r2 = cw_r2_t<UPPER>(F.A, f[sa][0] - fb[0], f[sa][1] - fb[1], f[sa][2] - fb[2]);
+                    Q.push(r2 < a.rc_max2, r2, G.q[sa] * qb, sa * a.ntypes_c + tb);
                 }
-                tail = __builtin_amdgcn_readfirstlane(tail + (unsigned)__popcll(mask));
-                if (tail - head >= 64) drain(64);
+#pragma unroll 1
+                while (Q.pending() >= 64) Q.drain(64, eval);
             }
         }
-        drain(tail - head);
-    }
-    // (2) reciprocal cross term, whole runs of consecutive n3 per lane; step i of round R reads
-    // the weighted structure factor at round base + 64 i + lane (consecutive across the lanes)
-    if (G.charged) {
-        const int4 *kn = a.kn + F.k_off;
-        const int r0 = a.round_off[u], r1 = a.round_off[u + 1];
-        double str[NS], sti[NS];
-#pragma unroll
-        for (int x = 0; x < NS; ++x) sincospi(2.0 * sf[x][2], &sti[x], &str[x]);
-        double acc = 0.0;
+        Q.drain(Q.pending(), eval);
+        // (3) reciprocal cross term
+        if (G.charged) {
+            const int m0 = F.kn_max[0] + 1, m1 = F.kn_max[1] + 1, tw = m0 + m1 + F.kn_max[2] + 1;
+            const float inv_tw = 1.0f / (float)tw;
 #pragma unroll 1
-        for (int R = r0; R < r1; ++R) {
-            const int2 ln = a.lines[(int64_t)R * 64 + lane];
-            if (ln.y == 0) continue;
-            const double2 *cr = csk + a.rounds[R].x + lane;
-            const int4 nn = kn[ln.x];
-            double zr[NS], zi[NS];
-#pragma unroll
-            for (int x = 0; x < NS; ++x)
-                sincospi(2.0 * (((double)nn.x * sf[x][0] + (double)nn.y * sf[x][1]) + (double)nn.z * sf[x][2]), &zi[x],
-                         &zr[x]);
+            for (int x = lane; x < NS * tw; x += 64) {
+                const int t = (int)(((float)x + 0.5f) * inv_tw), c = x - t * tw;
+                const int d = c < m0 ? 0 : (c < m0 + m1 ? 1 : 2);
+                tab[c * NS + t] = axis_power_const(wf[wv][i][3 * t + d], c - (d == 0 ? 0 : (d == 1 ? m0 : m0 + m1)));
+            }
+            fence();
+            const int4 *runs = a.kr.run + a.kr.run_off[u];
+            const int nruns = a.kr.run_off[u + 1] - a.kr.run_off[u];
+            // c = kprefactor S through buffer loads: zero past the end, for lanes without a k-vector
+            const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
+                (void *)(S.csk + slot * S.ctot + S.coff[s]), (short)0, F.nk * 16, 0x00020000);
+            auto load = [&](int p, int n) {
+                const uint32_t at = lane < n ? (uint32_t)(p + lane) : 0x07FFFFFFu;
+                return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(rc, (int)(at * 16u), 0, 0));
+            };
+            double acc = 0.0;
+            int pos = 0;
 #pragma unroll 1
-            for (int i = 0; i < ln.y; ++i) {
-                if (i > 0) {
+            for (int r0 = 0; r0 < nruns; r0 += 64) {
+                const int4 run = r0 + lane < nruns ? runs[r0 + lane] : make_int4(0, 0, 0, 0);
+                const int L = run.w;
+                auto count = [&](int l) { return (int)__popcll(__builtin_amdgcn_ballot_w64(L >= l)); };
+                const int n0 = count(1);
+                const double2 c0 = load(pos, n0);
+                pos += n0;
+                int np = count(2), nm = count(3);
+                double2 cp = load(pos, np), cm = load(pos + np, nm);
+                double v1[NS], v2[NS];
 #pragma unroll
-                    for (int x = 0; x < NS; ++x) {
-                        const double r = __builtin_fma(zr[x], str[x], -(zi[x] * sti[x]));
-                        const double im = __builtin_fma(zr[x], sti[x], zi[x] * str[x]);
-                        zr[x] = r;
-                        zi[x] = im;
+                for (int t = 0; t < NS; ++t) {
+                    v1[t] = c0.x;
+                    v2[t] = c0.y;
+                }
+                const double2 *tj = tab + (m0 + m1 + 1) * NS;
+#pragma unroll 1
+                for (int j = 2; np > 0; ++j) {
+                    double2 z[NS];
+#pragma unroll
+                    for (int t = 0; t < NS; ++t) z[t] = tj[t];
+                    tj += NS;
+                    pos += np + nm;
+                    np = count(2 * j);
+                    nm = count(2 * j + 1);
+                    const double2 cp2 = load(pos, np), cm2 = load(pos + np, nm);
+                    __builtin_amdgcn_sched_barrier(0);
+                    const double P = cp.x + cm.x, T = cp.y + cm.y, R = cp.y - cm.y, N = cm.x - cp.x;
+#pragma unroll
+                    for (int t = 0; t < NS; ++t) {
+                        v1[t] = __builtin_fma(z[t].x, P, __builtin_fma(z[t].y, R, v1[t]));
+                        v2[t] = __builtin_fma(z[t].x, T, __builtin_fma(z[t].y, N, v2[t]));
                     }
+                    cp = cp2;
+                    cm = cm2;
                 }
-                double gre = 0.0, gim = 0.0;
+                const double2 *tx = tab + abs(run.x) * NS, *ty = tab + (m0 + abs(run.y)) * NS,
+                              *tz = tab + (m0 + m1 + abs(run.z)) * NS;
 #pragma unroll
-                for (int x = 0; x < NS; ++x) {
-                    gre = __builtin_fma(G.q[x], zr[x], gre);
-                    gim = __builtin_fma(G.q[x], zi[x], gim);
+                for (int t = 0; t < NS; ++t) {
+                    const double2 x = cis_from_axes(tx[t], ty[t], tz[t], run.x, run.y, run.z);
+                    acc = __builtin_fma(G.q[t], __builtin_fma(x.x, v1[t], x.y * v2[t]), acc);
                 }
-                const double2 c = cr[(int64_t)i * 64];
-                acc = __builtin_fma(c.x, gre, __builtin_fma(c.y, gim, acc));
             }
+            e = __builtin_fma(2.0 * KE, acc, e);
+            fence();
         }
-        e += KE * (2.0 * acc);
+        e = wave_sum63(e);
+        if (lane == 63) a.dU[first + i] = e;
     }
-    // (3) guest-guest real space, one (guest, site, site) triple per lane step
-    const int ntrip = occ * NS * NS;
-#pragma unroll 1
-    for (int xi = lane; xi < ntrip; xi += 64) {
-        const int jj = xi / (NS * NS), sa = (xi / NS) % NS, sb = xi % NS;
-        const double4 p4 = gpos[jj], q4 = gquat[jj];
-        const double qj[4] = {q4.x, q4.y, q4.z, q4.w};
-        double r[3];
-        rotate(qj, G.site[sb], r);
-        const double pb[3] = {p4.x + r[0], p4.y + r[1], p4.z + r[2]};
-        double fb[3];
-        matvec(F.invA, pb, fb);
-        const double r2 = cw_r2_t<UPPER>(F.A, sf[sa][0] - fb[0], sf[sa][1] - fb[1], sf[sa][2] - fb[2]);
-        if (r2 < a.rc_lj2 || r2 < a.rc_ew2) {
-            const double2 p = a.pair64[sa * a.ntypes_c + G.type[sb]];
-            e += cw_pair(r2, p.x * p.x, 4.0 * p.y, KE * G.q[sa] * G.q[sb], F.alpha, a.rc_lj2, a.rc_ew2);
-        }
-    }
-
-    e = cw_wave_sum(e);
-    if (lane == 0) a.dU[item] = e;
 }
 
 // Snapshot slot `slot` of every system's live state (after an audit, or for insertions at
@@ -226,12 +218,11 @@ __global__ __launch_bounds__(256) void chain_snapshot_kernel(ChainSnap S, int64_
     const FwDesc &F = fw[fw_of[n]];
     const double *kw = kw_all + F.k_off;
     const double2 *sk = Sk + sk_off[n];
-    const int *perm = S.perm + F.k_off;
     double2 *dsk = S.csk + slot * S.ctot + S.coff[n];
     for (int k = tid; k < F.nk; k += 256) {
         const double w = kw[k];
         const double2 v = sk[k];
-        dsk[perm[k]] = make_double2(w * v.x, w * v.y);
+        dsk[k] = make_double2(w * v.x, w * v.y);
     }
     const int gr0 = guest_off[n], occ = occupancy[n];
     for (int i = tid; i < occ; i += 256) {
@@ -248,23 +239,32 @@ hipError_t launch_chain_snapshot(const ChainSnap &S, int64_t slot, const McArgs 
     return hipGetLastError();
 }
 
+template <int NS>
+static void launch_chain_widom_ns(const ChainWidomArgs &a, int per, int nwv, hipStream_t st)
+{
+    const dim3 grid((unsigned)(((a.nitems + per - 1) / per + nwv - 1) / nwv)), block((unsigned)(64 * nwv));
+    const size_t lds = a.guest.charged ? sizeof(double2) * nwv * NS * a.ktab_w : 0;
+    if (a.upper) hipLaunchKernelGGL((chain_widom_kernel<NS, true>), grid, block, lds, st, a, per);
+    else hipLaunchKernelGGL((chain_widom_kernel<NS, false>), grid, block, lds, st, a, per);
+}
+
 hipError_t launch_chain_widom(const ChainWidomArgs &a, hipStream_t st)
 {
     if (a.nitems <= 0) return hipSuccess;
-    const dim3 grid((unsigned)((a.nitems + CW_NW - 1) / CW_NW)), block(CW_WG);
-    switch (a.guest.nsites * 2 + (a.upper ? 1 : 0)) {
-    case 2: hipLaunchKernelGGL((chain_widom_kernel<1, false>), grid, block, 0, st, a); break;
-    case 3: hipLaunchKernelGGL((chain_widom_kernel<1, true>), grid, block, 0, st, a); break;
-    case 4: hipLaunchKernelGGL((chain_widom_kernel<2, false>), grid, block, 0, st, a); break;
-    case 5: hipLaunchKernelGGL((chain_widom_kernel<2, true>), grid, block, 0, st, a); break;
-    case 6: hipLaunchKernelGGL((chain_widom_kernel<3, false>), grid, block, 0, st, a); break;
-    case 7: hipLaunchKernelGGL((chain_widom_kernel<3, true>), grid, block, 0, st, a); break;
-    case 8: hipLaunchKernelGGL((chain_widom_kernel<4, false>), grid, block, 0, st, a); break;
-    case 9: hipLaunchKernelGGL((chain_widom_kernel<4, true>), grid, block, 0, st, a); break;
-    case 10: hipLaunchKernelGGL((chain_widom_kernel<5, false>), grid, block, 0, st, a); break;
-    case 11: hipLaunchKernelGGL((chain_widom_kernel<5, true>), grid, block, 0, st, a); break;
-    case 12: hipLaunchKernelGGL((chain_widom_kernel<6, false>), grid, block, 0, st, a); break;
-    case 13: hipLaunchKernelGGL((chain_widom_kernel<6, true>), grid, block, 0, st, a); break;
+    // the wavefronts of a workgroup share nothing: one where the phase tables of four would not fit
+    const size_t tab = a.guest.charged ? sizeof(double2) * a.guest.nsites * a.ktab_w : 0;
+    if (tab > 100 * 1024) return hipErrorInvalidValue;
+    const int nwv = CW_NW * tab > 100 * 1024 ? 1 : CW_NW;
+    // insertions per wavefront: one until there are some 16 wavefronts for every SIMD
+    int per = 1;
+    while (per < CW_BATCH && a.nitems / (2 * per) >= 16384) per *= 2;
+    switch (a.guest.nsites) {
+    case 1: launch_chain_widom_ns<1>(a, per, nwv, st); break;
+    case 2: launch_chain_widom_ns<2>(a, per, nwv, st); break;
+    case 3: launch_chain_widom_ns<3>(a, per, nwv, st); break;
+    case 4: launch_chain_widom_ns<4>(a, per, nwv, st); break;
+    case 5: launch_chain_widom_ns<5>(a, per, nwv, st); break;
+    case 6: launch_chain_widom_ns<6>(a, per, nwv, st); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

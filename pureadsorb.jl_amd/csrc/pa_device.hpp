@@ -564,14 +564,11 @@ constexpr int NMOVES = 5;
 // Snapshots of the chains' states for the test insertions (nvt_kernels.hip). Slot c holds, per
 // system n: occupancy at occ[c * nsys + n]; guests at pos/quat[c * nslots + guest_off[n] + i];
 // the weighted structure factor c_k = kprefactor_k * S_k of every k-vector at
-// csk[c * ctot + coff[n] + perm[F.k_off + p]] for the k-vector at position p (KRuns), the order
-// in which the insertion kernel's lanes read it (runs of consecutive n3 interleaved across the
-// 64 lanes).
+// csk[c * ctot + coff[n] + p] for the k-vector at position p (KRuns).
 struct ChainSnap {
     int nsys, nslots;
     int64_t ctot;
     const int *coff;           // per system: first entry of its slice of csk
-    const int *perm;           // per k-vector position of the batch: place within its framework's slice
     int *occ;
     double4 *pos, *quat;
     double2 *csk;
@@ -643,22 +640,10 @@ struct McArgs {
 struct ChainWidomArgs {
     const FwDesc *fw;
     const int *fw_of;
-    // framework atoms of every framework re-ordered into spatially compact chunks of 64
-    // (same per-framework offsets as the batch's atom tables)
-    const double4 *atomf64;     // fractional x, y, z and charge
-    const int *atype;           // compact type
-    const double4 *chunk;       // per chunk: centre (fractional x, y, z), radius (Å)
-    const int *chunk_off;       // nfw + 1
-    // k-vectors of every framework grouped into runs of consecutive n3 at fixed (n1, n2),
-    // longest first, 64 runs per round (one per lane; short rounds padded with empty runs)
-    const int2 *lines;          // per (round, lane): first k-vector (framework-relative), length
-    const int2 *rounds;         // per round: first entry of the round in the snapshot slice, 0
-    const int *round_off;       // nfw + 1
-    const double *half_perp;    // per framework: half the smallest perpendicular width (Å)
-    double cull_extra;          // largest cutoff + guest radius + rounding margin (Å)
+    NearLists near;             // the framework atoms near a pose
+    KRuns kr;                   // the k-vectors
+    int ktab_w;                 // max over frameworks of kn_max[0] + kn_max[1] + kn_max[2] + 3
     int upper;                  // every framework's A has A[1] == A[2] == A[5] == 0
-    const double4 *k64;         // kx, ky, kz, kprefactor (every k-vector)
-    const int4 *kn;
     const double2 *pair64;
     int ntypes_c;
     double rc_lj2, rc_ew2;

@@ -247,9 +247,7 @@ struct pa_batch {
 namespace pa {
 // Squared phase-0 rejection radii of system s at kT, NS x ntypes_c (build_rejection_tables).
 int rejection_radii(const pa_batch *b, int s, double kT, double eps_f, double *rho2, double *rmax2);
-// The batch's near lists (near_lists.hip): builds them once; their device form; the Morton-ordered
-// atoms they index.
+// The batch's near lists (near_lists.hip): builds them once; their device form.
 int ensure_near_lists(pa_batch *b);
 NearLists near_lists(const pa_batch *b);
-int near_atoms(const pa_batch *b, std::vector<double4> &af, std::vector<int> &at);
 }  // namespace pa
