@@ -3,6 +3,8 @@
 // over its full k table (src/batch.jl:360-389), both FP64, and the phase-0 near-stencil atom
 // lists. k = 2 pi A^-T n, so e^{i k.r} = e^{2 pi i n.f}
 // with f = A^-1 r; every phase is one own-sincospi of 2 n.f.
+#include <hipcub/hipcub.hpp>
+
 #include "pa_device.hpp"
 
 namespace pa {
@@ -64,12 +66,16 @@ __global__ __launch_bounds__(BK_WG) void self_term_kernel(const int4 *kn, const 
     if (w == 0) partial[(int64_t)blockIdx.x * 64 + lane] = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
 }
 
-// Phase-0 near-stencil lists: for every hard-core cell, the atoms (corefx, sorted by cell) of
-// its neighbour cells in the order i2, i1, i0, written from the cell's nbr_start offset. One
-// wavefront per cell; cell_fw_off (nfw + 1) maps the global cell index to its framework.
-__global__ __launch_bounds__(BK_WG) void nbr_fill_kernel(const FwDesc *fw, int nfw, const int *cell_fw_off, int ncells,
-                                                        const int *cell_start, const int *nbr_start,
-                                                        const uint4 *corefx, uint4 *nbr_atoms)
+// Phase-0 near lists: for every hard-core cell, the atoms within nbr_r of any point of it, by their
+// minimum-image distance to the cell's centre. One wavefront per cell, its lanes over the cells
+// within nbr_reach (each once where the reach goes around the axis). Without FILL the lists are
+// counted into nbr_start; with it they are written in three shells of growing distance, so that
+// an insertion's overlap is usually found among the first entries. cell_fw_off (nfw + 1) maps the
+// global cell index to its framework.
+template <bool FILL>
+__global__ __launch_bounds__(BK_WG) void nbr_kernel(const FwDesc *fw, int nfw, const int *cell_fw_off, int ncells,
+                                                   const int *cell_start, int *nbr_start, const uint4 *corefx,
+                                                   uint4 *nbr_atoms)
 {
     const int lane = threadIdx.x & 63;
     const int g = blockIdx.x * (BK_WG / 64) + (threadIdx.x >> 6);
@@ -79,31 +85,75 @@ __global__ __launch_bounds__(BK_WG) void nbr_fill_kernel(const FwDesc *fw, int n
         const int mid = (lo + hi + 1) >> 1;
         if (cell_fw_off[mid] <= g) lo = mid; else hi = mid - 1;
     }
-    const FwDesc &D = fw[lo];
+    const FwDesc &D = fw[__builtin_amdgcn_readfirstlane(lo)];
     const int c = g - cell_fw_off[lo];
-    const int nc0 = D.cg_nc[0], nc1 = D.cg_nc[1], nc2 = D.cg_nc[2];
-    const int k0 = nc0 < 3 ? nc0 : 3, k1 = nc1 < 3 ? nc1 : 3, k2 = nc2 < 3 ? nc2 : 3;
-    const int h0 = c % nc0, h1 = (c / nc0) % nc1, h2 = c / (nc0 * nc1);
+    const int nc[3] = {D.cg_nc[0], D.cg_nc[1], D.cg_nc[2]};
+    const int h[3] = {c % nc[0], (c / nc[0]) % nc[1], c / (nc[0] * nc[1])};
+    int k[3], first[3];
+    uint32_t x[3];
+    for (int d = 0; d < 3; ++d) {
+        const int w = 2 * D.nbr_reach[d] + 1;
+        k[d] = w < nc[d] ? w : nc[d];
+        first[d] = w < nc[d] ? h[d] - D.nbr_reach[d] + nc[d] : 0;
+        x[d] = to_fixed((h[d] + 0.5) / nc[d]);
+    }
+    const int ncand = k[0] * k[1] * k[2];
     const int *cs = cell_start + D.cg_off;
     const uint4 *src = corefx + D.atom_off;
-    int64_t pos = nbr_start[D.cg_off + c];
-    for (int i2 = 0; i2 < k2; ++i2)
-        for (int i1 = 0; i1 < k1; ++i1)
-            for (int i0 = 0; i0 < k0; ++i0) {
-                const int cc = nbr_cell_axis(h0, i0, k0, nc0) +
-                               nc0 * (nbr_cell_axis(h1, i1, k1, nc1) + nc1 * nbr_cell_axis(h2, i2, k2, nc2));
-                const int b0 = cs[cc], len = cs[cc + 1] - b0;
-                for (int i = lane; i < len; i += 64) nbr_atoms[pos + i] = src[b0 + i];
-                pos += len;
+    const float shell[4] = {-1.0f, 0.36f * D.nbr_thr2, 0.64f * D.nbr_thr2, D.nbr_thr2};
+    int total = 0;
+    const int64_t at0 = FILL ? nbr_start[D.cg_off + c] : 0;
+    for (int sh = 0; sh < (FILL ? 3 : 1); ++sh)
+        for (int i0 = 0; i0 < ncand; i0 += 64) {
+            const int i = i0 + lane;
+            int b0 = 0, len = 0;
+            if (i < ncand) {
+                const int c0 = (first[0] + i % k[0]) % nc[0], c1 = (first[1] + (i / k[0]) % k[1]) % nc[1],
+                          c2 = (first[2] + i / (k[0] * k[1])) % nc[2];
+                const int cc = c0 + nc[0] * (c1 + nc[1] * c2);
+                b0 = cs[cc];
+                len = cs[cc + 1] - b0;
             }
+            for (int j = 0; __builtin_amdgcn_ballot_w64(j < len); ++j) {
+                bool in = false;
+                uint4 at = make_uint4(0u, 0u, 0u, 0u);
+                if (j < len) {
+                    at = src[b0 + j];
+                    const float dx = (float)(int32_t)(x[0] - at.x), dy = (float)(int32_t)(x[1] - at.y),
+                                dz = (float)(int32_t)(x[2] - at.z);
+                    const float ex = D.Af[0] * dx + D.Af[3] * dy + D.Af[6] * dz;
+                    const float ey = D.Af[1] * dx + D.Af[4] * dy + D.Af[7] * dz;
+                    const float ez = D.Af[2] * dx + D.Af[5] * dy + D.Af[8] * dz;
+                    const float r2 = ex * ex + ey * ey + ez * ez;
+                    in = FILL ? r2 > shell[sh] && r2 <= shell[sh + 1] : r2 <= D.nbr_thr2;
+                }
+                const uint64_t m = __builtin_amdgcn_ballot_w64(in);
+                if (FILL && in) nbr_atoms[at0 + total + __popcll(m & ((1ull << lane) - 1ull))] = at;
+                total += __popcll(m);
+            }
+        }
+    if (!FILL && lane == 0) nbr_start[D.cg_off + c] = total;
+    // the slot past a framework's last cell: no atoms
+    if (!FILL && lane == 0 && g + 1 == cell_fw_off[lo + 1]) nbr_start[D.cg_off + c + 1] = 0;
 }
 
-hipError_t launch_nbr_fill(const FwDesc *fw, int nfw, const int *cell_fw_off, int ncells, const int *cell_start,
-                           const int *nbr_start, const uint4 *corefx, uint4 *nbr_atoms, hipStream_t st)
+// Exclusive scan of n counts in place (tmp == nullptr: only the temporary size).
+hipError_t scan_counts(int *counts, int n, void *tmp, size_t *tmp_bytes, hipStream_t st)
+{
+    return hipcub::DeviceScan::ExclusiveSum(tmp, *tmp_bytes, counts, counts, n, st);
+}
+
+hipError_t launch_nbr(bool fill, const FwDesc *fw, int nfw, const int *cell_fw_off, int ncells, const int *cell_start,
+                      int *nbr_start, const uint4 *corefx, uint4 *nbr_atoms, hipStream_t st)
 {
     if (ncells <= 0) return hipSuccess;
-    hipLaunchKernelGGL(nbr_fill_kernel, dim3((unsigned)((ncells + BK_WG / 64 - 1) / (BK_WG / 64))), dim3(BK_WG), 0, st, fw,
-                       nfw, cell_fw_off, ncells, cell_start, nbr_start, corefx, nbr_atoms);
+    const dim3 grid((unsigned)((ncells + BK_WG / 64 - 1) / (BK_WG / 64))), block(BK_WG);
+    if (fill)
+        hipLaunchKernelGGL(nbr_kernel<true>, grid, block, 0, st, fw, nfw, cell_fw_off, ncells, cell_start, nbr_start,
+                           corefx, nbr_atoms);
+    else
+        hipLaunchKernelGGL(nbr_kernel<false>, grid, block, 0, st, fw, nfw, cell_fw_off, ncells, cell_start, nbr_start,
+                           corefx, nbr_atoms);
     return hipGetLastError();
 }
 

@@ -22,6 +22,10 @@ struct FwDesc {
     int cg_off;            // hard-core cell grid: first entry of the framework in cell_start
     int cg_nc[3];          // cells per axis (fractional cell edge 1/cg_nc)
     int kn_max[3];         // largest |n_d| of the framework's k-vectors k = 2 pi A^-T n
+    // phase-0 near lists: each hard-core cell lists every atom within nbr_r (Å) of any point of it,
+    // found by its distance to the cell's centre (nbr_thr2, Å^2) among the cells within nbr_reach
+    float nbr_r, nbr_thr2;
+    int nbr_reach[3];
 };
 
 // The guest, with compact type indices.
@@ -84,7 +88,8 @@ struct BinSys {
     float rlist2;   // (max cutoff + guest radius + bin circumradius + margin)^2, Å^2
     float alt[3];   // an atom with |fractional offset| >= alt[i] on axis i also gets the image
                     // across the cell boundary on that axis (alt >= 0.5: never)
-    int reach[3];   // hard-core stencil half-width in grid cells per axis (reach[0] < 0: no check)
+    int hc_on;      // phase 0 runs: 1 with the cells' near lists, 2 when the largest rejection radius
+                    // exceeds theirs and the insertions they pass go through the full stencil too
     uint32_t hc_rf[3];  // largest rejection radius over the perpendicular width, 32-bit fixed point
                         // and rounded up: a site's hard-core partners lie within +-hc_rf[d];
                         // all ones: that range (plus one cell) reaches around the axis
@@ -157,7 +162,8 @@ struct BinnedArgs {
     const uint4 *corefx;       // fixed-point x, y, z and compact type, by cell
     const int *cell_start;     // per framework: cg_nc[0]*cg_nc[1]*cg_nc[2] + 1 offsets
     const int *nbr_start;      // same layout: each cell's range of nbr_atoms
-    const uint4 *nbr_atoms;    // per cell, the atoms of the cells within one cell (as corefx)
+    const uint4 *nbr_atoms;    // per cell, the atoms near it (as corefx), nearest to its centre first
+    int full_stencil;          // some system has hc_on == 2: bin_reject_kernel runs
     const float *rho2;         // nsys x NS x ntypes_c rejection radii^2 (Å^2), rounded down
     int *cand;                 // chunk-relative insertions left for the full phase-0 stencil
     int *ncand;                // their count
@@ -323,14 +329,6 @@ __device__ inline double cw_pair(double r2, double sg2, double ep4, double qq_ke
         e = __builtin_fma(qq_ke * (t * exp64_small(__builtin_fma(-z, z, p), C)), ir, e);
     }
     return e;
-}
-
-// Phase-0 near stencil: the i-th (i < k = min(3, nc)) neighbour along one axis of cell index h,
-// among nc cells (each cell once when the axis has fewer than 3 cells).
-__host__ __device__ inline int nbr_cell_axis(int h, int i, int k, int nc)
-{
-    const int f = k == nc ? 0 : (h - 1 + nc) % nc;
-    return (f + i) % nc;
 }
 
 // One site pair of the move path (FP64): Lennard-Jones inside rc_lj plus the screened Coulomb

@@ -38,8 +38,9 @@ hipError_t grad_select(const double *dU, const int64_t *seg, int nsys, const dou
                        unsigned char *flag, int64_t *list, int64_t *count, void *tmp, size_t *tmp_bytes, hipStream_t st);
 hipError_t launch_grad_recip(const GradArgs &a, const double4 *k64, const int4 *rblk, int nrblk, hipStream_t st);
 hipError_t launch_sk(const double4 *atoms, int natoms, const int4 *kreq, int nreq, double2 *out, hipStream_t st);
-hipError_t launch_nbr_fill(const FwDesc *fw, int nfw, const int *cell_fw_off, int ncells, const int *cell_start,
-                           const int *nbr_start, const uint4 *corefx, uint4 *nbr_atoms, hipStream_t st);
+hipError_t launch_nbr(bool fill, const FwDesc *fw, int nfw, const int *cell_fw_off, int ncells, const int *cell_start,
+                      int *nbr_start, const uint4 *corefx, uint4 *nbr_atoms, hipStream_t st);
+hipError_t scan_counts(int *counts, int n, void *tmp, size_t *tmp_bytes, hipStream_t st);
 hipError_t launch_self_term(const int4 *kn, const double *kpref, int nk, const double *gsf, const double *q, int ns,
                             double *partial, hipStream_t st);
 }  // namespace pa
@@ -346,9 +347,11 @@ double lj_pair(double r2, double sg, double ep)
     return 4.0 * ep * (x * x - x);
 }
 
-// Edge (Å) of the hard-core grid cells of phase 0. Typical rejection radii are 1-2.3 Å, so the
-// near stencil (the home cell and its neighbours) usually decides an insertion.
+// Edge (Å) of the hard-core grid cells of phase 0, and the temperature (K) whose rejection radii the
+// cells' near lists hold: the radii fall slowly with temperature (as T^-1/12), so lists for 77 K
+// serve every temperature above it and are a tenth longer than room temperature needs.
 constexpr double HC_CELL = 1.2;
+constexpr double HC_LIST_T = 77.0;
 
 // pair_energy (src/reject.jl:22): LJ plus K erfc(alpha r)/r with the pair series.
 double pair_energy_h(double r, double sg, double ep, double K, double alpha)
@@ -467,16 +470,14 @@ struct BatchTables {
     std::vector<int> coreidx, cell_start;
     std::vector<uint4> binfx;           // the atoms in Morton order (mixed path's list build)
     std::vector<int> bintype;
-    std::vector<int> nbr_start;         // per framework cell (cell_start layout): first entry in nbr_atoms
-    int64_t nbr_total = 0;              // entries of nbr_atoms (filled on the device from corefx)
     std::vector<int> cell_fw_off{0};    // prefix over frameworks of their cell counts
     std::vector<double2> pair64;
     std::vector<float2> pair32;
 };
 
 // Appends framework D's n atoms (fractional coordinates, Cartesian positions or NULL to take
-// A f, charges, compact LJ types) to the atom tables, with its hard-core cell grid and the
-// offsets of its near-stencil lists. L: the cell's perpendicular widths. Sets D.atom_off,
+// A f, charges, compact LJ types) to the atom tables, with its hard-core cell grid. L: the cell's
+// perpendicular widths. Sets D.atom_off,
 // D.natoms, D.cg_off and D.cg_nc.
 int add_atoms(BatchTables &T, FwDesc &D, const double *frac, const double *cart, const double *q, const int *ctype,
               int n, const double L[3])
@@ -549,43 +550,53 @@ int add_atoms(BatchTables &T, FwDesc &D, const double *frac, const double *cart,
         }
         T.corefx.insert(T.corefx.end(), sorted.begin(), sorted.end());
         T.coreidx.insert(T.coreidx.end(), sidx.begin(), sidx.end());
-        // near-stencil atom lists: for every cell, the atoms of the cells within one cell of
-        // it (each cell once when an axis has fewer than 3 cells), contiguous, so phase 0's
-        // near test reads one range per site
-        const int nc0 = D.cg_nc[0], nc1 = D.cg_nc[1], nc2 = D.cg_nc[2];
-        const int k0 = std::min(3, nc0), k1 = std::min(3, nc1), k2 = std::min(3, nc2);
-        // offsets only: nbr_fill_kernel copies the lists on the device (nbr_cells order)
-        auto axis_nbrs = [](int nc, int k) {
-            std::vector<int> t((size_t)nc * k);
-            for (int h = 0; h < nc; ++h)
-                for (int i = 0; i < k; ++i) t[(size_t)h * k + i] = nbr_cell_axis(h, i, k, nc);
-            return t;
-        };
-        const std::vector<int> nb0 = axis_nbrs(nc0, k0), nb1 = axis_nbrs(nc1, k1), nb2 = axis_nbrs(nc2, k2);
-        for (int h2 = 0; h2 < nc2; ++h2)
-            for (int h1 = 0; h1 < nc1; ++h1)
-                for (int h0 = 0; h0 < nc0; ++h0) {
-                    if (T.nbr_total > (int64_t)INT32_MAX)
-                        return fail(PA_ERR_ARG, "the frameworks' phase-0 neighbour lists exceed 2^31 entries");
-                    T.nbr_start.push_back((int)T.nbr_total);
-                    for (int i2 = 0; i2 < k2; ++i2)
-                        for (int i1 = 0; i1 < k1; ++i1) {
-                            const int row = nc0 * (nb1[(size_t)h1 * k1 + i1] + nc1 * nb2[(size_t)h2 * k2 + i2]);
-                            for (int i0 = 0; i0 < k0; ++i0) {
-                                const int cc = nb0[(size_t)h0 * k0 + i0] + row;
-                                T.nbr_total += cnt[cc + 1] - cnt[cc];
-                            }
-                        }
-                }
-        if (T.nbr_total > (int64_t)INT32_MAX)
-            return fail(PA_ERR_ARG, "the frameworks' phase-0 neighbour lists exceed 2^31 entries");
-        T.nbr_start.push_back((int)T.nbr_total);
         T.cell_fw_off.push_back(T.cell_fw_off.back() + nct);
     }
     return PA_OK;
 }
 
-// Creates the batch's stream and events, uploads every table and fills the near-stencil lists
+// Radius, distance threshold and cell reach of every framework's phase-0 near lists: the largest
+// rejection radius at HC_LIST_T, scaled down until the lists stay below 2^31 entries (each atom is
+// in at most prod(2 reach + 1) of them).
+int near_list_radii(pa_batch *b)
+{
+    std::vector<double> r(b->nfw, -1.0), rho2((size_t)b->nsites * b->ntypes_c);
+    for (int s = 0; s < b->nsys; ++s) {
+        const int u = b->fw_of[s];
+        if (r[u] >= 0.0) continue;
+        double rmax2 = 0.0;
+        if (rejection_radii(b, s, KB * HC_LIST_T, (double)FLT_EPSILON, rho2.data(), &rmax2)) rmax2 = 0.0;
+        r[u] = std::sqrt(rmax2) * (1.0 + 1e-6);
+    }
+    for (double scale = 1.0;; scale *= 0.7) {
+        double entries = 0.0;
+        for (int u = 0; u < b->nfw; ++u) {
+            FwDesc &D = b->desc[u];
+            const FwHost &h = b->info[u];
+            const double R = r[u] * scale;
+            double rc = 0.0, per_atom = 1.0;  // circumradius of a cell: half its longest body diagonal
+            for (int sy = -1; sy <= 1; sy += 2)
+                for (int sz = -1; sz <= 1; sz += 2) {
+                    const double f[3] = {0.5 / D.cg_nc[0], 0.5 * sy / D.cg_nc[1], 0.5 * sz / D.cg_nc[2]};
+                    double v[3];
+                    matvec(D.A, f, v);
+                    rc = std::max(rc, norm3(v));
+                }
+            const double thr = (R + rc) * (1.0 + 1.0e-5) + 1.0e-3;  // FP32 distances on the device
+            D.nbr_r = std::nextafter((float)R, 0.0f);
+            D.nbr_thr2 = (float)(thr * thr);
+            for (int d = 0; d < 3; ++d) {
+                D.nbr_reach[d] = std::max(1, (int)std::ceil(thr * D.cg_nc[d] / h.perp[d] + 0.5));
+                per_atom *= std::min(D.cg_nc[d], 2 * D.nbr_reach[d] + 1);
+            }
+            entries += per_atom * D.natoms;
+        }
+        if (entries < (double)INT32_MAX) return PA_OK;
+        if (scale < 0.05) return fail(PA_ERR_ARG, "the frameworks' phase-0 neighbour lists exceed 2^31 entries");
+    }
+}
+
+// Creates the batch's stream and events, uploads every table and builds the phase-0 near lists
 // on the device.
 int upload_batch(pa_batch *b, const BatchTables &T)
 {
@@ -596,6 +607,7 @@ int upload_batch(pa_batch *b, const BatchTables &T)
     // timing-only events: no system-scope fence (no cache write-back and invalidation around the
     // kernels they bracket); results reach the host through copies and stream synchronisation
     for (auto &e : b->ev) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableSystemFence));
+    if (int e = near_list_radii(b)) return e;
     HIP_TRY(upload(b->d_fw, b->desc));
     HIP_TRY(upload(b->d_fw_of, b->fw_of));
     HIP_TRY(upload(b->d_atom64, T.atom64));
@@ -612,15 +624,26 @@ int upload_batch(pa_batch *b, const BatchTables &T)
     HIP_TRY(upload(b->d_bintype, T.bintype));
     HIP_TRY(upload(b->d_coreidx, T.coreidx));
     HIP_TRY(upload(b->d_cell_start, T.cell_start));
-    HIP_TRY(upload(b->d_nbr_start, T.nbr_start));
-    HIP_TRY(b->d_nbr_atoms.ensure(sizeof(uint4) * (size_t)std::max<int64_t>(1, T.nbr_total)));
     {
-        DevAlloc d_cfo;
+        DevAlloc d_cfo, tmp;
         HIP_TRY(upload(d_cfo, T.cell_fw_off));
-        HIP_TRY(launch_nbr_fill(b->d_fw.as<FwDesc>(), b->nfw, d_cfo.as<int>(), T.cell_fw_off.back(),
-                                b->d_cell_start.as<int>(), b->d_nbr_start.as<int>(), b->d_corefx.as<uint4>(),
-                                b->d_nbr_atoms.as<uint4>(), nullptr));
-        HIP_TRY(hipDeviceSynchronize());
+        const int n = (int)T.cell_start.size(), ncells = T.cell_fw_off.back();
+        HIP_TRY(b->d_nbr_start.ensure(sizeof(int) * std::max(n, 1)));
+        int *start = b->d_nbr_start.as<int>(), total = 0;
+        auto nbr = [&](bool fill, uint4 *out) {
+            return launch_nbr(fill, b->d_fw.as<FwDesc>(), b->nfw, d_cfo.as<int>(), ncells, b->d_cell_start.as<int>(), start,
+                              b->d_corefx.as<uint4>(), out, b->stream);
+        };
+        HIP_TRY(nbr(false, nullptr));
+        size_t bytes = 0;
+        HIP_TRY(scan_counts(start, n, nullptr, &bytes, b->stream));
+        HIP_TRY(tmp.ensure(bytes));
+        HIP_TRY(scan_counts(start, n, tmp.p, &bytes, b->stream));
+        HIP_TRY(hipMemcpyAsync(&total, start + (n - 1), sizeof(int), hipMemcpyDeviceToHost, b->stream));
+        HIP_TRY(hipStreamSynchronize(b->stream));
+        HIP_TRY(b->d_nbr_atoms.ensure(sizeof(uint4) * (size_t)std::max(1, total)));
+        HIP_TRY(nbr(true, b->d_nbr_atoms.as<uint4>()));
+        HIP_TRY(hipStreamSynchronize(b->stream));
     }
     return PA_OK;
 }
@@ -1457,7 +1480,7 @@ static int run_energies(pa_batch *b, const std::vector<int64_t> &seg, int64_t gb
         const double d0 = std::max(0.0, rcmax - rb - b->r_guest - 0.05);
         B.cls_d0 = (float)d0;
         B.cls_inv_w = (float)((binned_nclasses() - 1) / std::max(R - d0, 1e-3));
-        B.reach[0] = B.reach[1] = B.reach[2] = -1;
+        B.hc_on = 0;
         B.hc_rf[0] = B.hc_rf[1] = B.hc_rf[2] = 0u;
         for (int d = 0; d < 3; ++d) B.alt[d] = (float)std::max(0.0, 1.0 - R / h.perp[d]);
         B.bin_base = base[s];
@@ -1467,6 +1490,7 @@ static int run_energies(pa_batch *b, const std::vector<int64_t> &seg, int64_t gb
     // phase-0 rejection radii for this kT (src/widom.jl:202-253): margin = (theta + 2) kT + safety
     // + B_s - c_s with the FP32 rounding allowance of the mixed path's pair terms
     std::vector<float> rho2((size_t)nsys * b->nsites * b->ntypes_c, 0.0f);
+    bool full_stencil = false;
     if (kT > 0.0) {
         const int NS = b->nsites, NTC = b->ntypes_c;
         if (b->rr_kT != kT) {
@@ -1494,9 +1518,10 @@ static int run_energies(pa_batch *b, const std::vector<int64_t> &seg, int64_t gb
             }
             const FwHost &h = b->info[b->fw_of[s]];
             const FwDesc &D = b->desc[b->fw_of[s]];
-            if (rmax2 > 0.0)
+            if (rmax2 > 0.0) {
+                bins[s].hc_on = std::sqrt(rmax2) <= (double)D.nbr_r ? 1 : 2;
+                full_stencil = full_stencil || bins[s].hc_on == 2;
                 for (int d = 0; d < 3; ++d) {
-                    bins[s].reach[d] = (int)std::ceil(std::sqrt(rmax2) * D.cg_nc[d] / h.perp[d]);
                     bins[s].hc_rf[d] = (uint32_t)std::min(4294967295.0,
                                                           std::ceil(std::sqrt(rmax2) / h.perp[d] * 4294967296.0) + 2.0);
                     // +-hc_rf plus one cell reaching around the axis: every cell, marked by the
@@ -1504,6 +1529,7 @@ static int run_energies(pa_batch *b, const std::vector<int64_t> &seg, int64_t gb
                     const uint64_t rf = bins[s].hc_rf[d], nc = (uint64_t)D.cg_nc[d];
                     if (2 * rf + ((uint64_t)1 << 32) / nc >= ((uint64_t)1 << 32)) bins[s].hc_rf[d] = 0xFFFFFFFFu;
                 }
+            }
         }
     }
     const int nbins = base[nsys];
@@ -1587,6 +1613,7 @@ static int run_energies(pa_batch *b, const std::vector<int64_t> &seg, int64_t gb
     A.nbr_start = b->d_nbr_start.as<int>();
     A.nbr_atoms = b->d_nbr_atoms.as<uint4>();
     A.rho2 = d_rho2;
+    A.full_stencil = full_stencil;
     for (int64_t g0 = gb; g0 < ge; g0 += CH) {
         A.g0 = g0;
         A.g1 = std::min(ge, g0 + CH);

@@ -144,10 +144,14 @@ __device__ inline bool stencil_hit(const BinnedArgs &a, const FwDesc &F, int s, 
     return hit;
 }
 
-// Pose, bin and the near part of phase 0 of every insertion of the chunk. The near stencil
-// (the home cell and its neighbours) rejects most insertions that phase 0 rejects; an insertion
-// whose full stencil reaches further and that the near stencil did not reject is appended to
-// the candidate list for bin_reject_kernel, which finishes phase 0 on full wavefronts.
+// Pose, bin and phase 0 of every insertion of the chunk. Each site's hard-core cell lists the
+// atoms within the rejection radii of any point of it, nearest first: one contiguous range per
+// site decides. With the atoms of the 27 cells around it instead, half of the insertions into a
+// porous framework went to a second kernel's wider stencil, by a list whose one atomic counter
+// cost 8 ns a wavefront: 1e6 insertions of CO2 into the 2,160-atom hexagonal cell took 199 us here
+// and 148 us there, 63-101 us now (RUBTAK 3x3x3, whose radii fitted the 27 cells, 72 -> 91 us).
+// Only below the temperature that the lists were built for does an insertion that passes go on
+// to bin_reject_kernel.
 template <int NS>
 __global__ __launch_bounds__(256) void bin_pose_kernel(BinnedArgs a)
 {
@@ -177,9 +181,7 @@ __global__ __launch_bounds__(256) void bin_pose_kernel(BinnedArgs a)
     const int bz = min(B.nb[2] - 1, (int)(f[2] * B.nb[2]));
     const int key = B.bin_base + bx + B.nb[0] * (by + B.nb[1] * bz);
     bool pending = false;
-    if (B.reach[0] >= 0) {
-        // the near stencil (home cell and its neighbours; reach >= 1 whenever phase 0 runs) from
-        // the home cell's precomputed atom list: one contiguous range per site
+    if (B.hc_on) {
         const int *nbs = a.nbr_start + F.cg_off;
         const float *rho = a.rho2 + (size_t)s * NS * a.ntypes_c;
         int j0[NS], j1[NS];
@@ -213,22 +215,7 @@ __global__ __launch_bounds__(256) void bin_pose_kernel(BinnedArgs a)
             a.dU[g - a.out_base] = INFINITY;
             return;
         }
-        // the full test is pending when some site's cells within the largest radius reach
-        // beyond the home cell's neighbours
-        if (B.reach[0] > 1 || B.reach[1] > 1 || B.reach[2] > 1) {
-#pragma unroll
-            for (int t = 0; t < NS; ++t)
-                for (int d = 0; d < 3; ++d) {
-                    const int nc = F.cg_nc[d];
-                    if (nc <= 3) continue;
-                    const int home = (int)(((uint64_t)sp[t][d] * (uint64_t)nc) >> 32);
-                    int st, cnt;
-                    cell_range(sp[t][d], B.hc_rf[d], nc, st, cnt);
-                    // cells [st, st + cnt) against [home - 1, home + 1], both wrapping
-                    const int below = home - st < 0 ? home - st + nc : home - st;
-                    if (below > 1 || cnt - below > 2) pending = true;
-                }
-        }
+        pending = B.hc_on == 2;
     }
     a.key[g - a.g0] = key;
     if (!pending) {
@@ -844,8 +831,10 @@ static hipError_t launch_binned_ns(const BinnedArgs &a, bool upper, hipStream_t 
     const int64_t n = a.g1 - a.g0;
     const dim3 g256((unsigned)((n + 255) / 256)), b256(256);
     hipLaunchKernelGGL((bin_pose_kernel<NS>), g256, b256, 0, st, a);
-    const dim3 gr((unsigned)std::min<int64_t>((n + 255) / 256, 2048));
-    hipLaunchKernelGGL((bin_reject_kernel<NS>), gr, b256, 0, st, a);
+    if (a.full_stencil) {
+        const dim3 gr((unsigned)std::min<int64_t>((n + 255) / 256, 2048));
+        hipLaunchKernelGGL((bin_reject_kernel<NS>), gr, b256, 0, st, a);
+    }
     return hipGetLastError();
 }
 
