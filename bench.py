@@ -179,7 +179,7 @@ def main():
                          "rubtak: the reference's own benchmark system (RUBTAK 3x3x3 + CO2, TraPPE, 12 A); "
                          "nvt: NVT move cost and Widom insertion along the chain (RUBTAK 3x3x3 + 50 CO2)")
     ap.add_argument("--bin-scale", type=float, default=0.0,
-                    help="mixed-path bin edge multiplier (0: the library tunes it on the first call)")
+                    help="mixed-path bin edge multiplier (0: the library's rule on the sizes)")
     ap.add_argument("--gcmc-warmup", type=int, default=20000)
     ap.add_argument("--gcmc-production", type=int, default=50000)
     ap.add_argument("--nvt-moves", type=int, default=20000, help="nvt: translation attempts per chain count, in total")

@@ -187,7 +187,7 @@ int pa_widom(pa_batch *batch, const pa_guest *guest, double T, int64_t ninsert, 
 /* pa_widom that allocates no device memory. No counterpart in the reference: it is for callers
  * that cannot allocate (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc). Same arguments, kernels and results as pa_widom with the batch's bin scale as it
- * stands (it never runs the bin-scale tuner; fix the scale with pa_batch_set_bin_scale to
+ * stands (the scale of the last long pa_widom call, 1 before one; fix it with pa_batch_set_bin_scale to
  * compare results bit for bit). Every per-call device buffer (energies, bins, pose coordinates,
  * tile sums, scan storage) is carved from one static device array of PA_NOALLOC_SCRATCH_BYTES per
  * device (64 MiB, held until the process ends): 1e6 insertions of a 3-site guest fit with the
@@ -387,10 +387,10 @@ typedef struct pa_nvt_timing {
 int pa_nvt_last_timing(const pa_state *state, pa_nvt_timing *out);
 
 /* Mixed-path bin edge multiplier of `batch` (no counterpart in the reference): every system's
- * spatial bin edge is kappa * max(2 Å, (64 V / insertions)^(1/3)). 0 (the initial value) lets the
- * first large enough pa_widom call time a few values of kappa and keep the fastest; a fixed
- * kappa makes results reproducible across processes (the bin only changes FP32 rounding of the
- * coordinates relative to its centre, ~1e-7 relative in dU). */
+ * spatial bin edge is kappa * max(2 Å, (64 V / insertions)^(1/3)). 0 (the initial value) takes
+ * it from a rule on the batch's sizes and the call's insertions. pa_batch_bin_scale gives a pinned
+ * kappa, or else that of the last pa_widom call of at least 2^18 insertions (0 before one). The bin
+ * only changes FP32 rounding of the coordinates relative to its centre, ~1e-7 relative in dU. */
 int pa_batch_set_bin_scale(pa_batch *batch, double kappa);
 int pa_batch_bin_scale(const pa_batch *batch, double *kappa);
 

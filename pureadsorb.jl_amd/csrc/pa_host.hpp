@@ -209,7 +209,9 @@ struct pa_batch {
     std::vector<double> hc_bs, hc_kmin;
     // host copies of the FP64 tables (the move path's from-scratch energies and audit)
     bool fullk = false;
-    double bin_scale = 0.0;  // mixed path: bin edge multiplier (0: not yet tuned, 1 used meanwhile)
+    double bin_scale = 0.0;       // mixed path: pinned bin edge multiplier (0: chosen by a rule)
+    double bin_scale_used = 0.0;  // the last mixed-path call's
+    double bin_scale_seen = 0.0;  // that of the last long Widom call (0: none yet)
     pa::CallScratch scr;     // where the current call's per-call buffers come from
     int device = 0;          // HIP device the batch's tables live on
     int list_cap = 0;        // mixed path: fixed neighbour-list capacity (0: sized per call)

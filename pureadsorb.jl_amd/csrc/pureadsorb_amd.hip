@@ -1351,10 +1351,49 @@ static int scratch_fail(const pa_batch *b, hipError_t e, const char *what, int l
         if (e_ != hipSuccess) return scratch_fail(b, e_, #expr, __LINE__);                              \
     } while (0)
 
-// Smallest bin edge (Å) of the mixed path, and the insertions a bin aims to hold when a system
-// has few insertions for its volume.
+// Smallest bin edge (Å) of the mixed path, and, under a pinned bin scale, the insertions a bin aims
+// to hold when a system has few insertions for its volume.
 constexpr double BIN_EDGE_MIN = 2.0;
 constexpr double BIN_TARGET_INSERTIONS = 64.0;
+
+// Bin edge multiplier of a call whose bin scale is not pinned; system s has n[s] of its N insertions
+// (0: not part of it). Short calls take 1: their time is not in the bins. In a long one a bin costs
+// its list build, B + natoms (barriers, the atoms scanned), and a surviving insertion sweeps list
+// rows in proportion to its NS sites, the density and the edge (rows that some site's cutoff cuts).
+// The sum is least at
+//     e^4 = 3 V (B + natoms) / (density n_survivors NS C),
+// with survivors n exp(-15 A^3 density) and B = 4700, C = 450 instruction slots, and 2,048 bins fill
+// and balance the chip. The nearest step to the systems' mean is taken, so that pinning what
+// pa_batch_bin_scale reports repeats a call bit for bit.
+// Widom calls, rule / best of 1, 1.25, 1.5 (us): RUBTAK 1e6 1286 / 1295, 3e5 536 / 541; hexagonal
+// 80-atom cell 1e6 884 / 884, 40-atom cell 1e6 885 / 866; 32 frameworks x 1e5 3254 / 3265. It replaced
+// timing seven multipliers twice on a batch's first long call: that call's 26.0 (RUBTAK 1e6) and
+// 71 ms (32 frameworks) are 1.9 and 4.6 ms now, at the same multipliers up to one step.
+static const double BIN_SCALE_STEPS[] = {0.75, 1.0, 1.25, 1.5, 1.75, 2.0, 2.5};
+constexpr int64_t BIN_SCALE_LONG = (int64_t)1 << 18;
+static inline double bin_edge_unit(double V, double n)
+{
+    return std::max(BIN_EDGE_MIN, std::cbrt(BIN_TARGET_INSERTIONS * V / n));
+}
+static double bin_scale_rule(const pa_batch *b, const std::vector<double> &n)
+{
+    double N = 0.0, Vtot = 0.0, mean = 0.0;
+    for (size_t s = 0; s < n.size(); ++s)
+        if (n[s] > 0.0) N += n[s], Vtot += b->info[b->fw_of[s]].volume;
+    if (N < (double)BIN_SCALE_LONG) return 1.0;
+    for (size_t s = 0; s < n.size(); ++s) {
+        if (!(n[s] > 0.0)) continue;
+        const FwHost &h = b->info[b->fw_of[s]];
+        const double rho = std::max(h.natoms, 1) / h.volume;
+        const double survivors = std::max(n[s] * std::exp(-15.0 * rho), 1.0);
+        const double e = std::pow(3.0 * h.volume * (4700.0 + h.natoms) / (rho * survivors * b->nsites * 450.0), 0.25);
+        mean += n[s] / N * std::max(BIN_EDGE_MIN, std::min(e, std::cbrt(Vtot / 2048.0))) / bin_edge_unit(h.volume, n[s]);
+    }
+    double best = BIN_SCALE_STEPS[0];
+    for (double k : BIN_SCALE_STEPS)
+        if (std::fabs(k - mean) < std::fabs(best - mean)) best = k;
+    return best;
+}
 
 // Delta U of flattened insertions g in [gb, ge) (system s owns g in [seg[s], seg[s+1])) into
 // b->d_dU[g - out_base], in chunks of at most `chunk` insertions. Records a HIP event pair around
@@ -1433,13 +1472,18 @@ static int run_energies(pa_batch *b, const std::vector<int64_t> &seg, int64_t gb
     std::vector<BinSys> bins(nsys);
     std::vector<int> base(nsys + 1, 0);
     double cap_est = 256.0;
+    std::vector<double> n_of(nsys);
+    for (int s = 0; s < nsys; ++s) n_of[s] = (double)std::max<int64_t>(std::min(ge, seg[s + 1]) - std::max(gb, seg[s]), 0);
+    // a call into a fixed scratch region keeps the last long call's multiplier, if there was one: what
+    // it needs of the region does not depend on the rule
+    const double kappa = b->bin_scale_used = b->bin_scale > 0.0 ? b->bin_scale
+                                             : scr.base         ? (b->bin_scale_seen > 0.0 ? b->bin_scale_seen : 1.0)
+                                                                : bin_scale_rule(b, n_of);
     for (int s = 0; s < nsys; ++s) {
         const FwHost &h = b->info[b->fw_of[s]];
         const FwDesc &D = b->desc[b->fw_of[s]];
-        const int64_t lo = std::max(gb, seg[s]), hi = std::min(ge, seg[s + 1]);
-        const double nins = (double)std::max<int64_t>(hi - lo, 1);
-        const double kappa = b->bin_scale > 0.0 ? b->bin_scale : 1.0;
-        const double edge = kappa * std::max(BIN_EDGE_MIN, std::cbrt(BIN_TARGET_INSERTIONS * h.volume / nins));
+        const double nins = std::max(n_of[s], 1.0);
+        const double edge = kappa * bin_edge_unit(h.volume, nins);
         BinSys &B = bins[s];
         for (int d = 0; d < 3; ++d) B.nb[d] = std::max(1, std::min(1024, (int)std::floor(h.perp[d] / edge)));
         // circumradius of one bin: half its longest body diagonal
@@ -1718,45 +1762,14 @@ static int widom_core(pa_batch *b, const pa_guest *guest, double T, int64_t nins
     }
 
     const double kT_phase0 = (precision & PA_SINGLE_PHASE) ? 0.0 : kT;
-    // a call into a fixed scratch region never tunes: it uses the batch's bin scale as it stands
-    if ((precision & ~PA_SINGLE_PHASE) == PA_PREC_MIXED && b->bin_scale == 0.0 && G >= ((int64_t)1 << 18) &&
-        !scr.base) {
-        // autotune the bin edge multiplier once per batch: time the energy pipeline for each
-        // candidate and keep the fastest. Candidates differ by a few percent, and which one wins
-        // depends on the batch's mix of framework sizes, so the sample is the whole call up to
-        // 2^25 insertions; a longer call is sampled in four windows of 2^22 spread over it
-        // (insertions run system-major: each window holds whole systems at the call's density)
-        const double cand[] = {0.75, 1.0, 1.25, 1.5, 1.75, 2.0, 2.5};
-        const int64_t W = (int64_t)1 << 22;
-        const int nwin = G > ((int64_t)1 << 25) ? 4 : 1;
-        int64_t wb[4], we[4];
-        for (int r = 0; r < nwin; ++r) {
-            wb[r] = nwin == 1 ? 0 : (G - W) * r / (nwin - 1);
-            we[r] = nwin == 1 ? G : wb[r] + W;
-        }
-        double best = 1.0, best_ms = INFINITY;
-        for (int rep = 0; rep < 2; ++rep)
-            for (double kappa : cand) {
-                b->bin_scale = kappa;
-                HIP_TRY(hipEventRecord(b->ev[0], b->stream));
-                for (int r = 0; r < nwin; ++r) {
-                    int64_t nl = 0;
-                    st = run_energies(b, seg, wb[r], we[r], 0, seed, precision, chunk, &nl, kT_phase0, dU);
-                    if (st) { b->bin_scale = 0.0; return st; }
-                }
-                HIP_TRY(hipEventRecord(b->ev[1], b->stream));
-                HIP_TRY(hipEventSynchronize(b->ev[1]));
-                float ms = 0.0f;
-                HIP_TRY(hipEventElapsedTime(&ms, b->ev[0], b->ev[1]));
-                if (rep == 1 && ms < best_ms) { best_ms = ms; best = kappa; }
-            }
-        b->bin_scale = best;
-    }
     HIP_TRY(hipEventRecord(b->ev[0], b->stream));
     int64_t launches = 0;
     // phase 0 (hard-core rejection) unless PA_SINGLE_PHASE
     st = run_energies(b, seg, 0, G, 0, seed, precision, chunk, &launches, kT_phase0, dU);
     if (st) return st;
+    // reported by pa_batch_bin_scale from the first call of this length on
+    if ((precision & ~PA_SINGLE_PHASE) == PA_PREC_MIXED && G >= BIN_SCALE_LONG && !scr.base)
+        b->bin_scale_seen = b->bin_scale_used;
     HIP_TRY(hipEventRecord(b->ev[1], b->stream));
     HIP_TRY(launch_tiles(dU, d_tile_g0, d_tile_n, ntiles, kT, d_tiles, b->stream));
     HIP_TRY(hipEventRecord(b->ev[2], b->stream));
@@ -2283,15 +2296,16 @@ extern "C" int pa_widom_poses(pa_batch *b, int32_t sys, uint64_t seed, int64_t j
 extern "C" int pa_batch_set_bin_scale(pa_batch *b, double kappa)
 {
     if (!b) return fail(PA_ERR_ARG, "NULL batch");
-    if (!(kappa >= 0.0) || kappa > 8.0) return fail(PA_ERR_ARG, "bin scale %g must be in (0, 8], or 0 to re-tune", kappa);
+    if (!(kappa >= 0.0) || kappa > 8.0) return fail(PA_ERR_ARG, "bin scale %g must be in (0, 8], or 0 to unpin", kappa);
     b->bin_scale = kappa;
+    b->bin_scale_seen = 0.0;
     return ok();
 }
 
 extern "C" int pa_batch_bin_scale(const pa_batch *b, double *kappa)
 {
     if (!b || !kappa) return fail(PA_ERR_ARG, "NULL argument");
-    *kappa = b->bin_scale;
+    *kappa = b->bin_scale > 0.0 ? b->bin_scale : b->bin_scale_seen;
     return ok();
 }
 

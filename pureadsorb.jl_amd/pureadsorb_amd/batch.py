@@ -185,7 +185,7 @@ class FrameworkBatch:
 
     @property
     def bin_scale(self) -> float:
-        """Mixed-path bin edge multiplier (0: tuned by the first large widom call)."""
+        """Mixed-path bin edge multiplier (0: from a rule on the sizes; reads as the last long widom call's)."""
         k = ctypes.c_double()
         _lib.check(_lib.lib().pa_batch_bin_scale(self.handle, ctypes.byref(k)))
         return k.value

@@ -75,7 +75,7 @@ def widom(batch: FrameworkBatch, guest: Guest, *, T, ninsert: int, backend: str 
 
     `no_alloc=True` calls pa_widom_noalloc: no device allocation, every per-call buffer from one
     fixed 64 MiB device array shared by all such calls on the device (overlapping calls race),
-    and no bin-scale tuning (the batch's scale as it stands).
+    at the batch's bin scale as it stands.
     """
     if backend not in ("mi355x", "hip"):
         raise _lib.ArgumentError(f"backend={backend!r}: this backend runs on the MI355X ('mi355x')")
