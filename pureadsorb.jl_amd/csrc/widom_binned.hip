@@ -416,9 +416,13 @@ __global__ __launch_bounds__(BIN_WG, 6) void widom_binned_kernel(BinnedArgs a)
     // heaviest bins first, so that the launch does not end on a few crowded bins
     const int b = a.bin_perm ? a.bin_perm[blockIdx.x] : (int)blockIdx.x;
     // this workgroup's share of the bin's insertions (launch_binned_energy_ns)
-    const int nbin = a.bin_start[b + 1] - a.bin_start[b];
-    const int i0 = a.bin_start[b] + (int)((int64_t)nbin * blockIdx.y / gridDim.y);
-    const int nins = a.bin_start[b] + (int)((int64_t)nbin * (blockIdx.y + 1) / gridDim.y) - i0;
+    const int end = a.bin_start[b + 1];
+    int i0 = a.bin_start[b], nins = end - i0;
+    if (gridDim.y > 1) {
+        const int share = (int)(((uint32_t)nins + gridDim.y - 1) / gridDim.y);
+        i0 = min(end, i0 + share * (int)blockIdx.y);
+        nins = min(share, end - i0);
+    }
     if (nins == 0) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int cap = a.listcap;
@@ -652,18 +656,38 @@ __global__ __launch_bounds__(BIN_WG, 6) void widom_binned_kernel(BinnedArgs a)
         // index and claims the next unclaimed one when it finishes (costs differ per insertion)
         for (int ii = wave; ii < nins;) {
             const int grel = a.order[i0 + ii];
-            const uint32_t *sf = a.sitefx + (size_t)grel * 3 * NS;
+            // lane 4 t + d sets up coordinate d of site t (d = 3: nothing), each value once and not in
+            // every lane; the sweep takes them as scalars. The kernel is bound by the issue of vector
+            // instructions, and this takes some 120 of 3,200 off a survivor: RUBTAK 1e6 1.29 ->
+            // 1.25 ms, hexagonal 80-atom cell 0.884 -> 0.863, 32 frameworks x 1e5 3.25 -> 3.22
+            const int ts = min(lane >> 2, NS - 1), ds = min(lane & 3, 2);
+            const uint32_t *sf = a.sitefx + (size_t)grel * 3 * NS + 3 * ts;
+            const uint32_t s0 = sf[0], s1 = sf[1], s2 = sf[2];
+            const double *M = F.A + ds;
+            const double f0 = (double)(int32_t)(s0 - cx) * FIX;
+            const double f1 = (double)(int32_t)(s1 - cy) * FIX;
+            const double f2 = (double)(int32_t)(s2 - cz) * FIX;
+            const float coord = (float)__builtin_fma(M[6], f2, __builtin_fma(M[0], f0, M[3] * f1));
+            // distance from the bin's centre, a sum over the site's four lanes (v_sqrt_f32: 1 ulp,
+            // far inside ROW_MARGIN)
+            float dist = (lane & 3) < 3 ? coord * coord : 0.0f;
+            dist += __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(dist), 0xB1, 0xf, 0xf, true));
+            dist += __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(dist), 0x4E, 0xf, 0xf, true));
+            dist = __builtin_amdgcn_sqrtf(dist);
+            auto scalar = [](float v, int l) {
+                return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), l));
+            };
             uint32_t sfx[NS][3];
-            float sxr[NS], syr[NS], szr[NS], qk[NS];
+            float sxr[NS], syr[NS], szr[NS], delta[NS], qk[NS];
 #pragma unroll
             for (int t = 0; t < NS; ++t) {
-                for (int d = 0; d < 3; ++d) sfx[t][d] = __builtin_amdgcn_readfirstlane(sf[3 * t + d]);
-                const double f0 = (double)(int32_t)(sfx[t][0] - cx) * FIX;
-                const double f1 = (double)(int32_t)(sfx[t][1] - cy) * FIX;
-                const double f2 = (double)(int32_t)(sfx[t][2] - cz) * FIX;
-                sxr[t] = (float)(A0 * f0 + A3 * f1 + A6 * f2);
-                syr[t] = (float)(A1 * f0 + A4 * f1 + A7 * f2);
-                szr[t] = (float)(A2 * f0 + A5 * f1 + A8 * f2);
+                sfx[t][0] = (uint32_t)__builtin_amdgcn_readlane((int)s0, 4 * t);
+                sfx[t][1] = (uint32_t)__builtin_amdgcn_readlane((int)s1, 4 * t);
+                sfx[t][2] = (uint32_t)__builtin_amdgcn_readlane((int)s2, 4 * t);
+                sxr[t] = scalar(coord, 4 * t);
+                syr[t] = scalar(coord, 4 * t + 1);
+                szr[t] = scalar(coord, 4 * t + 2);
+                delta[t] = scalar(dist, 4 * t);
                 qk[t] = a.guest.qke[t];
             }
             double acc = 0.0;
@@ -671,8 +695,7 @@ __global__ __launch_bounds__(BIN_WG, 6) void widom_binned_kernel(BinnedArgs a)
 #pragma unroll
             for (int t = 0; t < NS; ++t) {
                 // rows [0, ra) lie inside the cutoff of this site, rows [rb, nrows) outside it
-                const float delta = __builtin_sqrtf(sxr[t] * sxr[t] + syr[t] * syr[t] + szr[t] * szr[t]);
-                const float thr_in = rc_max - delta - ROW_MARGIN, thr_out = rc_max + delta + ROW_MARGIN;
+                const float thr_in = rc_max - delta[t] - ROW_MARGIN, thr_out = rc_max + delta[t] + ROW_MARGIN;
                 int ra = 0, rskip = 0;
                 for (int r0 = 0; r0 < nrows; r0 += 64) {
                     const int r = r0 + lane;
