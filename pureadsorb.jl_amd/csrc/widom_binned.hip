@@ -356,15 +356,21 @@ constexpr int BUF_RSRC_WORD3 = 0x00020000;
 typedef __attribute__((address_space(3))) const f32x2 lds_f32x2;
 typedef __attribute__((address_space(3))) unsigned char lds_byte;
 
+// Squared distance, plus the 1e-30 that keeps 1/r finite at a coincident site (below every other
+// r2's last bit): it rides in a multiply-add, where a floor would be an instruction per pair of some 38
+// (with the row limits of all sites from one read: hexagonal 80-atom cell 1e6 863 -> 841 us, 40-atom
+// cell 845 -> 815, 32 frameworks x 1e5 3.22 -> 3.15 ms).
+__device__ inline float pair_r2(float dx, float dy, float dz)
+{
+    return __builtin_fmaf(dz, dz, __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, 1.0e-30f)));
+}
+
 // One compacted (site, atom) pair: r2 (Å^2), qq = KE q_site q_atom (FP32) and the LDS address of
 // the (sigma^2, 4 eps) pair parameters.
 template <bool CHARGED, int CUT>
 __device__ inline float pair_term(float r2, float qq, uint32_t paddr, float rc_lj2, float rc_ew2, float alpha,
                                   float alpha2)
 {
-    // r2 >= +0, and the bit patterns of non-negative floats order like their values: an integer
-    // max is the 1e-30 floor that keeps 1/r finite at a coincident site
-    r2 = __uint_as_float(max(__float_as_uint(r2), 0x0DA24260u));
     float e = 0.0f;
     if (CUT != CUT_LJ || r2 < rc_lj2) {
         const f32x2 p = *(lds_f32x2 *)(uintptr_t)paddr;
@@ -690,28 +696,30 @@ __global__ __launch_bounds__(BIN_WG, 6) void widom_binned_kernel(BinnedArgs a)
                 delta[t] = scalar(dist, 4 * t);
                 qk[t] = a.guest.qke[t];
             }
+            // rows [0, rin) lie inside the cutoff of a site, the last rout ones outside it
+            int rin[NS] = {}, rout[NS] = {};
+            for (int r0 = 0; r0 < nrows; r0 += 64) {
+                const int r = r0 + lane;
+                const float2 c = r < nrows ? rowc[r] : make_float2(INFINITY, -INFINITY);
+#pragma unroll
+                for (int t = 0; t < NS; ++t) {
+                    rin[t] += __popcll(__builtin_amdgcn_ballot_w64(c.x < rc_max - delta[t] - ROW_MARGIN));
+                    rout[t] += __popcll(__builtin_amdgcn_ballot_w64(c.y > rc_max + delta[t] + ROW_MARGIN));
+                }
+            }
             double acc = 0.0;
             uint32_t head = 0, tail = 0;
 #pragma unroll
             for (int t = 0; t < NS; ++t) {
-                // rows [0, ra) lie inside the cutoff of this site, rows [rb, nrows) outside it
-                const float thr_in = rc_max - delta[t] - ROW_MARGIN, thr_out = rc_max + delta[t] + ROW_MARGIN;
-                int ra = 0, rskip = 0;
-                for (int r0 = 0; r0 < nrows; r0 += 64) {
-                    const int r = r0 + lane;
-                    const float2 c = r < nrows ? rowc[r] : make_float2(INFINITY, INFINITY);
-                    ra += __popcll(__builtin_amdgcn_ballot_w64(c.x < thr_in));
-                    rskip += __popcll(__builtin_amdgcn_ballot_w64(r < nrows && c.y > thr_out));
-                }
-                ra = __builtin_amdgcn_readfirstlane(ra);
-                const int rend = __builtin_amdgcn_readfirstlane(nrows - rskip);
+                const int ra = __builtin_amdgcn_readfirstlane(rin[t]);
+                const int rend = __builtin_amdgcn_readfirstlane(nrows - rout[t]);
                 const uint32_t tofs = pair_addr + 8u * (uint32_t)(t * ntc);
                 for (int r = 0; r < ra; ++r) {
                     // every entry of the row is in range: evaluate without compaction
                     const float4 E = ent[r * 64 + lane];
                     const uint32_t paddr = tofs + 8u * (uint32_t)etype[r * 64 + lane];
                     const float dx = sxr[t] - E.x, dy = syr[t] - E.y, dz = szr[t] - E.z;
-                    const float r2 = dx * dx + dy * dy + dz * dz;
+                    const float r2 = pair_r2(dx, dy, dz);
                     acc += (double)pair_term<CHARGED, CUT>(r2, CHARGED ? qk[t] * E.w : 0.0f, paddr, rc_lj2, rc_ew2, alpha,
                                                            alpha2);
                 }
@@ -719,7 +727,7 @@ __global__ __launch_bounds__(BIN_WG, 6) void widom_binned_kernel(BinnedArgs a)
                     const float4 E = ent[r * 64 + lane];
                     const uint32_t paddr = tofs + 8u * (uint32_t)etype[r * 64 + lane];
                     const float dx = sxr[t] - E.x, dy = syr[t] - E.y, dz = szr[t] - E.z;
-                    const float r2 = dx * dx + dy * dy + dz * dz;
+                    const float r2 = pair_r2(dx, dy, dz);
                     // sentinel entries: r2 overflows to +inf and fails the test
                     const bool in = r2 < rc_max2;
                     const uint64_t mask = __builtin_amdgcn_ballot_w64(in);
