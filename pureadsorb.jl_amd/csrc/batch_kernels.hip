@@ -1,11 +1,11 @@
 // batch_kernels.hip -- FrameworkBatch tables on gfx950: the host structure factor at the
 // k-vectors a framework keeps (src/batch.jl:173-195) and the 64-orientation guest self term
-// over its full k table (src/batch.jl:360-389), both FP64, and the phase-0 near-stencil atom
-// lists. k = 2 pi A^-T n, so e^{i k.r} = e^{2 pi i n.f}
+// over its full k table (src/batch.jl:360-389), both FP64, the phase-0 atom lists and
+// the FP64 paths' near lists. k = 2 pi A^-T n, so e^{i k.r} = e^{2 pi i n.f}
 // with f = A^-1 r; every phase is one own-sincospi of 2 n.f.
 #include <hipcub/hipcub.hpp>
 
-#include "pa_device.hpp"
+#include "pa_host.hpp"
 
 namespace pa {
 
@@ -172,6 +172,221 @@ hipError_t launch_self_term(const int4 *kn, const double *kpref, int nk, const d
     hipLaunchKernelGGL(self_term_kernel, dim3((unsigned)((nk + 63) / 64)), dim3(BK_WG), 0, st, kn, kpref, nk, gsf, q, ns,
                        partial);
     return hipGetLastError();
+}
+
+// ------------------------------------------------------------------------------------------
+// Near lists: per-framework lists of the atoms near a point, for the FP64 paths.
+//
+// Every unique framework's cell is cut into bins of about NEAR_EDGE Å; a bin lists the atoms of
+// which some image lies within R = max cutoff + largest site distance + bin circumradius of the
+// bin's centre. The atoms that any site of a guest with its reference point in the bin can have
+// inside the cutoff are then among them, whatever image is the nearest: the image that a site
+// sees differs from the nearest one to the centre by at most one cell along each axis (both
+// offsets are within half a cell, and the site within a small part of one of the centre), and
+// all 27 are tried. On RUBTAK 3x3x3 a list holds 790 of 3,078 atoms, of which a site has 360 inside
+// its cutoff. Smaller bins have shorter lists (R falls with the circumradius) and more of them:
+// 2.5 Å takes 11 MB on RUBTAK, and the edge grows until a batch's lists fit NEAR_MAX_ENTRIES.
+// ------------------------------------------------------------------------------------------
+
+constexpr double NEAR_EDGE = 2.5;
+constexpr double NEAR_MAX_ENTRIES = 268435456.0;  // 1 GiB of 4-byte entries
+
+struct NearBuild {
+    const FwDesc *fw;
+    const NearDesc *nd;
+    const int *bin_fw;         // nfw + 1: first bin of every framework
+    int nfw, nbins;
+    const double4 *atomf;
+    const int *atype;
+    int *start;                // nbins + 1: counts (first pass), then offsets
+    uint32_t *ent;             // entries (second pass)
+};
+
+// One wavefront per bin. FILL: writes the entries at the bin's offset, else counts them.
+template <bool FILL>
+__global__ __launch_bounds__(256) void near_kernel(NearBuild a)
+{
+    const int lane = threadIdx.x & 63, b = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (b >= a.nbins) return;
+    int lo = 0, hi = a.nfw - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (a.bin_fw[mid] <= b) lo = mid; else hi = mid - 1;
+    }
+    const int u = __builtin_amdgcn_readfirstlane(lo);
+    const FwDesc &F = a.fw[u];
+    const NearDesc D = a.nd[u];
+    const int local = b - a.bin_fw[u];
+    const int bx = local % D.nb[0], by = (local / D.nb[0]) % D.nb[1], bz = local / (D.nb[0] * D.nb[1]);
+    const double c0 = (bx + 0.5) / D.nb[0], c1 = (by + 0.5) / D.nb[1], c2 = (bz + 0.5) / D.nb[2];
+    int total = 0;
+    const int at0 = FILL ? a.start[b] : 0;
+    // filled in two sweeps: the atoms close to the bin come first, so that a caller that tests for
+    // overlaps finds them among the first entries
+    for (int cls = 0; cls < (FILL ? 2 : 1); ++cls)
+    for (int j0 = 0; j0 < F.natoms; j0 += 64) {
+        const int j = j0 + lane;
+        bool in = false;
+        double best = INFINITY;
+        if (j < F.natoms) {
+            const double4 h = a.atomf[F.atom_off + j];
+            double f[3] = {h.x - c0, h.y - c1, h.z - c2};
+            for (int d = 0; d < 3; ++d) f[d] -= __builtin_rint(f[d]);
+            for (int s = 0; s < 27; ++s) {
+                const double g0 = f[0] + (s % 3 - 1), g1 = f[1] + ((s / 3) % 3 - 1), g2 = f[2] + (s / 9 - 1);
+                // an offset's component times the perpendicular width bounds its length from below
+                if (fabs(g0) > D.reach[0] || fabs(g1) > D.reach[1] || fabs(g2) > D.reach[2]) continue;
+                const double x = F.A[0] * g0 + F.A[3] * g1 + F.A[6] * g2;
+                const double y = F.A[1] * g0 + F.A[4] * g1 + F.A[7] * g2;
+                const double z = F.A[2] * g0 + F.A[5] * g1 + F.A[8] * g2;
+                best = fmin(best, x * x + y * y + z * z);
+            }
+            in = best <= D.r2 && (!FILL || (best <= D.close2) == (cls == 0));
+        }
+        const uint64_t mask = __builtin_amdgcn_ballot_w64(in);
+        if (FILL && in) {
+            const int below = __popcll(mask & ((1ull << lane) - 1ull));
+            a.ent[at0 + total + below] = (uint32_t)j | ((uint32_t)a.atype[F.atom_off + j] << NEAR_TYPE_SHIFT);
+        }
+        total += __popcll(mask);
+    }
+    if (!FILL && lane == 0) a.start[b] = total;
+}
+
+// Spreads the low 10 bits of v to every third bit (Morton interleave).
+static uint32_t spread3(uint32_t v)
+{
+    v &= 0x3FF;
+    v = (v | (v << 16)) & 0x030000FF;
+    v = (v | (v << 8)) & 0x0300F00F;
+    v = (v | (v << 4)) & 0x030C30C3;
+    v = (v | (v << 2)) & 0x09249249;
+    return v;
+}
+
+// Every framework's atoms (fractional coordinates in [0, 1), charge; compact type) in Morton
+// order of a ~4 Å cell grid, so that 64 consecutive atoms lie close together.
+static int near_atoms(const pa_batch *b, std::vector<double4> &af, std::vector<int> &at)
+{
+    const size_t na = std::max<size_t>(b->atom64_h.size(), 1);
+    af.assign(na, make_double4(0, 0, 0, 0));
+    at.assign(na, 0);
+    for (int u = 0; u < b->nfw; ++u) {
+        const FwDesc &F = b->desc[u];
+        const FwHost &h = b->info[u];
+        const std::vector<double> &fr = b->fgh[u].frac;
+        const int n = F.natoms;
+        if ((int)fr.size() != 3 * n) return fail(PA_ERR_INTERNAL, "framework %d: fractional table missing", u + 1);
+        int nc[3];
+        for (int d = 0; d < 3; ++d) nc[d] = std::max(1, std::min(1024, (int)std::floor(h.perp[d] / 4.0)));
+        std::vector<uint64_t> key(n);
+        std::vector<double> f(3 * (size_t)n);
+        for (int j = 0; j < n; ++j) {
+            uint32_t c[3];
+            for (int d = 0; d < 3; ++d) {
+                const double x = fr[3 * j + d] - std::floor(fr[3 * j + d]);
+                f[3 * j + d] = x;
+                c[d] = (uint32_t)std::min(nc[d] - 1, (int)(x * nc[d]));
+            }
+            const uint64_t m = spread3(c[0]) | (spread3(c[1]) << 1) | (spread3(c[2]) << 2);
+            key[j] = (m << 32) | (uint32_t)j;
+        }
+        std::sort(key.begin(), key.end());
+        for (int i = 0; i < n; ++i) {
+            const int j = (int)(key[i] & 0xFFFFFFFFu);
+            af[F.atom_off + i] = make_double4(f[3 * j], f[3 * j + 1], f[3 * j + 2], b->atom64_h[F.atom_off + j].w);
+            at[F.atom_off + i] = b->atype_h[F.atom_off + j];
+        }
+    }
+    return PA_OK;
+}
+
+// Builds the batch's near lists once (the first chain state or FP64 Widom call needs them).
+int ensure_near_lists(pa_batch *b)
+{
+    if (b->near_ready) return PA_OK;
+    std::vector<double4> af;
+    std::vector<int> at;
+    int st = near_atoms(b, af, at);
+    if (st) return st;
+    const double rcmax = std::max(b->rc_lj, b->gdev.charged ? b->rc_ew : 0.0);
+    std::vector<NearDesc> nd(b->nfw);
+    std::vector<int> bin_fw(b->nfw + 1, 0);
+    for (double edge = NEAR_EDGE;; edge *= 1.26) {
+        double entries = 0.0;
+        int64_t nbins = 0;
+        for (int u = 0; u < b->nfw; ++u) {
+            const FwHost &h = b->info[u];
+            const FwDesc &F = b->desc[u];
+            if (F.natoms >= (1 << NEAR_TYPE_SHIFT))
+                return fail(PA_ERR_ARG, "framework %d: %d atoms exceed 2^%d", u + 1, F.natoms, NEAR_TYPE_SHIFT);
+            NearDesc &D = nd[u];
+            for (int d = 0; d < 3; ++d) D.nb[d] = std::max(1, std::min(512, (int)std::ceil(h.perp[d] / edge)));
+            double rb = 0.0;  // circumradius: half the longest body diagonal
+            for (int sy = -1; sy <= 1; sy += 2)
+                for (int sz = -1; sz <= 1; sz += 2) {
+                    const double f[3] = {0.5 / D.nb[0], 0.5 * sy / D.nb[1], 0.5 * sz / D.nb[2]};
+                    double v[3];
+                    matvec(F.A, f, v);
+                    rb = std::max(rb, std::sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]));
+                }
+            const double R = rcmax + b->r_guest + rb + 1.0e-6;
+            D.r2 = R * R;
+            D.close2 = (rb + b->r_guest + 2.0) * (rb + b->r_guest + 2.0);
+            for (int d = 0; d < 3; ++d) D.reach[d] = R / h.perp[d] * (1.0 + 1.0e-9);
+            D.bin_off = (int)nbins;
+            bin_fw[u] = (int)nbins;
+            const int64_t n = (int64_t)D.nb[0] * D.nb[1] * D.nb[2];
+            nbins += n;
+            entries += (double)n * std::min<double>(F.natoms, F.natoms / h.volume * (4.0 / 3.0) * PI * R * R * R);
+        }
+        bin_fw[b->nfw] = (int)std::min<int64_t>(nbins, INT32_MAX);
+        if ((entries <= NEAR_MAX_ENTRIES && nbins < (1 << 26)) || edge > 1000.0) break;
+    }
+    const int nbins = bin_fw[b->nfw];
+    HIP_TRY(upload(b->d_nearf, af));
+    HIP_TRY(upload(b->d_neart, at));
+    HIP_TRY(upload(b->d_near_desc, nd));
+    DevAlloc d_fw;
+    HIP_TRY(upload(d_fw, bin_fw));
+    HIP_TRY(b->d_near_start.ensure(sizeof(int) * (nbins + 1)));
+    NearBuild a{};
+    a.fw = b->d_fw.as<FwDesc>();
+    a.nd = b->d_near_desc.as<NearDesc>();
+    a.bin_fw = d_fw.as<int>();
+    a.nfw = b->nfw;
+    a.nbins = nbins;
+    a.atomf = b->d_nearf.as<double4>();
+    a.atype = b->d_neart.as<int>();
+    a.start = b->d_near_start.as<int>();
+    const dim3 grid((unsigned)((nbins + 3) / 4)), block(256);
+    hipLaunchKernelGGL(near_kernel<false>, grid, block, 0, b->stream, a);
+    HIP_TRY(hipGetLastError());
+    std::vector<int> cnt(nbins + 1);
+    HIP_TRY(hipMemcpyAsync(cnt.data(), b->d_near_start.p, sizeof(int) * nbins, hipMemcpyDeviceToHost, b->stream));
+    HIP_TRY(hipStreamSynchronize(b->stream));
+    int64_t run = 0;
+    for (int i = 0; i < nbins; ++i) {
+        const int c = cnt[i];
+        cnt[i] = (int)run;
+        run += c;
+        if (run > (int64_t)INT32_MAX) return fail(PA_ERR_ARG, "the frameworks' near lists exceed 2^31 entries");
+    }
+    cnt[nbins] = (int)run;
+    HIP_TRY(hipMemcpyAsync(b->d_near_start.p, cnt.data(), sizeof(int) * (nbins + 1), hipMemcpyHostToDevice, b->stream));
+    HIP_TRY(b->d_near_ent.ensure(sizeof(uint32_t) * (size_t)std::max<int64_t>(run, 1)));
+    a.ent = b->d_near_ent.as<uint32_t>();
+    hipLaunchKernelGGL(near_kernel<true>, grid, block, 0, b->stream, a);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipStreamSynchronize(b->stream));
+    b->near_ready = true;
+    return PA_OK;
+}
+
+NearLists near_lists(const pa_batch *b)
+{
+    return NearLists{b->d_nearf.as<double4>(), b->d_near_desc.as<NearDesc>(), b->d_near_start.as<int>(),
+                     b->d_near_ent.as<uint32_t>()};
 }
 
 }  // namespace pa

@@ -6,7 +6,7 @@
 // lane from the chain's counter-based stream (select_and_propose, src/moves.jl:275-288). Four
 // wavefronts evaluate an attempt, splitting the three sums a move needs across their lanes:
 //   * the new pose's host-guest real-space energy over the framework atoms near it
-//     (host_guest_realspace_energy_range, src/guest.jl:176-200; near_lists.hip), pairs inside the cutoff
+//     (host_guest_realspace_energy_range, src/guest.jl:176-200; batch_kernels.hip), pairs inside the cutoff
 //     compacted through LDS before the LJ + erfc evaluation (fused multiply-adds, FP64),
 //   * the guest-guest real-space change over (other guest, site) pairs against the sites of the
 //     old and the new pose (guest_guest_move_delta / guest_pair_realspace_energy_range,

@@ -8,7 +8,7 @@
 // (the host adds insertion_constant_term, src/nvt.jl:44-66).
 //
 // One wavefront per insertion:
-//   * host-guest: the near list of the insertion's bin (near_lists.hip), pairs inside the cutoff
+//   * host-guest: the near list of the insertion's bin (batch_kernels.hip), pairs inside the cutoff
 //     queued in LDS and evaluated 64 at a time;
 //   * reciprocal: the chain's k-vectors in the order of the move kernel (KRuns), one run of
 //     consecutive n3 per lane, walked from its middle. The pair m +- j of a run whose middle has

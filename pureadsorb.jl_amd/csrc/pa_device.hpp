@@ -474,7 +474,7 @@ __device__ inline double wave_sum63(double v)
     return dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
 }
 
-// Lists of the atoms near a point (near_lists.hip): bins of framework u's cell, and per bin the
+// Lists of the atoms near a point (batch_kernels.hip): bins of framework u's cell, and per bin the
 // atoms that a guest with its reference point in the bin can have inside the cutoff. An entry is
 // the atom's index (Morton order, framework-relative) and above it its compact type.
 constexpr int NEAR_TYPE_SHIFT = 26;
