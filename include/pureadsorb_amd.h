@@ -29,13 +29,16 @@ extern "C" {
 #define PA_ERR_INTERNAL 4
 
 /* Precision of pa_widom / pa_widom_energies. */
-#define PA_PREC_F64 0   /* FP64 plain path: one work-item per insertion, every pair in FP64 */
+#define PA_PREC_F64 0   /* every pair and k-space term in FP64 */
 #define PA_PREC_MIXED 1 /* FP32 pair + k-space arithmetic, FP64 accumulation and tables */
-/* OR-ed into the precision of pa_widom / pa_widom_grad: skip the mixed path's phase-0 hard-core
- * rejection (the reference's widom_singlephase, src/widom.jl:298). Without it the mixed path
+/* OR-ed into the precision of pa_widom / pa_widom_grad: skip the phase-0 hard-core
+ * rejection (the reference's widom_singlephase, src/widom.jl:298). Without it a call
  * first rejects every insertion whose sites come closer than rho_at to an atom of type t, with
  * radii from the rigorous bound of src/reject.jl, so that its Boltzmann weight is exactly 0.0 in
- * FP64; results are identical either way. The FP64 plain path always evaluates every insertion. */
+ * FP64; results are identical either way in mixed precision, and equal to rounding in FP64, where
+ * the flag takes the plain kernel that tests every pair. Where nothing binds, so that rejected
+ * insertions count beside a system's best one, an FP64 call evaluates that system again without
+ * rejection. */
 #define PA_SINGLE_PHASE 0x100u
 
 /* pa_batch_create flags */

@@ -1286,9 +1286,15 @@ static int check_precision(const pa_batch *b, uint32_t precision)
 // Rejection radii^2 of system s at kT (build_rejection_tables, src/widom.jl:222-253): margin =
 // (theta_F + 2) kT + safety + B_s - c_s, safety sized for energies summed at unit roundoff
 // eps_f / 2. rho2: NS x ntypes_c, Å^2 (0: no rejection for that pair of types).
-int pa::rejection_radii(const pa_batch *b, int s, double kT, double eps_f, double *rho2, double *rmax2)
+static double theta_F()
 {
     static const double theta = theta_f64();
+    return theta;
+}
+
+int pa::rejection_radii(const pa_batch *b, int s, double kT, double eps_f, double *rho2, double *rmax2)
+{
+    const double theta = theta_F();
     const int NS = b->nsites, NTC = b->ntypes_c;
     const int u = b->fw_of[s];
     const FwHost &h = b->info[u];
@@ -1395,54 +1401,88 @@ static double bin_scale_rule(const pa_batch *b, const std::vector<double> &n)
     return best;
 }
 
+// The default cuts a range of n insertions into equal chunks of at most 2^24 (a short last chunk would run
+// the energy kernel on a fraction of the device; each launch ends on a tail of unevenly
+// sized bins, so fewer launches are faster: 52 B of scratch per insertion, 0.9 GB at 2^24);
+// an explicit chunk is taken as given.
+static int64_t chunk_size(int64_t n, int64_t chunk)
+{
+    if (chunk > 0) return std::max<int64_t>(chunk, 64);
+    const int64_t CH = (int64_t)1 << 24;
+    if (n <= CH) return CH;
+    const int64_t parts = (n + CH - 1) / CH;
+    return ((n + parts - 1) / parts + 255) / 256 * 256;
+}
+
+// Event pairs around the energy launches; a call into a fixed scratch region creates and records none.
+static hipError_t energy_events(pa_batch *b, int64_t launches)
+{
+    while (!b->scr.base && (int64_t)b->kev.size() < 2 * launches) {
+        hipEvent_t e;
+        const hipError_t st = hipEventCreateWithFlags(&e, hipEventDisableSystemFence);
+        if (st != hipSuccess) return st;
+        b->kev.push_back(e);
+    }
+    return hipSuccess;
+}
+
+// What the FP64 launches of one call share: the system offsets and which kernel they take.
+struct F64Call {
+    const int64_t *d_seg;
+    bool near;                 // over the near lists, else the plain kernel
+    int tab_w;                 // widest per-axis phase table
+};
+
+// FP64 energies of g in [gb, ge). rho2: phase-0 radii (the near kernel's rejections get +inf), or null.
+static int launch_f64(pa_batch *b, const F64Call &c, const double *rho2, int64_t gb, int64_t ge, int64_t out_base,
+                      uint64_t seed, int64_t chunk, int64_t *launches, double *dU)
+{
+    const int64_t CH = chunk_size(ge - gb, chunk);
+    const bool timed = b->scr.base == nullptr;
+    WidomArgs a = base_args(b);
+    a.seg = c.d_seg;
+    a.seed = seed;
+    a.dU = dU;
+    a.out_base = out_base;
+    HIP_TRY(energy_events(b, *launches + (ge - gb + CH - 1) / CH));
+    for (int64_t g0 = gb; g0 < ge; g0 += CH) {
+        a.g0 = g0;
+        a.g1 = std::min(ge, g0 + CH);
+        if (timed) HIP_TRY(hipEventRecord(b->kev[2 * *launches], b->stream));
+        if (c.near) HIP_TRY(launch_near(a, near_lists(b), rho2, b->upper_all, c.tab_w, b->stream));
+        else HIP_TRY(launch_energy(a, (int)PA_PREC_F64, b->upper_all, b->stream));
+        if (timed) HIP_TRY(hipEventRecord(b->kev[2 * *launches + 1], b->stream));
+        ++*launches;
+    }
+    return PA_OK;
+}
+
 // Delta U of flattened insertions g in [gb, ge) (system s owns g in [seg[s], seg[s+1])) into
 // b->d_dU[g - out_base], in chunks of at most `chunk` insertions. Records a HIP event pair around
 // every energy-kernel launch (b->kev) and returns the launch count in *launches.
-// With kT > 0 and the mixed path, insertions that phase 0 rejects get Delta U = +inf.
+// With kT > 0, insertions that phase 0 rejects get Delta U = +inf. `f64`: the FP64 path's choices, for
+// a caller that evaluates part of the range again.
 // With keys_out, the mixed path stops after phase 0 and binning and returns each insertion's
 // bin key (-1: rejected) instead of energies.
 static int run_energies(pa_batch *b, const std::vector<int64_t> &seg, int64_t gb, int64_t ge, int64_t out_base,
                         uint64_t seed, uint32_t precision, int64_t chunk, int64_t *launches, double kT, double *dU,
-                        std::vector<int> *keys_out = nullptr)
+                        std::vector<int> *keys_out = nullptr, F64Call *f64 = nullptr)
 {
     const int nsys = b->nsys;
     pa::CallScratch &scr = b->scr;
     int64_t *d_seg = nullptr;
     SCR_TRY(b, scr.put(b->d_seg, seg, &d_seg));
-    // the default cuts the range into equal chunks of at most 2^24 (a short last chunk would run
-    // the energy kernel on a fraction of the device; each launch ends on a tail of unevenly
-    // sized bins, so fewer launches are faster: 52 B of scratch per insertion, 0.9 GB at 2^24);
-    // an explicit chunk is taken as given
-    int64_t CH = chunk > 0 ? std::max<int64_t>(chunk, 64) : ((int64_t)1 << 24);
-    if (chunk <= 0 && ge - gb > CH) {
-        const int64_t n = (ge - gb + CH - 1) / CH;
-        CH = ((ge - gb + n - 1) / n + 255) / 256 * 256;
-    }
-    const int64_t nchunks = (ge - gb + CH - 1) / CH;
-    // event pairs around the energy launches; a call into a fixed scratch region creates none
-    // and records none
-    const bool timed = scr.base == nullptr;
-    while (timed && (int64_t)b->kev.size() < 2 * nchunks) {
-        hipEvent_t e;
-        HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableSystemFence));
-        b->kev.push_back(e);
-    }
     *launches = 0;
     if ((precision & ~PA_SINGLE_PHASE) == PA_PREC_F64) {
-        WidomArgs a = base_args(b);
-        a.seg = d_seg;
-        a.seed = seed;
-        a.dU = dU;
-        a.out_base = out_base;
         // two-phase calls (kT > 0) go over the near lists, which the first of them builds; a call
         // into a fixed scratch region uses them only if they are there. Single energies and
         // PA_SINGLE_PHASE calls take the plain kernel.
-        int tab_w = 0;
-        for (const FwDesc &D : b->desc) tab_w = std::max(tab_w, D.kn_max[0] + D.kn_max[1] + D.kn_max[2] + 3);
-        bool near = kT > 0.0 && (!b->gdev.charged || tab_w <= near_tab_max(b->nsites));
-        if (near && !b->near_ready) near = !scr.base && ensure_near_lists(b) == PA_OK;
+        F64Call c{d_seg, false, 0};
+        for (const FwDesc &D : b->desc) c.tab_w = std::max(c.tab_w, D.kn_max[0] + D.kn_max[1] + D.kn_max[2] + 3);
+        c.near = kT > 0.0 && (!b->gdev.charged || c.tab_w <= near_tab_max(b->nsites));
+        if (c.near && !b->near_ready) c.near = !scr.base && ensure_near_lists(b) == PA_OK;
         double *d_r2 = nullptr;
-        if (near) {
+        if (c.near) {
             const size_t per_sys = (size_t)b->nsites * b->ntypes_c;
             if (b->rr64_kT != kT) {
                 // a system without a valid radius rejects nothing
@@ -1456,17 +1496,12 @@ static int run_energies(pa_batch *b, const std::vector<int64_t> &seg, int64_t gb
             }
             SCR_TRY(b, scr.put(b->d_rho2_64, b->rr64_r2, &d_r2));
         }
-        for (int64_t g0 = gb; g0 < ge; g0 += CH) {
-            a.g0 = g0;
-            a.g1 = std::min(ge, g0 + CH);
-            if (timed) HIP_TRY(hipEventRecord(b->kev[2 * *launches], b->stream));
-            if (near) HIP_TRY(launch_near(a, near_lists(b), d_r2, b->upper_all, tab_w, b->stream));
-            else HIP_TRY(launch_energy(a, (int)precision, b->upper_all, b->stream));
-            if (timed) HIP_TRY(hipEventRecord(b->kev[2 * *launches + 1], b->stream));
-            ++*launches;
-        }
-        return PA_OK;
+        if (f64) *f64 = c;
+        return launch_f64(b, c, d_r2, gb, ge, out_base, seed, chunk, launches, dU);
     }
+    const int64_t CH = chunk_size(ge - gb, chunk);
+    const bool timed = scr.base == nullptr;
+    HIP_TRY(energy_events(b, (ge - gb + CH - 1) / CH));
     // ---- mixed path: bin grid of every system, sized by its insertions in [gb, ge)
     const double rcmax = std::max(b->rc_lj, b->gdev.charged ? b->rc_ew : 0.0);
     std::vector<BinSys> bins(nsys);
@@ -1765,14 +1800,12 @@ static int widom_core(pa_batch *b, const pa_guest *guest, double T, int64_t nins
     HIP_TRY(hipEventRecord(b->ev[0], b->stream));
     int64_t launches = 0;
     // phase 0 (hard-core rejection) unless PA_SINGLE_PHASE
-    st = run_energies(b, seg, 0, G, 0, seed, precision, chunk, &launches, kT_phase0, dU);
+    F64Call f64{};
+    st = run_energies(b, seg, 0, G, 0, seed, precision, chunk, &launches, kT_phase0, dU, nullptr, &f64);
     if (st) return st;
     // reported by pa_batch_bin_scale from the first call of this length on
     if ((precision & ~PA_SINGLE_PHASE) == PA_PREC_MIXED && G >= BIN_SCALE_LONG && !scr.base)
         b->bin_scale_seen = b->bin_scale_used;
-    HIP_TRY(hipEventRecord(b->ev[1], b->stream));
-    HIP_TRY(launch_tiles(dU, d_tile_g0, d_tile_n, ntiles, kT, d_tiles, b->stream));
-    HIP_TRY(hipEventRecord(b->ev[2], b->stream));
     // the tile sums back into page-locked memory (a call into a fixed scratch region allocates
     // nothing, so it reads them into ordinary host memory)
     std::vector<double4> tiles_pageable;
@@ -1784,8 +1817,36 @@ static int widom_core(pa_batch *b, const pa_guest *guest, double T, int64_t nins
         HIP_TRY(b->h_tiles.ensure(sizeof(double4) * std::max(ntiles, 1)));
         tiles = b->h_tiles.as<double4>();
     }
-    HIP_TRY(hipMemcpyAsync(tiles, d_tiles, sizeof(double4) * ntiles, hipMemcpyDeviceToHost, b->stream));
-    HIP_TRY(hipStreamSynchronize(b->stream));
+    auto sum_tiles = [&]() -> int {
+        HIP_TRY(hipEventRecord(b->ev[1], b->stream));
+        HIP_TRY(launch_tiles(dU, d_tile_g0, d_tile_n, ntiles, kT, d_tiles, b->stream));
+        HIP_TRY(hipEventRecord(b->ev[2], b->stream));
+        HIP_TRY(hipMemcpyAsync(tiles, d_tiles, sizeof(double4) * ntiles, hipMemcpyDeviceToHost, b->stream));
+        HIP_TRY(hipStreamSynchronize(b->stream));
+        return PA_OK;
+    };
+    st = sum_tiles();
+    if (st) return st;
+    if (f64.near) {
+        // The sums are relative to a system's best insertion. A rejected one has log w < -(theta + 2): zero
+        // as a Float64, but where nothing binds the best insertion lies as deep, and rejected ones count
+        // beside it or hold it. Above the line below they are less than e^-50 of it each; a system
+        // that stays under it (also one with every insertion rejected) is evaluated without rejection.
+        const double line = 50.0 - (theta_F() + 2.0);
+        std::vector<double> best(nsys, -INFINITY);
+        for (int t = 0; t < ntiles; ++t) best[tile_owner[t] / nblocks] = std::max(best[tile_owner[t] / nblocks], tiles[t].x);
+        bool again = false;
+        for (int64_t s = 0; s < nsys; ++s) {
+            int64_t e = s;
+            while (e < nsys && best[e] < line) ++e;
+            if (e == s) continue;
+            st = launch_f64(b, f64, nullptr, seg[s], seg[e], 0, seed, chunk, &launches, dU);
+            if (st) return st;
+            again = true;
+            s = e;
+        }
+        if (again && (st = sum_tiles())) return st;
+    }
     float e01 = 0, e12 = 0, e02 = 0;
     HIP_TRY(hipEventElapsedTime(&e01, b->ev[0], b->ev[1]));
     HIP_TRY(hipEventElapsedTime(&e12, b->ev[1], b->ev[2]));

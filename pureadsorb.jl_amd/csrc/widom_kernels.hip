@@ -103,7 +103,8 @@ __global__ __launch_bounds__(256) void widom_f64_kernel(WidomArgs a)
 // inside the cutoff under divergence, a fifth of the lanes at a time, with some 250 instructions
 // each; here an insertion reads the 790 of RUBTAK's 3,078 atoms near it and evaluates full
 // wavefronts of pairs (cw_pair, some 65 instructions). With rho2, an insertion that the phase-0
-// radii reject (Boltzmann weight exactly zero) gets Delta U = +inf after the first 64 atoms.
+// radii reject (Boltzmann weight exactly zero) gets Delta U = +inf after the first 64 atoms; a system
+// where nothing binds is evaluated again without them (widom_core).
 // FP64 issue bounds it. 100,000 insertions of CO2 into RUBTAK 3x3x3: 9.01 ms with the plain kernel,
 // 0.77 ms here.
 constexpr int WN_WAVES = 4, WN_BATCH = 32;

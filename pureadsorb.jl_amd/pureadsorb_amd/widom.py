@@ -71,7 +71,8 @@ def widom(batch: FrameworkBatch, guest: Guest, *, T, ninsert: int, backend: str 
     Insertions whose Boltzmann weight a rigorous bound proves to be exactly 0.0 in Float64 are
     rejected first (src/widom.jl:99-151, src/reject.jl); `single_phase=True` evaluates every
     insertion instead (the reference's `widom_singlephase`), in Float64 with the plain kernel that
-    tests every pair. Results are the same (in Float64 to rounding).
+    tests every pair. Results are the same (in Float64 to rounding; a system where nothing binds,
+    whose rejected insertions count beside its best one, is evaluated again without rejection).
 
     `no_alloc=True` calls pa_widom_noalloc: no device allocation, every per-call buffer from one
     fixed 64 MiB device array shared by all such calls on the device (overlapping calls race),
