@@ -66,6 +66,23 @@ __global__ __launch_bounds__(BK_WG) void self_term_kernel(const int4 *kn, const 
     if (w == 0) partial[(int64_t)blockIdx.x * 64 + lane] = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
 }
 
+// Squared length of A (x, y, z). A list kernel's counting and its filling instantiation have to agree
+// on every atom, to the last bit, or an entry is left unwritten or written into the next list: the
+// fused operations are spelt out, so that neither depends on what the compiler contracts.
+template <class R>
+__device__ inline R length2(const R A[9], R x, R y, R z)
+{
+#pragma clang fp contract(off)
+    auto fma = [](R a, R b, R c) -> R {
+        if constexpr (sizeof(R) == 8) return __builtin_fma(a, b, c);
+        else return __builtin_fmaf(a, b, c);
+    };
+    const R ex = fma(A[6], z, fma(A[0], x, A[3] * y));
+    const R ey = fma(A[7], z, fma(A[1], x, A[4] * y));
+    const R ez = fma(A[8], z, fma(A[2], x, A[5] * y));
+    return fma(ez, ez, fma(ex, ex, ey * ey));
+}
+
 // Phase-0 near lists: for every hard-core cell, the atoms within nbr_r of any point of it, by their
 // minimum-image distance to the cell's centre. One wavefront per cell, its lanes over the cells
 // within nbr_reach (each once where the reach goes around the axis). Without FILL the lists are
@@ -119,12 +136,8 @@ __global__ __launch_bounds__(BK_WG) void nbr_kernel(const FwDesc *fw, int nfw, c
                 uint4 at = make_uint4(0u, 0u, 0u, 0u);
                 if (j < len) {
                     at = src[b0 + j];
-                    const float dx = (float)(int32_t)(x[0] - at.x), dy = (float)(int32_t)(x[1] - at.y),
-                                dz = (float)(int32_t)(x[2] - at.z);
-                    const float ex = D.Af[0] * dx + D.Af[3] * dy + D.Af[6] * dz;
-                    const float ey = D.Af[1] * dx + D.Af[4] * dy + D.Af[7] * dz;
-                    const float ez = D.Af[2] * dx + D.Af[5] * dy + D.Af[8] * dz;
-                    const float r2 = ex * ex + ey * ey + ez * ez;
+                    const float r2 = length2(D.Af, (float)(int32_t)(x[0] - at.x), (float)(int32_t)(x[1] - at.y),
+                                             (float)(int32_t)(x[2] - at.z));
                     in = FILL ? r2 > shell[sh] && r2 <= shell[sh + 1] : r2 <= D.nbr_thr2;
                 }
                 const uint64_t m = __builtin_amdgcn_ballot_w64(in);
@@ -236,10 +249,7 @@ __global__ __launch_bounds__(256) void near_kernel(NearBuild a)
                 const double g0 = f[0] + (s % 3 - 1), g1 = f[1] + ((s / 3) % 3 - 1), g2 = f[2] + (s / 9 - 1);
                 // an offset's component times the perpendicular width bounds its length from below
                 if (fabs(g0) > D.reach[0] || fabs(g1) > D.reach[1] || fabs(g2) > D.reach[2]) continue;
-                const double x = F.A[0] * g0 + F.A[3] * g1 + F.A[6] * g2;
-                const double y = F.A[1] * g0 + F.A[4] * g1 + F.A[7] * g2;
-                const double z = F.A[2] * g0 + F.A[5] * g1 + F.A[8] * g2;
-                best = fmin(best, x * x + y * y + z * z);
+                best = fmin(best, length2(F.A, g0, g1, g2));
             }
             in = best <= D.r2 && (!FILL || (best <= D.close2) == (cls == 0));
         }
