@@ -196,7 +196,9 @@ hipError_t launch_self_term(const int4 *kn, const double *kpref, int nk, const d
 // inside the cutoff are then among them, whatever image is the nearest: the image that a site
 // sees differs from the nearest one to the centre by at most one cell along each axis (both
 // offsets are within half a cell, and the site within a small part of one of the centre), and
-// all 27 are tried. On RUBTAK 3x3x3 a list holds 790 of 3,078 atoms, of which a site has 360 inside
+// all 27 are tried. Atoms are tried in runs of 64 neighbours in Morton order, and only the runs whose
+// bounding sphere comes within R of the centre: trying every atom, the lists of a framework of 60,000
+// took 100 ms, 15 ms so. On RUBTAK 3x3x3 a list holds 790 of 3,078 atoms, of which a site has 360 inside
 // its cutoff. Smaller bins have shorter lists (R falls with the circumradius) and more of them:
 // 2.5 Å takes 11 MB on RUBTAK, and the edge grows until a batch's lists fit NEAR_MAX_ENTRIES.
 // ------------------------------------------------------------------------------------------
@@ -211,9 +213,37 @@ struct NearBuild {
     int nfw, nbins;
     const double4 *atomf;
     const int *atype;
+    const double4 *run;        // per run of 64 atoms: centre (fractional), radius (Å)
+    const int *run_off;        // nfw + 1
     int *start;                // nbins + 1: counts (first pass), then offsets
     uint32_t *ent;             // entries (second pass)
 };
+
+// Squared distance (Å^2) of the nearest of 27 images of the fractional offset f, those left out whose
+// component on an axis alone (reach: distance over the perpendicular widths) exceeds what is asked for:
+// with a reach below half a cell that leaves an axis's nearest image alone.
+__device__ inline double image_dist2(const FwDesc &F, double f0, double f1, double f2, double reach0, double reach1,
+                                     double reach2)
+{
+    f0 -= __builtin_rint(f0);
+    f1 -= __builtin_rint(f1);
+    f2 -= __builtin_rint(f2);
+    double best = INFINITY;
+    const int n0 = reach0 < 0.5 ? 0 : 1, n1 = reach1 < 0.5 ? 0 : 1, n2 = reach2 < 0.5 ? 0 : 1;
+    for (int s2 = -n2; s2 <= n2; ++s2) {
+        const double g2 = f2 + s2;
+        if (fabs(g2) > reach2) continue;
+        for (int s1 = -n1; s1 <= n1; ++s1) {
+            const double g1 = f1 + s1;
+            if (fabs(g1) > reach1) continue;
+            for (int s0 = -n0; s0 <= n0; ++s0) {
+                const double g0 = f0 + s0;
+                if (fabs(g0) <= reach0) best = fmin(best, length2(F.A, g0, g1, g2));
+            }
+        }
+    }
+    return best;
+}
 
 // One wavefront per bin. FILL: writes the entries at the bin's offset, else counts them.
 template <bool FILL>
@@ -232,34 +262,41 @@ __global__ __launch_bounds__(256) void near_kernel(NearBuild a)
     const int local = b - a.bin_fw[u];
     const int bx = local % D.nb[0], by = (local / D.nb[0]) % D.nb[1], bz = local / (D.nb[0] * D.nb[1]);
     const double c0 = (bx + 0.5) / D.nb[0], c1 = (by + 0.5) / D.nb[1], c2 = (bz + 0.5) / D.nb[2];
+    const double R = __builtin_sqrt(D.r2);
+    const double4 *run = a.run + a.run_off[u];
+    const int nrun = a.run_off[u + 1] - a.run_off[u];
     int total = 0;
     const int at0 = FILL ? a.start[b] : 0;
     // filled in two sweeps: the atoms close to the bin come first, so that a caller that tests for
     // overlaps finds them among the first entries
     for (int cls = 0; cls < (FILL ? 2 : 1); ++cls)
-    for (int j0 = 0; j0 < F.natoms; j0 += 64) {
-        const int j = j0 + lane;
-        bool in = false;
-        double best = INFINITY;
-        if (j < F.natoms) {
-            const double4 h = a.atomf[F.atom_off + j];
-            double f[3] = {h.x - c0, h.y - c1, h.z - c2};
-            for (int d = 0; d < 3; ++d) f[d] -= __builtin_rint(f[d]);
-            for (int s = 0; s < 27; ++s) {
-                const double g0 = f[0] + (s % 3 - 1), g1 = f[1] + ((s / 3) % 3 - 1), g2 = f[2] + (s / 9 - 1);
-                // an offset's component times the perpendicular width bounds its length from below
-                if (fabs(g0) > D.reach[0] || fabs(g1) > D.reach[1] || fabs(g2) > D.reach[2]) continue;
-                best = fmin(best, length2(F.A, g0, g1, g2));
+        for (int q0 = 0; q0 < nrun; q0 += 64) {
+            // 64 runs at once, one per lane: whether an atom of the run can be within R. A run wider than
+            // the 27 images are sure to cover (an offset of up to a whole cell) is taken as it is.
+            bool cand = false;
+            if (q0 + lane < nrun) {
+                const double4 c = run[q0 + lane];
+                const double lim = R + c.w, k = lim / R * (1.0 + 1.0e-9);
+                const double r0 = D.reach[0] * k, r1 = D.reach[1] * k, r2 = D.reach[2] * k;
+                cand = fmax(r0, fmax(r1, r2)) > 1.0 ||
+                       image_dist2(F, c.x - c0, c.y - c1, c.z - c2, r0, r1, r2) <= lim * lim * (1.0 + 1.0e-9);
             }
-            in = best <= D.r2 && (!FILL || (best <= D.close2) == (cls == 0));
+            for (uint64_t todo = __builtin_amdgcn_ballot_w64(cand); todo; todo &= todo - 1) {
+                const int j = (q0 + __builtin_ctzll(todo)) * 64 + lane;
+                bool in = false;
+                if (j < F.natoms) {
+                    const double4 h = a.atomf[F.atom_off + j];
+                    const double best = image_dist2(F, h.x - c0, h.y - c1, h.z - c2, D.reach[0], D.reach[1], D.reach[2]);
+                    in = best <= D.r2 && (!FILL || (best <= D.close2) == (cls == 0));
+                }
+                const uint64_t mask = __builtin_amdgcn_ballot_w64(in);
+                if (FILL && in) {
+                    const int below = __popcll(mask & ((1ull << lane) - 1ull));
+                    a.ent[at0 + total + below] = (uint32_t)j | ((uint32_t)a.atype[F.atom_off + j] << NEAR_TYPE_SHIFT);
+                }
+                total += __popcll(mask);
+            }
         }
-        const uint64_t mask = __builtin_amdgcn_ballot_w64(in);
-        if (FILL && in) {
-            const int below = __popcll(mask & ((1ull << lane) - 1ull));
-            a.ent[at0 + total + below] = (uint32_t)j | ((uint32_t)a.atype[F.atom_off + j] << NEAR_TYPE_SHIFT);
-        }
-        total += __popcll(mask);
-    }
     if (!FILL && lane == 0) a.start[b] = total;
 }
 
@@ -275,12 +312,16 @@ static uint32_t spread3(uint32_t v)
 }
 
 // Every framework's atoms (fractional coordinates in [0, 1), charge; compact type) in Morton
-// order of a ~4 Å cell grid, so that 64 consecutive atoms lie close together.
-static int near_atoms(const pa_batch *b, std::vector<double4> &af, std::vector<int> &at)
+// order of a ~4 Å cell grid, so that 64 consecutive atoms lie close together; and of every run of 64
+// a centre and the radius around it, by each atom's nearest image to the run's first one.
+static int near_atoms(const pa_batch *b, std::vector<double4> &af, std::vector<int> &at, std::vector<double4> &run,
+                      std::vector<int> &run_off)
 {
     const size_t na = std::max<size_t>(b->atom64_h.size(), 1);
     af.assign(na, make_double4(0, 0, 0, 0));
     at.assign(na, 0);
+    run.clear();
+    run_off.assign(1, 0);
     for (int u = 0; u < b->nfw; ++u) {
         const FwDesc &F = b->desc[u];
         const FwHost &h = b->info[u];
@@ -307,7 +348,28 @@ static int near_atoms(const pa_batch *b, std::vector<double4> &af, std::vector<i
             af[F.atom_off + i] = make_double4(f[3 * j], f[3 * j + 1], f[3 * j + 2], b->atom64_h[F.atom_off + j].w);
             at[F.atom_off + i] = b->atype_h[F.atom_off + j];
         }
+        for (int i0 = 0; i0 < n; i0 += 64) {
+            const int m = std::min(64, n - i0);
+            const double4 *p = &af[F.atom_off + i0];
+            double x[64][3], c[3] = {0, 0, 0}, rad2 = 0.0;
+            for (int i = 0; i < m; ++i) {
+                const double d[3] = {p[i].x - p[0].x, p[i].y - p[0].y, p[i].z - p[0].z};
+                for (int e = 0; e < 3; ++e) {
+                    x[i][e] = d[e] - std::rint(d[e]);
+                    c[e] += x[i][e] / m;
+                }
+            }
+            for (int i = 0; i < m; ++i) {
+                const double d[3] = {x[i][0] - c[0], x[i][1] - c[1], x[i][2] - c[2]};
+                double v[3];
+                matvec(F.A, d, v);
+                rad2 = std::max(rad2, v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+            }
+            run.push_back(make_double4(p[0].x + c[0], p[0].y + c[1], p[0].z + c[2], std::sqrt(rad2) + 1.0e-6));
+        }
+        run_off.push_back((int)run.size());
     }
+    if (run.empty()) run.push_back(make_double4(0, 0, 0, 0));
     return PA_OK;
 }
 
@@ -315,9 +377,9 @@ static int near_atoms(const pa_batch *b, std::vector<double4> &af, std::vector<i
 int ensure_near_lists(pa_batch *b)
 {
     if (b->near_ready) return PA_OK;
-    std::vector<double4> af;
-    std::vector<int> at;
-    int st = near_atoms(b, af, at);
+    std::vector<double4> af, run;
+    std::vector<int> at, run_off;
+    int st = near_atoms(b, af, at, run, run_off);
     if (st) return st;
     const double rcmax = std::max(b->rc_lj, b->gdev.charged ? b->rc_ew : 0.0);
     std::vector<NearDesc> nd(b->nfw);
@@ -357,8 +419,10 @@ int ensure_near_lists(pa_batch *b)
     HIP_TRY(upload(b->d_nearf, af));
     HIP_TRY(upload(b->d_neart, at));
     HIP_TRY(upload(b->d_near_desc, nd));
-    DevAlloc d_fw;
+    DevAlloc d_fw, d_run, d_run_off;
     HIP_TRY(upload(d_fw, bin_fw));
+    HIP_TRY(upload(d_run, run));
+    HIP_TRY(upload(d_run_off, run_off));
     HIP_TRY(b->d_near_start.ensure(sizeof(int) * (nbins + 1)));
     NearBuild a{};
     a.fw = b->d_fw.as<FwDesc>();
@@ -368,6 +432,8 @@ int ensure_near_lists(pa_batch *b)
     a.nbins = nbins;
     a.atomf = b->d_nearf.as<double4>();
     a.atype = b->d_neart.as<int>();
+    a.run = d_run.as<double4>();
+    a.run_off = d_run_off.as<int>();
     a.start = b->d_near_start.as<int>();
     const dim3 grid((unsigned)((nbins + 3) / 4)), block(256);
     hipLaunchKernelGGL(near_kernel<false>, grid, block, 0, b->stream, a);
@@ -375,16 +441,16 @@ int ensure_near_lists(pa_batch *b)
     std::vector<int> cnt(nbins + 1);
     HIP_TRY(hipMemcpyAsync(cnt.data(), b->d_near_start.p, sizeof(int) * nbins, hipMemcpyDeviceToHost, b->stream));
     HIP_TRY(hipStreamSynchronize(b->stream));
-    int64_t run = 0;
+    int64_t total = 0;
     for (int i = 0; i < nbins; ++i) {
         const int c = cnt[i];
-        cnt[i] = (int)run;
-        run += c;
-        if (run > (int64_t)INT32_MAX) return fail(PA_ERR_ARG, "the frameworks' near lists exceed 2^31 entries");
+        cnt[i] = (int)total;
+        total += c;
+        if (total > (int64_t)INT32_MAX) return fail(PA_ERR_ARG, "the frameworks' near lists exceed 2^31 entries");
     }
-    cnt[nbins] = (int)run;
+    cnt[nbins] = (int)total;
     HIP_TRY(hipMemcpyAsync(b->d_near_start.p, cnt.data(), sizeof(int) * (nbins + 1), hipMemcpyHostToDevice, b->stream));
-    HIP_TRY(b->d_near_ent.ensure(sizeof(uint32_t) * (size_t)std::max<int64_t>(run, 1)));
+    HIP_TRY(b->d_near_ent.ensure(sizeof(uint32_t) * (size_t)std::max<int64_t>(total, 1)));
     a.ent = b->d_near_ent.as<uint32_t>();
     hipLaunchKernelGGL(near_kernel<true>, grid, block, 0, b->stream, a);
     HIP_TRY(hipGetLastError());
