@@ -198,7 +198,7 @@ hipError_t launch_self_term(const int4 *kn, const double *kpref, int nk, const d
 // offsets are within half a cell, and the site within a small part of one of the centre), and
 // all 27 are tried. Atoms are tried in runs of 64 neighbours in Morton order, and only the runs whose
 // bounding sphere comes within R of the centre: trying every atom, the lists of a framework of 60,000
-// took 100 ms, 15 ms so. On RUBTAK 3x3x3 a list holds 790 of 3,078 atoms, of which a site has 360 inside
+// took 100 ms, some 10 ms so. On RUBTAK 3x3x3 a list holds 790 of 3,078 atoms, of which a site has 360 inside
 // its cutoff. Smaller bins have shorter lists (R falls with the circumradius) and more of them:
 // 2.5 Å takes 11 MB on RUBTAK, and the edge grows until a batch's lists fit NEAR_MAX_ENTRIES.
 // ------------------------------------------------------------------------------------------
@@ -206,18 +206,30 @@ hipError_t launch_self_term(const int4 *kn, const double *kpref, int nk, const d
 constexpr double NEAR_EDGE = 2.5;
 constexpr double NEAR_MAX_ENTRIES = 268435456.0;  // 1 GiB of 4-byte entries
 
-struct NearBuild {
-    const FwDesc *fw;
-    const NearDesc *nd;
-    const int *bin_fw;         // nfw + 1: first bin of every framework
-    int nfw, nbins;
-    const double4 *atomf;
-    const int *atype;
-    const double4 *run;        // per run of 64 atoms: centre (fractional), radius (Å)
-    const int *run_off;        // nfw + 1
-    int *start;                // nbins + 1: counts (first pass), then offsets
-    uint32_t *ent;             // entries (second pass)
-};
+// Centre (fractional) and radius (Å) of every run of 64 atoms, by each atom's nearest image to the run's
+// first one. One wavefront per run.
+__global__ __launch_bounds__(256) void near_run_kernel(NearBuild a)
+{
+    const int lane = threadIdx.x & 63, r = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (r >= a.nruns) return;
+    int lo = 0, hi = a.nfw - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (a.run_off[mid] <= r) lo = mid; else hi = mid - 1;
+    }
+    const FwDesc &F = a.fw[__builtin_amdgcn_readfirstlane(lo)];
+    const int i0 = (r - a.run_off[lo]) * 64, m = min(64, F.natoms - i0);
+    const double4 *p = a.atomf + F.atom_off + i0;
+    const double4 h = p[min(lane, m - 1)], h0 = p[0];
+    double d[3] = {h.x - h0.x, h.y - h0.y, h.z - h0.z}, c[3];
+    for (int e = 0; e < 3; ++e) {
+        d[e] -= __builtin_rint(d[e]);
+        c[e] = __shfl(wave_sum63(lane < m ? d[e] : 0.0), 63, 64) / m;
+    }
+    double rad2 = length2(F.A, d[0] - c[0], d[1] - c[1], d[2] - c[2]);
+    for (int off = 32; off >= 1; off >>= 1) rad2 = fmax(rad2, __shfl_xor(rad2, off, 64));
+    if (lane == 0) a.run[r] = make_double4(h0.x + c[0], h0.y + c[1], h0.z + c[2], __builtin_sqrt(rad2) + 1.0e-6);
+}
 
 // Squared distance (Å^2) of the nearest of 27 images of the fractional offset f, those left out whose
 // component on an axis alone (reach: distance over the perpendicular widths) exceeds what is asked for:
@@ -297,101 +309,46 @@ __global__ __launch_bounds__(256) void near_kernel(NearBuild a)
                 total += __popcll(mask);
             }
         }
-    if (!FILL && lane == 0) a.start[b] = total;
-}
-
-// Spreads the low 10 bits of v to every third bit (Morton interleave).
-static uint32_t spread3(uint32_t v)
-{
-    v &= 0x3FF;
-    v = (v | (v << 16)) & 0x030000FF;
-    v = (v | (v << 8)) & 0x0300F00F;
-    v = (v | (v << 4)) & 0x030C30C3;
-    v = (v | (v << 2)) & 0x09249249;
-    return v;
-}
-
-// Every framework's atoms (fractional coordinates in [0, 1), charge; compact type) in Morton
-// order of a ~4 Å cell grid, so that 64 consecutive atoms lie close together; and of every run of 64
-// a centre and the radius around it, by each atom's nearest image to the run's first one.
-static int near_atoms(const pa_batch *b, std::vector<double4> &af, std::vector<int> &at, std::vector<double4> &run,
-                      std::vector<int> &run_off)
-{
-    const size_t na = std::max<size_t>(b->atom64_h.size(), 1);
-    af.assign(na, make_double4(0, 0, 0, 0));
-    at.assign(na, 0);
-    run.clear();
-    run_off.assign(1, 0);
-    for (int u = 0; u < b->nfw; ++u) {
-        const FwDesc &F = b->desc[u];
-        const FwHost &h = b->info[u];
-        const std::vector<double> &fr = b->fgh[u].frac;
-        const int n = F.natoms;
-        if ((int)fr.size() != 3 * n) return fail(PA_ERR_INTERNAL, "framework %d: fractional table missing", u + 1);
-        int nc[3];
-        for (int d = 0; d < 3; ++d) nc[d] = std::max(1, std::min(1024, (int)std::floor(h.perp[d] / 4.0)));
-        std::vector<uint64_t> key(n);
-        std::vector<double> f(3 * (size_t)n);
-        for (int j = 0; j < n; ++j) {
-            uint32_t c[3];
-            for (int d = 0; d < 3; ++d) {
-                const double x = fr[3 * j + d] - std::floor(fr[3 * j + d]);
-                f[3 * j + d] = x;
-                c[d] = (uint32_t)std::min(nc[d] - 1, (int)(x * nc[d]));
-            }
-            const uint64_t m = spread3(c[0]) | (spread3(c[1]) << 1) | (spread3(c[2]) << 2);
-            key[j] = (m << 32) | (uint32_t)j;
-        }
-        std::sort(key.begin(), key.end());
-        for (int i = 0; i < n; ++i) {
-            const int j = (int)(key[i] & 0xFFFFFFFFu);
-            af[F.atom_off + i] = make_double4(f[3 * j], f[3 * j + 1], f[3 * j + 2], b->atom64_h[F.atom_off + j].w);
-            at[F.atom_off + i] = b->atype_h[F.atom_off + j];
-        }
-        for (int i0 = 0; i0 < n; i0 += 64) {
-            const int m = std::min(64, n - i0);
-            const double4 *p = &af[F.atom_off + i0];
-            double x[64][3], c[3] = {0, 0, 0}, rad2 = 0.0;
-            for (int i = 0; i < m; ++i) {
-                const double d[3] = {p[i].x - p[0].x, p[i].y - p[0].y, p[i].z - p[0].z};
-                for (int e = 0; e < 3; ++e) {
-                    x[i][e] = d[e] - std::rint(d[e]);
-                    c[e] += x[i][e] / m;
-                }
-            }
-            for (int i = 0; i < m; ++i) {
-                const double d[3] = {x[i][0] - c[0], x[i][1] - c[1], x[i][2] - c[2]};
-                double v[3];
-                matvec(F.A, d, v);
-                rad2 = std::max(rad2, v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-            }
-            run.push_back(make_double4(p[0].x + c[0], p[0].y + c[1], p[0].z + c[2], std::sqrt(rad2) + 1.0e-6));
-        }
-        run_off.push_back((int)run.size());
+    if (!FILL && lane == 0) {
+        a.start[b] = total;
+        if (b + 1 == a.nbins) a.start[b + 1] = 0;  // the slot past the last bin
     }
-    if (run.empty()) run.push_back(make_double4(0, 0, 0, 0));
-    return PA_OK;
 }
 
-// Builds the batch's near lists once (the first chain state or FP64 Widom call needs them).
-int ensure_near_lists(pa_batch *b)
+hipError_t launch_near_runs(const NearBuild &a, hipStream_t st)
 {
-    if (b->near_ready) return PA_OK;
-    std::vector<double4> af, run;
-    std::vector<int> at, run_off;
-    int st = near_atoms(b, af, at, run, run_off);
-    if (st) return st;
+    if (a.nruns <= 0) return hipSuccess;
+    hipLaunchKernelGGL(near_run_kernel, dim3((unsigned)((a.nruns + 3) / 4)), dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_near_build(bool fill, const NearBuild &a, hipStream_t st)
+{
+    const dim3 grid((unsigned)((a.nbins + 3) / 4)), block(256);
+    if (fill) hipLaunchKernelGGL(near_kernel<true>, grid, block, 0, st, a);
+    else hipLaunchKernelGGL(near_kernel<false>, grid, block, 0, st, a);
+    return hipGetLastError();
+}
+
+// The near lists' bins of every framework, and what their kernels share. False: the batch has none, since a
+// framework has more atoms than an entry can name, or the lists would not fit.
+bool near_bins(const pa_batch *b, NearBuild &a, std::vector<NearDesc> &nd, std::vector<int> &bin_fw, std::vector<int> &run_off)
+{
     const double rcmax = std::max(b->rc_lj, b->gdev.charged ? b->rc_ew : 0.0);
-    std::vector<NearDesc> nd(b->nfw);
-    std::vector<int> bin_fw(b->nfw + 1, 0);
+    nd.resize(b->nfw);
+    bin_fw.assign(b->nfw + 1, 0);
+    run_off.assign(b->nfw + 1, 0);
+    for (int u = 0; u < b->nfw; ++u) {
+        if (b->desc[u].natoms >= (1 << NEAR_TYPE_SHIFT)) return false;
+        run_off[u + 1] = run_off[u] + (b->desc[u].natoms + 63) / 64;
+    }
     for (double edge = NEAR_EDGE;; edge *= 1.26) {
+        if (edge > 1000.0) return false;
         double entries = 0.0;
         int64_t nbins = 0;
         for (int u = 0; u < b->nfw; ++u) {
             const FwHost &h = b->info[u];
             const FwDesc &F = b->desc[u];
-            if (F.natoms >= (1 << NEAR_TYPE_SHIFT))
-                return fail(PA_ERR_ARG, "framework %d: %d atoms exceed 2^%d", u + 1, F.natoms, NEAR_TYPE_SHIFT);
             NearDesc &D = nd[u];
             for (int d = 0; d < 3; ++d) D.nb[d] = std::max(1, std::min(512, (int)std::ceil(h.perp[d] / edge)));
             double rb = 0.0;  // circumradius: half the longest body diagonal
@@ -412,51 +369,15 @@ int ensure_near_lists(pa_batch *b)
             nbins += n;
             entries += (double)n * std::min<double>(F.natoms, F.natoms / h.volume * (4.0 / 3.0) * PI * R * R * R);
         }
-        bin_fw[b->nfw] = (int)std::min<int64_t>(nbins, INT32_MAX);
-        if ((entries <= NEAR_MAX_ENTRIES && nbins < (1 << 26)) || edge > 1000.0) break;
+        // an atom is in at most ((R + rb) / R)^3 < 8 times as many lists as the volume of its sphere
+        // holds bins, so that lists of 2^28 entries by volume have offsets below 2^31
+        if (entries > NEAR_MAX_ENTRIES || nbins >= (1 << 26)) continue;
+        bin_fw[b->nfw] = (int)nbins;
+        a.nfw = b->nfw;
+        a.nbins = (int)nbins;
+        a.nruns = run_off[b->nfw];
+        return true;
     }
-    const int nbins = bin_fw[b->nfw];
-    HIP_TRY(upload(b->d_nearf, af));
-    HIP_TRY(upload(b->d_neart, at));
-    HIP_TRY(upload(b->d_near_desc, nd));
-    DevAlloc d_fw, d_run, d_run_off;
-    HIP_TRY(upload(d_fw, bin_fw));
-    HIP_TRY(upload(d_run, run));
-    HIP_TRY(upload(d_run_off, run_off));
-    HIP_TRY(b->d_near_start.ensure(sizeof(int) * (nbins + 1)));
-    NearBuild a{};
-    a.fw = b->d_fw.as<FwDesc>();
-    a.nd = b->d_near_desc.as<NearDesc>();
-    a.bin_fw = d_fw.as<int>();
-    a.nfw = b->nfw;
-    a.nbins = nbins;
-    a.atomf = b->d_nearf.as<double4>();
-    a.atype = b->d_neart.as<int>();
-    a.run = d_run.as<double4>();
-    a.run_off = d_run_off.as<int>();
-    a.start = b->d_near_start.as<int>();
-    const dim3 grid((unsigned)((nbins + 3) / 4)), block(256);
-    hipLaunchKernelGGL(near_kernel<false>, grid, block, 0, b->stream, a);
-    HIP_TRY(hipGetLastError());
-    std::vector<int> cnt(nbins + 1);
-    HIP_TRY(hipMemcpyAsync(cnt.data(), b->d_near_start.p, sizeof(int) * nbins, hipMemcpyDeviceToHost, b->stream));
-    HIP_TRY(hipStreamSynchronize(b->stream));
-    int64_t total = 0;
-    for (int i = 0; i < nbins; ++i) {
-        const int c = cnt[i];
-        cnt[i] = (int)total;
-        total += c;
-        if (total > (int64_t)INT32_MAX) return fail(PA_ERR_ARG, "the frameworks' near lists exceed 2^31 entries");
-    }
-    cnt[nbins] = (int)total;
-    HIP_TRY(hipMemcpyAsync(b->d_near_start.p, cnt.data(), sizeof(int) * (nbins + 1), hipMemcpyHostToDevice, b->stream));
-    HIP_TRY(b->d_near_ent.ensure(sizeof(uint32_t) * (size_t)std::max<int64_t>(total, 1)));
-    a.ent = b->d_near_ent.as<uint32_t>();
-    hipLaunchKernelGGL(near_kernel<true>, grid, block, 0, b->stream, a);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(b->stream));
-    b->near_ready = true;
-    return PA_OK;
 }
 
 NearLists near_lists(const pa_batch *b)

@@ -1176,12 +1176,14 @@ int build_k_runs(pa_state *st)
     return PA_OK;
 }
 
-// Tables of the move and chain-insertion kernels beyond build_k_runs: the batch's near lists, and
-// each system's slice of a snapshot's structure factors.
+// Tables of the move and chain-insertion kernels beyond build_k_runs: each system's slice of a
+// snapshot's structure factors. (Their real-space part goes over the batch's near lists.)
 int ensure_chain_tables(pa_state *st)
 {
     if (st->d_coff.p) return PA_OK;
-    if (int e = ensure_near_lists(st->b)) return e;
+    if (!st->b->near_ready)
+        return fail(PA_ERR_ARG, "a framework of the batch has more atoms (2^%d) than the chains' lists of near atoms hold",
+                    NEAR_TYPE_SHIFT);
     st->ctot = st->sk_off[st->nsys];
     HIP_TRY(upload(st->d_coff, st->sk_off));
     return PA_OK;

@@ -493,6 +493,20 @@ struct NearLists {
     const uint32_t *ent;
 };
 
+// What the kernels share that build the lists (batch_kernels.hip).
+struct NearBuild {
+    const FwDesc *fw;
+    const NearDesc *nd;
+    const int *bin_fw;         // nfw + 1: first bin of every framework
+    const int *run_off;        // nfw + 1: first run of 64 atoms of every framework
+    int nfw, nbins, nruns;
+    const double4 *atomf;
+    const int *atype;          // in the same order
+    double4 *run;              // per run of 64 atoms: centre (fractional), radius (Å)
+    int *start;                // nbins + 1: counts (first pass), then offsets
+    uint32_t *ent;             // entries (second pass)
+};
+
 // The bin of a point with fractional coordinates f.
 __device__ inline int near_bin(const NearDesc &D, const double f[3])
 {

@@ -222,9 +222,9 @@ struct pa_batch {
     std::vector<double2> S64_h;
     std::vector<int> atype_h;
     pa::DevAlloc d_corefx, d_coreidx, d_cell_start, d_rho2, d_cand, d_ncand, d_nbr_start, d_nbr_atoms, d_passes;
-    pa::DevAlloc d_binfx, d_bintype;  // the atoms in Morton order, for the mixed path's list build
-    // FP64 paths: lists of the atoms near a point, built on first use (batch_kernels.hip)
-    pa::DevAlloc d_nearf, d_neart, d_near_desc, d_near_start, d_near_ent, d_rho2_64;
+    pa::DevAlloc d_binfx, d_bintype;  // the atoms in Morton order, as d_nearf, for the mixed path's list build
+    // FP64 paths: lists of the atoms near a point, if near_ready (batch_kernels.hip)
+    pa::DevAlloc d_nearf, d_near_desc, d_near_start, d_near_ent, d_rho2_64;
     bool near_ready = false;
     // gradient scratch
     pa::PinnedAlloc h_acc_q;  // gradient path: the per-atom charge accumulators read back
@@ -249,7 +249,6 @@ struct pa_batch {
 namespace pa {
 // Squared phase-0 rejection radii of system s at kT, NS x ntypes_c (build_rejection_tables).
 int rejection_radii(const pa_batch *b, int s, double kT, double eps_f, double *rho2, double *rmax2);
-// The batch's near lists (batch_kernels.hip): builds them once; their device form.
-int ensure_near_lists(pa_batch *b);
+// The device form of the batch's near lists.
 NearLists near_lists(const pa_batch *b);
 }  // namespace pa

@@ -40,6 +40,9 @@ hipError_t launch_grad_recip(const GradArgs &a, const double4 *k64, const int4 *
 hipError_t launch_sk(const double4 *atoms, int natoms, const int4 *kreq, int nreq, double2 *out, hipStream_t st);
 hipError_t launch_nbr(bool fill, const FwDesc *fw, int nfw, const int *cell_fw_off, int ncells, const int *cell_start,
                       int *nbr_start, const uint4 *corefx, uint4 *nbr_atoms, hipStream_t st);
+bool near_bins(const pa_batch *b, NearBuild &a, std::vector<NearDesc> &nd, std::vector<int> &bin_fw, std::vector<int> &run_off);
+hipError_t launch_near_runs(const NearBuild &a, hipStream_t st);
+hipError_t launch_near_build(bool fill, const NearBuild &a, hipStream_t st);
 hipError_t scan_counts(int *counts, int n, void *tmp, size_t *tmp_bytes, hipStream_t st);
 hipError_t launch_self_term(const int4 *kn, const double *kpref, int nk, const double *gsf, const double *q, int ns,
                             double *partial, hipStream_t st);
@@ -470,6 +473,7 @@ struct BatchTables {
     std::vector<int> coreidx, cell_start;
     std::vector<uint4> binfx;           // the atoms in Morton order (mixed path's list build)
     std::vector<int> bintype;
+    std::vector<double4> nearf;         // fractional coordinates in [0, 1) and charge, same order
     std::vector<int> cell_fw_off{0};    // prefix over frameworks of their cell counts
     std::vector<double2> pair64;
     std::vector<float2> pair32;
@@ -500,24 +504,29 @@ int add_atoms(BatchTables &T, FwDesc &D, const double *frac, const double *cart,
         std::memcpy(&qb, &qf, 4);
         T.atomfx.push_back(make_uint4(to_fixed(f[0]), to_fixed(f[1]), to_fixed(f[2]), qb));
     }
-    // the mixed path's list build reads the atoms in Morton order of their fixed-point coordinates
+    // the mixed path's list build and the FP64 paths' lists read the atoms in Morton order of their fixed-point coordinates
     // (the top 10 bits per axis, ties by index): a wavefront's 64 atoms then lie close together,
     // so an image across a cell boundary is either needed by some of them or skipped by all
     {
-        auto spread = [](uint32_t v) {
-            uint64_t x = 0;
-            for (int i = 0; i < 10; ++i) x |= (uint64_t)((v >> i) & 1u) << (3 * i);
-            return x;
+        auto spread = [](uint32_t v) {  // the low 10 bits to every third bit
+            v = (v | (v << 16)) & 0x030000FF;
+            v = (v | (v << 8)) & 0x0300F00F;
+            v = (v | (v << 4)) & 0x030C30C3;
+            return (v | (v << 2)) & 0x09249249;
         };
-        std::vector<std::pair<uint64_t, int>> key((size_t)n);
+        std::vector<uint64_t> key((size_t)n);
         for (int j = 0; j < n; ++j) {
             const uint4 &x = T.atomfx[D.atom_off + j];
-            key[j] = {spread(x.x >> 22) | (spread(x.y >> 22) << 1) | (spread(x.z >> 22) << 2), j};
+            const uint32_t m = spread(x.x >> 22) | (spread(x.y >> 22) << 1) | (spread(x.z >> 22) << 2);
+            key[j] = ((uint64_t)m << 32) | (uint32_t)j;
         }
         std::sort(key.begin(), key.end());
         for (int i = 0; i < n; ++i) {
-            T.binfx.push_back(T.atomfx[D.atom_off + key[i].second]);
-            T.bintype.push_back(T.atype[D.atom_off + key[i].second]);
+            const int j = (int)(uint32_t)key[i];
+            T.binfx.push_back(T.atomfx[D.atom_off + j]);
+            T.bintype.push_back(T.atype[D.atom_off + j]);
+            const double *f = frac + 3 * (size_t)j;
+            T.nearf.push_back(make_double4(f[0] - std::floor(f[0]), f[1] - std::floor(f[1]), f[2] - std::floor(f[2]), q[j]));
         }
     }
     // hard-core cell grid: cells of at least HC_CELL Å, at most 64 per axis; atoms sorted by cell
@@ -597,7 +606,8 @@ int near_list_radii(pa_batch *b)
 }
 
 // Creates the batch's stream and events, uploads every table and builds the phase-0 near lists
-// on the device.
+// and those of the FP64 paths on the device. (The latter with the batch and not on the first FP64 call:
+// that call may be one that must not allocate, or one of several states made on several threads.)
 int upload_batch(pa_batch *b, const BatchTables &T)
 {
     int st = device_ready();
@@ -624,26 +634,60 @@ int upload_batch(pa_batch *b, const BatchTables &T)
     HIP_TRY(upload(b->d_bintype, T.bintype));
     HIP_TRY(upload(b->d_coreidx, T.coreidx));
     HIP_TRY(upload(b->d_cell_start, T.cell_start));
+    HIP_TRY(upload(b->d_nearf, T.nearf));
+    HIP_TRY(b->d_rho2_64.ensure(sizeof(double) * (size_t)b->nsys * b->nsites * b->ntypes_c));
     {
-        DevAlloc d_cfo, tmp;
-        HIP_TRY(upload(d_cfo, T.cell_fw_off));
+        // both kinds of lists together: counted, scanned to offsets, filled
+        std::vector<NearDesc> nd;
+        std::vector<int> ints, run_off;
+        NearBuild nb{};
+        const bool near = near_bins(b, nb, nd, ints, run_off);
+        const size_t bin_fw_n = ints.size();
+        ints.insert(ints.end(), run_off.begin(), run_off.end());
+        ints.insert(ints.end(), T.cell_fw_off.begin(), T.cell_fw_off.end());
+        DevAlloc d_ints, d_run, tmp;
+        HIP_TRY(upload(d_ints, ints));
+        const int *cell_fw_off = d_ints.as<int>() + bin_fw_n + run_off.size();
         const int n = (int)T.cell_start.size(), ncells = T.cell_fw_off.back();
         HIP_TRY(b->d_nbr_start.ensure(sizeof(int) * std::max(n, 1)));
-        int *start = b->d_nbr_start.as<int>(), total = 0;
+        int *start = b->d_nbr_start.as<int>(), total[2] = {0, 0};
         auto nbr = [&](bool fill, uint4 *out) {
-            return launch_nbr(fill, b->d_fw.as<FwDesc>(), b->nfw, d_cfo.as<int>(), ncells, b->d_cell_start.as<int>(), start,
+            return launch_nbr(fill, b->d_fw.as<FwDesc>(), b->nfw, cell_fw_off, ncells, b->d_cell_start.as<int>(), start,
                               b->d_corefx.as<uint4>(), out, b->stream);
         };
-        HIP_TRY(nbr(false, nullptr));
         size_t bytes = 0;
-        HIP_TRY(scan_counts(start, n, nullptr, &bytes, b->stream));
+        HIP_TRY(scan_counts(start, std::max(n, nb.nbins + 1), nullptr, &bytes, b->stream));
         HIP_TRY(tmp.ensure(bytes));
+        HIP_TRY(nbr(false, nullptr));
         HIP_TRY(scan_counts(start, n, tmp.p, &bytes, b->stream));
-        HIP_TRY(hipMemcpyAsync(&total, start + (n - 1), sizeof(int), hipMemcpyDeviceToHost, b->stream));
+        HIP_TRY(hipMemcpyAsync(&total[0], start + (n - 1), sizeof(int), hipMemcpyDeviceToHost, b->stream));
+        if (near) {
+            HIP_TRY(upload(b->d_near_desc, nd));
+            HIP_TRY(b->d_near_start.ensure(sizeof(int) * ((size_t)nb.nbins + 1)));
+            HIP_TRY(d_run.ensure(sizeof(double4) * (size_t)std::max(nb.nruns, 1)));
+            nb.fw = b->d_fw.as<FwDesc>();
+            nb.nd = b->d_near_desc.as<NearDesc>();
+            nb.bin_fw = d_ints.as<int>();
+            nb.run_off = d_ints.as<int>() + bin_fw_n;
+            nb.atomf = b->d_nearf.as<double4>();
+            nb.atype = b->d_bintype.as<int>();
+            nb.run = d_run.as<double4>();
+            nb.start = b->d_near_start.as<int>();
+            HIP_TRY(launch_near_runs(nb, b->stream));
+            HIP_TRY(launch_near_build(false, nb, b->stream));
+            HIP_TRY(scan_counts(nb.start, nb.nbins + 1, tmp.p, &bytes, b->stream));
+            HIP_TRY(hipMemcpyAsync(&total[1], nb.start + nb.nbins, sizeof(int), hipMemcpyDeviceToHost, b->stream));
+        }
         HIP_TRY(hipStreamSynchronize(b->stream));
-        HIP_TRY(b->d_nbr_atoms.ensure(sizeof(uint4) * (size_t)std::max(1, total)));
+        HIP_TRY(b->d_nbr_atoms.ensure(sizeof(uint4) * (size_t)std::max(1, total[0])));
         HIP_TRY(nbr(true, b->d_nbr_atoms.as<uint4>()));
+        if (near) {
+            HIP_TRY(b->d_near_ent.ensure(sizeof(uint32_t) * (size_t)std::max(1, total[1])));
+            nb.ent = b->d_near_ent.as<uint32_t>();
+            HIP_TRY(launch_near_build(true, nb, b->stream));
+        }
         HIP_TRY(hipStreamSynchronize(b->stream));
+        b->near_ready = near;
     }
     return PA_OK;
 }
@@ -1474,13 +1518,12 @@ static int run_energies(pa_batch *b, const std::vector<int64_t> &seg, int64_t gb
     SCR_TRY(b, scr.put(b->d_seg, seg, &d_seg));
     *launches = 0;
     if ((precision & ~PA_SINGLE_PHASE) == PA_PREC_F64) {
-        // two-phase calls (kT > 0) go over the near lists, which the first of them builds; a call
-        // into a fixed scratch region uses them only if they are there. Single energies and
-        // PA_SINGLE_PHASE calls take the plain kernel.
+        // two-phase calls (kT > 0) go over the near lists; single energies and PA_SINGLE_PHASE calls
+        // take the plain kernel. The choice follows from the batch's sizes alone, so that a call
+        // into a fixed scratch region makes the same one whatever ran before it.
         F64Call c{d_seg, false, 0};
         for (const FwDesc &D : b->desc) c.tab_w = std::max(c.tab_w, D.kn_max[0] + D.kn_max[1] + D.kn_max[2] + 3);
-        c.near = kT > 0.0 && (!b->gdev.charged || c.tab_w <= near_tab_max(b->nsites));
-        if (c.near && !b->near_ready) c.near = !scr.base && ensure_near_lists(b) == PA_OK;
+        c.near = kT > 0.0 && b->near_ready && (!b->gdev.charged || c.tab_w <= near_tab_max(b->nsites));
         double *d_r2 = nullptr;
         if (c.near) {
             const size_t per_sys = (size_t)b->nsites * b->ntypes_c;
@@ -1494,7 +1537,10 @@ static int run_energies(pa_batch *b, const std::vector<int64_t> &seg, int64_t gb
                 }
                 b->rr64_kT = kT;
             }
-            SCR_TRY(b, scr.put(b->d_rho2_64, b->rr64_r2, &d_r2));
+            // into the batch's own buffer, allocated with it: a fixed scratch region has to hold no more
+            // than for the plain kernel
+            HIP_TRY(upload_cached(b->d_rho2_64, b->rr64_r2));
+            d_r2 = b->d_rho2_64.as<double>();
         }
         if (f64) *f64 = c;
         return launch_f64(b, c, d_r2, gb, ge, out_base, seed, chunk, launches, dU);

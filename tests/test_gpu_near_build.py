@@ -1,8 +1,11 @@
-"""The FP64 paths' near lists as they are built (MI355X): large and long cells, whose
-atoms the build tries in runs of 64.
+"""The FP64 paths' near lists as the batch's creation builds them (MI355X): large and long cells, whose
+atoms the build tries in runs of 64, and what finds the lists: a no-allocation call that comes
+first, and states made on several host threads.
 
 Two-phase against single_phase (the plain kernel, every pair): FP64 sums of some 1e3 terms in
 another order, 1e-9 as for the FP64 results against the oracle."""
+import threading
+
 import pytest
 
 import pureadsorb_amd as pa
@@ -34,3 +37,40 @@ def test_lists_of_large_and_long_cells(cell, atoms, guest):
     for r, p in zip(near, plain):
         for k in FIELDS:
             assert getattr(r, k) == pytest.approx(getattr(p, k), rel=1e-9, abs=1e-9 if k == "q_st_err" else 1e-300), k
+
+
+@pytest.mark.parametrize("precision", ["f64", "mixed"])
+def test_first_call_without_allocation(precision):
+    """On a batch that has made no other call, then beside pa_widom, then again: the same fields."""
+    ff, g, ew = _system()
+    fws = [pa.replicate(synth.synthetic_framework(13.0, 13.0, 15.0, 90, 90, 120, n, 42, charge_sd=0.2), (3, 3, 2))
+           for n in (40, 300)]
+    # (the second one binds nothing, which the mixed path refuses)
+    b = pa.FrameworkBatch(fws if precision == "f64" else fws[:1], ff, g, ew)
+    kw = dict(T=T, ninsert=10_000, seed=3, nblocks=5, precision=precision)
+    first = pa.widom(b, g, **kw, no_alloc=True)
+    assert first == pa.widom(b, g, **kw) == pa.widom(b, g, **kw, no_alloc=True)
+
+
+def test_states_made_on_several_threads():
+    ff, g, ew = _system()
+    fw = pa.replicate(synth.synthetic_framework(13.0, 13.0, 15.0, 90, 90, 120, 40, 42, charge_sd=0.2), (3, 3, 2))
+    b = pa.FrameworkBatch([fw] * 4, ff, g, ew, fullk=True)
+    want = pa.SystemState(b, g, [3] * 4, T=T, seed=7, capacities=[20] * 4)
+    got, errors = [None] * 6, []
+
+    def make(i):
+        try:
+            got[i] = pa.SystemState(b, g, [3] * 4, T=T, seed=7, capacities=[20] * 4)
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=make, args=(i,)) for i in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
+    ref = pa.mc_moves(want, pa.MOVE_TRANSLATION, 40, T=T, step_trans=0.5, trace=True)
+    for st in got:
+        assert (pa.mc_moves(st, pa.MOVE_TRANSLATION, 40, T=T, step_trans=0.5, trace=True) == ref).all()
