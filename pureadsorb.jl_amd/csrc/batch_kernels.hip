@@ -86,13 +86,13 @@ __device__ inline R length2(const R A[9], R x, R y, R z)
 // Phase-0 near lists: for every hard-core cell, the atoms within nbr_r of any point of it, by their
 // minimum-image distance to the cell's centre. One wavefront per cell, its lanes over the cells
 // within nbr_reach (each once where the reach goes around the axis). Without FILL the lists are
-// counted into nbr_start; with it they are written in three shells of growing distance, so that
+// counted into nbr_start (and their sum added to *sum); with it they are written in three shells of growing distance, so that
 // an insertion's overlap is usually found among the first entries. cell_fw_off (nfw + 1) maps the
 // global cell index to its framework.
 template <bool FILL>
 __global__ __launch_bounds__(BK_WG) void nbr_kernel(const FwDesc *fw, int nfw, const int *cell_fw_off, int ncells,
                                                    const int *cell_start, int *nbr_start, const uint4 *corefx,
-                                                   uint4 *nbr_atoms)
+                                                   uint4 *nbr_atoms, unsigned long long *sum)
 {
     const int lane = threadIdx.x & 63;
     const int g = blockIdx.x * (BK_WG / 64) + (threadIdx.x >> 6);
@@ -146,6 +146,7 @@ __global__ __launch_bounds__(BK_WG) void nbr_kernel(const FwDesc *fw, int nfw, c
             }
         }
     if (!FILL && lane == 0) nbr_start[D.cg_off + c] = total;
+    if (!FILL && sum && lane == 0 && total) atomicAdd(sum, (unsigned long long)total);
     // the slot past a framework's last cell: no atoms
     if (!FILL && lane == 0 && g + 1 == cell_fw_off[lo + 1]) nbr_start[D.cg_off + c + 1] = 0;
 }
@@ -157,16 +158,16 @@ hipError_t scan_counts(int *counts, int n, void *tmp, size_t *tmp_bytes, hipStre
 }
 
 hipError_t launch_nbr(bool fill, const FwDesc *fw, int nfw, const int *cell_fw_off, int ncells, const int *cell_start,
-                      int *nbr_start, const uint4 *corefx, uint4 *nbr_atoms, hipStream_t st)
+                      int *nbr_start, const uint4 *corefx, uint4 *nbr_atoms, unsigned long long *sum, hipStream_t st)
 {
     if (ncells <= 0) return hipSuccess;
     const dim3 grid((unsigned)((ncells + BK_WG / 64 - 1) / (BK_WG / 64))), block(BK_WG);
     if (fill)
         hipLaunchKernelGGL(nbr_kernel<true>, grid, block, 0, st, fw, nfw, cell_fw_off, ncells, cell_start, nbr_start,
-                           corefx, nbr_atoms);
+                           corefx, nbr_atoms, sum);
     else
         hipLaunchKernelGGL(nbr_kernel<false>, grid, block, 0, st, fw, nfw, cell_fw_off, ncells, cell_start, nbr_start,
-                           corefx, nbr_atoms);
+                           corefx, nbr_atoms, sum);
     return hipGetLastError();
 }
 

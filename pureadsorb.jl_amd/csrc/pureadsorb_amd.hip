@@ -39,7 +39,7 @@ hipError_t grad_select(const double *dU, const int64_t *seg, int nsys, const dou
 hipError_t launch_grad_recip(const GradArgs &a, const double4 *k64, const int4 *rblk, int nrblk, hipStream_t st);
 hipError_t launch_sk(const double4 *atoms, int natoms, const int4 *kreq, int nreq, double2 *out, hipStream_t st);
 hipError_t launch_nbr(bool fill, const FwDesc *fw, int nfw, const int *cell_fw_off, int ncells, const int *cell_start,
-                      int *nbr_start, const uint4 *corefx, uint4 *nbr_atoms, hipStream_t st);
+                      int *nbr_start, const uint4 *corefx, uint4 *nbr_atoms, unsigned long long *sum, hipStream_t st);
 bool near_bins(const pa_batch *b, NearBuild &a, std::vector<NearDesc> &nd, std::vector<int> &bin_fw, std::vector<int> &run_off);
 hipError_t launch_near_runs(const NearBuild &a, hipStream_t st);
 hipError_t launch_near_build(bool fill, const NearBuild &a, hipStream_t st);
@@ -564,10 +564,8 @@ int add_atoms(BatchTables &T, FwDesc &D, const double *frac, const double *cart,
     return PA_OK;
 }
 
-// Radius, distance threshold and cell reach of every framework's phase-0 near lists: the largest
-// rejection radius at HC_LIST_T, scaled down until the lists stay below 2^31 entries (each atom is
-// in at most prod(2 reach + 1) of them).
-int near_list_radii(pa_batch *b)
+// The largest phase-0 rejection radius at HC_LIST_T, per framework.
+std::vector<double> near_list_radii(const pa_batch *b)
 {
     std::vector<double> r(b->nfw, -1.0), rho2((size_t)b->nsites * b->ntypes_c);
     for (int s = 0; s < b->nsys; ++s) {
@@ -577,32 +575,37 @@ int near_list_radii(pa_batch *b)
         if (rejection_radii(b, s, KB * HC_LIST_T, (double)FLT_EPSILON, rho2.data(), &rmax2)) rmax2 = 0.0;
         r[u] = std::sqrt(rmax2) * (1.0 + 1e-6);
     }
-    for (double scale = 1.0;; scale *= 0.7) {
-        double entries = 0.0;
-        for (int u = 0; u < b->nfw; ++u) {
-            FwDesc &D = b->desc[u];
-            const FwHost &h = b->info[u];
-            const double R = r[u] * scale;
-            double rc = 0.0, per_atom = 1.0;  // circumradius of a cell: half its longest body diagonal
-            for (int sy = -1; sy <= 1; sy += 2)
-                for (int sz = -1; sz <= 1; sz += 2) {
-                    const double f[3] = {0.5 / D.cg_nc[0], 0.5 * sy / D.cg_nc[1], 0.5 * sz / D.cg_nc[2]};
-                    double v[3];
-                    matvec(D.A, f, v);
-                    rc = std::max(rc, norm3(v));
-                }
-            const double thr = (R + rc) * (1.0 + 1.0e-5) + 1.0e-3;  // FP32 distances on the device
-            D.nbr_r = std::nextafter((float)R, 0.0f);
-            D.nbr_thr2 = (float)(thr * thr);
-            for (int d = 0; d < 3; ++d) {
-                D.nbr_reach[d] = std::max(1, (int)std::ceil(thr * D.cg_nc[d] / h.perp[d] + 0.5));
-                per_atom *= std::min(D.cg_nc[d], 2 * D.nbr_reach[d] + 1);
+    return r;
+}
+
+// Radius, distance threshold and cell reach of every framework's phase-0 near lists for the radii r.
+// Returns a bound on their entries: an atom is in the lists of the cells whose centres lie within thr of
+// it, and those cells lie in the sphere of thr and their circumradius.
+double set_near_radii(pa_batch *b, const std::vector<double> &r)
+{
+    double entries = 0.0;
+    for (int u = 0; u < b->nfw; ++u) {
+        FwDesc &D = b->desc[u];
+        const FwHost &h = b->info[u];
+        double rc = 0.0, cells = 1.0;  // circumradius of a cell: half its longest body diagonal
+        for (int sy = -1; sy <= 1; sy += 2)
+            for (int sz = -1; sz <= 1; sz += 2) {
+                const double f[3] = {0.5 / D.cg_nc[0], 0.5 * sy / D.cg_nc[1], 0.5 * sz / D.cg_nc[2]};
+                double v[3];
+                matvec(D.A, f, v);
+                rc = std::max(rc, norm3(v));
             }
-            entries += per_atom * D.natoms;
+        const double thr = (r[u] + rc) * (1.0 + 1.0e-5) + 1.0e-3;  // FP32 distances on the device
+        D.nbr_r = std::nextafter((float)r[u], 0.0f);
+        D.nbr_thr2 = (float)(thr * thr);
+        for (int d = 0; d < 3; ++d) {
+            D.nbr_reach[d] = std::max(1, (int)std::ceil(thr * D.cg_nc[d] / h.perp[d] + 0.5));
+            cells *= D.cg_nc[d];
         }
-        if (entries < (double)INT32_MAX) return PA_OK;
-        if (scale < 0.05) return fail(PA_ERR_ARG, "the frameworks' phase-0 neighbour lists exceed 2^31 entries");
+        const double far = thr + rc;
+        entries += D.natoms * std::min(cells, 4.0 / 3.0 * PI * far * far * far * cells / h.volume * (1.0 + 1.0e-3));
     }
+    return entries;
 }
 
 // Creates the batch's stream and events, uploads every table and builds the phase-0 near lists
@@ -617,8 +620,6 @@ int upload_batch(pa_batch *b, const BatchTables &T)
     // timing-only events: no system-scope fence (no cache write-back and invalidation around the
     // kernels they bracket); results reach the host through copies and stream synchronisation
     for (auto &e : b->ev) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableSystemFence));
-    if (int e = near_list_radii(b)) return e;
-    HIP_TRY(upload(b->d_fw, b->desc));
     HIP_TRY(upload(b->d_fw_of, b->fw_of));
     HIP_TRY(upload(b->d_atom64, T.atom64));
     HIP_TRY(upload(b->d_atype, T.atype));
@@ -651,14 +652,31 @@ int upload_batch(pa_batch *b, const BatchTables &T)
         const int n = (int)T.cell_start.size(), ncells = T.cell_fw_off.back();
         HIP_TRY(b->d_nbr_start.ensure(sizeof(int) * std::max(n, 1)));
         int *start = b->d_nbr_start.as<int>(), total[2] = {0, 0};
-        auto nbr = [&](bool fill, uint4 *out) {
+        auto nbr = [&](bool fill, uint4 *out, unsigned long long *sum) {
             return launch_nbr(fill, b->d_fw.as<FwDesc>(), b->nfw, cell_fw_off, ncells, b->d_cell_start.as<int>(), start,
-                              b->d_corefx.as<uint4>(), out, b->stream);
+                              b->d_corefx.as<uint4>(), out, sum, b->stream);
         };
         size_t bytes = 0;
         HIP_TRY(scan_counts(start, std::max(n, nb.nbins + 1), nullptr, &bytes, b->stream));
         HIP_TRY(tmp.ensure(bytes));
-        HIP_TRY(nbr(false, nullptr));
+        // The phase-0 lists' offsets have 31 bits. Where a bound does not settle that (from some ten million
+        // atoms on) the entries are counted, and only lists that really exceed it get smaller radii,
+        // with which phase 0 has to go through the full stencil too.
+        std::vector<double> r = near_list_radii(b);
+        DevAlloc d_sum;
+        for (double scale = 1.0;; scale *= 0.8) {
+            const bool sure = set_near_radii(b, r) < (double)INT32_MAX;
+            unsigned long long sum = 0;
+            HIP_TRY(upload(b->d_fw, b->desc));
+            if (!sure) HIP_TRY(upload(d_sum, std::vector<unsigned long long>(1, 0)));
+            HIP_TRY(nbr(false, nullptr, sure ? nullptr : d_sum.as<unsigned long long>()));
+            if (sure) break;
+            HIP_TRY(hipMemcpyAsync(&sum, d_sum.p, sizeof sum, hipMemcpyDeviceToHost, b->stream));
+            HIP_TRY(hipStreamSynchronize(b->stream));
+            if (sum < (unsigned long long)INT32_MAX) break;
+            if (scale < 0.05) return fail(PA_ERR_ARG, "the frameworks' phase-0 neighbour lists exceed 2^31 entries");
+            for (double &x : r) x *= 0.8;
+        }
         HIP_TRY(scan_counts(start, n, tmp.p, &bytes, b->stream));
         HIP_TRY(hipMemcpyAsync(&total[0], start + (n - 1), sizeof(int), hipMemcpyDeviceToHost, b->stream));
         if (near) {
@@ -680,7 +698,7 @@ int upload_batch(pa_batch *b, const BatchTables &T)
         }
         HIP_TRY(hipStreamSynchronize(b->stream));
         HIP_TRY(b->d_nbr_atoms.ensure(sizeof(uint4) * (size_t)std::max(1, total[0])));
-        HIP_TRY(nbr(true, b->d_nbr_atoms.as<uint4>()));
+        HIP_TRY(nbr(true, b->d_nbr_atoms.as<uint4>(), nullptr));
         if (near) {
             HIP_TRY(b->d_near_ent.ensure(sizeof(uint32_t) * (size_t)std::max(1, total[1])));
             nb.ent = b->d_near_ent.as<uint32_t>();
