@@ -17,7 +17,8 @@
 //       x_r [z_r (c+_r + c-_r) + z_i (c+_i - c-_i)] + x_i [z_r (c+_i + c-_i) + z_i (c-_r - c+_r)],
 //     so the brackets are summed over j first: 4 fused multiply-adds per site for two k-vectors
 //     (a recurrence with one complex product per k-vector and site took 8 each). Phases come from
-//     per-axis tables in LDS;
+//     per-axis tables in LDS, or are evaluated where they are used in a cell so long that LDS does not
+//     hold its tables;
 //   * guest-guest: lanes take (guest, site) pairs against every site, through the same queue.
 // The pose is drawn exactly as the Widom path draws it, `per` insertions of a wavefront one per
 // lane; the energy terms use fused multiply-adds. FP64 issue bounds
@@ -30,8 +31,8 @@ constexpr int CW_NW = 4;
 constexpr int CW_BATCH = 16;  // insertions of one wavefront
 
 // Guests of up to three sites fit 4 wavefronts per SIMD without spilling; larger guests keep
-// the compiler's own register budget.
-template <int NS, bool UPPER>
+// the compiler's own register budget. TAB: the phases come from tables in LDS.
+template <int NS, bool UPPER, bool TAB>
 __global__ __launch_bounds__(64 * CW_NW, (NS <= 3 ? 4 : 1)) void chain_widom_kernel(ChainWidomArgs a, int per)
 {
     __shared__ PairRing rings[CW_NW];
@@ -135,14 +136,21 @@ __global__ __launch_bounds__(64 * CW_NW, (NS <= 3 ? 4 : 1)) void chain_widom_ker
         // (3) reciprocal cross term
         if (G.charged) {
             const int m0 = F.kn_max[0] + 1, m1 = F.kn_max[1] + 1, tw = m0 + m1 + F.kn_max[2] + 1;
-            const float inv_tw = 1.0f / (float)tw;
+            if constexpr (TAB) {
+                const float inv_tw = 1.0f / (float)tw;
 #pragma unroll 1
-            for (int x = lane; x < NS * tw; x += 64) {
-                const int t = (int)(((float)x + 0.5f) * inv_tw), c = x - t * tw;
-                const int d = c < m0 ? 0 : (c < m0 + m1 ? 1 : 2);
-                tab[c * NS + t] = axis_power_const(wf[wv][i][3 * t + d], c - (d == 0 ? 0 : (d == 1 ? m0 : m0 + m1)));
+                for (int x = lane; x < NS * tw; x += 64) {
+                    const int t = (int)(((float)x + 0.5f) * inv_tw), c = x - t * tw;
+                    const int d = c < m0 ? 0 : (c < m0 + m1 ? 1 : 2);
+                    tab[c * NS + t] = axis_power_const(wf[wv][i][3 * t + d], c - (d == 0 ? 0 : (d == 1 ? m0 : m0 + m1)));
+                }
+                fence();
             }
-            fence();
+            // e^{2 pi i m f_d} of site t, the table's row `at` of axis d
+            auto phase = [&](const double2 *at, int d, int m, int t) {
+                if constexpr (TAB) return at[t];
+                else return axis_power_const(wf[wv][i][3 * t + d], m);
+            };
             const int4 *runs = a.kr.run + a.kr.run_off[u];
             const int nruns = a.kr.run_off[u + 1] - a.kr.run_off[u];
             // c = kprefactor S through buffer loads: zero past the end, for lanes without a k-vector
@@ -175,7 +183,7 @@ __global__ __launch_bounds__(64 * CW_NW, (NS <= 3 ? 4 : 1)) void chain_widom_ker
                 for (int j = 2; np > 0; ++j) {
                     double2 z[NS];
 #pragma unroll
-                    for (int t = 0; t < NS; ++t) z[t] = tj[t];
+                    for (int t = 0; t < NS; ++t) z[t] = phase(tj, 2, j - 1, t);
                     tj += NS;
                     pos += np + nm;
                     np = count(2 * j);
@@ -195,7 +203,8 @@ __global__ __launch_bounds__(64 * CW_NW, (NS <= 3 ? 4 : 1)) void chain_widom_ker
                               *tz = tab + (m0 + m1 + abs(run.z)) * NS;
 #pragma unroll
                 for (int t = 0; t < NS; ++t) {
-                    const double2 x = cis_from_axes(tx[t], ty[t], tz[t], run.x, run.y, run.z);
+                    const double2 x = cis_from_axes(phase(tx, 0, abs(run.x), t), phase(ty, 1, abs(run.y), t),
+                                                    phase(tz, 2, abs(run.z), t), run.x, run.y, run.z);
                     acc = __builtin_fma(G.q[t], __builtin_fma(x.x, v1[t], x.y * v2[t]), acc);
                 }
             }
@@ -241,31 +250,33 @@ hipError_t launch_chain_snapshot(const ChainSnap &S, int64_t slot, const McArgs 
 }
 
 template <int NS>
-static void launch_chain_widom_ns(const ChainWidomArgs &a, int per, int nwv, hipStream_t st)
+static void launch_chain_widom_ns(const ChainWidomArgs &a, int per, int nwv, bool tab, hipStream_t st)
 {
     const dim3 grid((unsigned)(((a.nitems + per - 1) / per + nwv - 1) / nwv)), block((unsigned)(64 * nwv));
     const size_t lds = a.guest.charged ? sizeof(double2) * nwv * NS * a.ktab_w : 0;
-    if (a.upper) hipLaunchKernelGGL((chain_widom_kernel<NS, true>), grid, block, lds, st, a, per);
-    else hipLaunchKernelGGL((chain_widom_kernel<NS, false>), grid, block, lds, st, a, per);
+    if (!tab) hipLaunchKernelGGL((chain_widom_kernel<NS, false, false>), grid, block, 0, st, a, per);
+    else if (a.upper) hipLaunchKernelGGL((chain_widom_kernel<NS, true, true>), grid, block, lds, st, a, per);
+    else hipLaunchKernelGGL((chain_widom_kernel<NS, false, true>), grid, block, lds, st, a, per);
 }
 
 hipError_t launch_chain_widom(const ChainWidomArgs &a, hipStream_t st)
 {
     if (a.nitems <= 0) return hipSuccess;
-    // the wavefronts of a workgroup share nothing: one where the phase tables of four would not fit
-    const size_t tab = a.guest.charged ? sizeof(double2) * a.guest.nsites * a.ktab_w : 0;
-    if (tab > 100 * 1024) return hipErrorInvalidValue;
-    const int nwv = CW_NW * tab > 100 * 1024 ? 1 : CW_NW;
+    // the wavefronts of a workgroup share nothing: one where the phase tables of four would not fit, and
+    // no tables where one wavefront's would not (a six-site guest in a cell of 3,300 Å)
+    const size_t bytes = a.guest.charged ? sizeof(double2) * a.guest.nsites * a.ktab_w : 0;
+    const bool tab = bytes <= 100 * 1024;
+    const int nwv = tab && CW_NW * bytes > 100 * 1024 ? 1 : CW_NW;
     // insertions per wavefront: one until there are some 16 wavefronts for every SIMD
     int per = 1;
     while (per < CW_BATCH && a.nitems / (2 * per) >= 16384) per *= 2;
     switch (a.guest.nsites) {
-    case 1: launch_chain_widom_ns<1>(a, per, nwv, st); break;
-    case 2: launch_chain_widom_ns<2>(a, per, nwv, st); break;
-    case 3: launch_chain_widom_ns<3>(a, per, nwv, st); break;
-    case 4: launch_chain_widom_ns<4>(a, per, nwv, st); break;
-    case 5: launch_chain_widom_ns<5>(a, per, nwv, st); break;
-    case 6: launch_chain_widom_ns<6>(a, per, nwv, st); break;
+    case 1: launch_chain_widom_ns<1>(a, per, nwv, tab, st); break;
+    case 2: launch_chain_widom_ns<2>(a, per, nwv, tab, st); break;
+    case 3: launch_chain_widom_ns<3>(a, per, nwv, tab, st); break;
+    case 4: launch_chain_widom_ns<4>(a, per, nwv, tab, st); break;
+    case 5: launch_chain_widom_ns<5>(a, per, nwv, tab, st); break;
+    case 6: launch_chain_widom_ns<6>(a, per, nwv, tab, st); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

@@ -78,3 +78,19 @@ def test_move_variants_of_other_guests(ns):
     assert np.array_equal(fin, np.isfinite(t2[:, 2]))
     assert np.all(np.abs(t1[fin, 2] - t2[fin, 2]) <= 1e-9 * (1 + np.abs(t1[fin, 2])))
     assert i1["occupancy"] == i2["occupancy"] and i1["rng_counter"] == i2["rng_counter"]
+
+
+def test_chain_insertions_into_a_very_long_cell():
+    """A cell of 3,420 Å whose k-vectors' phase tables for six sites (over 100 KB) LDS does not hold: without
+    guests a chain insertion is a Widom insertion (1e-10 as in test_gpu_nvt.py)."""
+    ff = synth.synthetic_forcefield(12.0)
+    g = _guest(ff, 6)
+    fw = synth.synthetic_framework(24.1, 24.2, 3420.0, 90, 90, 90, 3000, 5, charge_sd=0.1)
+    b = pa.FrameworkBatch([fw], ff, g, pa.EwaldParams(12.0, 1e-6), fullk=True)
+    st = pa.SystemState(b, g, [0], T=T, seed=5, capacities=[2])
+    pos, quat = pa.widom_poses(b, 0, 777, 0, 200)
+    dU = pa.widom_chain_energies(st, 0, pos, quat)
+    ref = pa.widom_energies(b, 0, 777, 0, 200, precision="f64")
+    fin = np.isfinite(ref) & (np.abs(ref) < 1e8)
+    assert fin.sum() > 100
+    assert np.all(np.abs(dU[fin] - ref[fin]) <= 1e-10 * (1 + np.abs(ref[fin])))
