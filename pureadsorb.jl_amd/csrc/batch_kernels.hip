@@ -86,13 +86,14 @@ __device__ inline R length2(const R A[9], R x, R y, R z)
 // Phase-0 near lists: for every hard-core cell, the atoms within nbr_r of any point of it, by their
 // minimum-image distance to the cell's centre. One wavefront per cell, its lanes over the cells
 // within nbr_reach (each once where the reach goes around the axis). Without FILL the lists are
-// counted into nbr_start (and their sum added to *sum); with it they are written in three shells of growing distance, so that
-// an insertion's overlap is usually found among the first entries. cell_fw_off (nfw + 1) maps the
-// global cell index to its framework.
+// counted into nbr_start (and their sum added to *sum); with it they are written in shells of growing
+// distance, so that an insertion's overlap is usually found among the first entries and a call of smaller
+// radii stops at the end of the last shell that can hold one, and nbr_range gets the start and those ends.
+// cell_fw_off (nfw + 1) maps the global cell index to its framework.
 template <bool FILL>
 __global__ __launch_bounds__(BK_WG) void nbr_kernel(const FwDesc *fw, int nfw, const int *cell_fw_off, int ncells,
                                                    const int *cell_start, int *nbr_start, const uint4 *corefx,
-                                                   uint4 *nbr_atoms, unsigned long long *sum)
+                                                   uint4 *nbr_atoms, int4 *nbr_range, unsigned long long *sum)
 {
     const int lane = threadIdx.x & 63;
     const int g = blockIdx.x * (BK_WG / 64) + (threadIdx.x >> 6);
@@ -117,10 +118,13 @@ __global__ __launch_bounds__(BK_WG) void nbr_kernel(const FwDesc *fw, int nfw, c
     const int ncand = k[0] * k[1] * k[2];
     const int *cs = cell_start + D.cg_off;
     const uint4 *src = corefx + D.atom_off;
-    const float shell[4] = {-1.0f, 0.36f * D.nbr_thr2, 0.64f * D.nbr_thr2, D.nbr_thr2};
+    constexpr int SHELLS = 2 + NBR_RADII;
     int total = 0;
     const int64_t at0 = FILL ? nbr_start[D.cg_off + c] : 0;
-    for (int sh = 0; sh < (FILL ? 3 : 1); ++sh)
+    int end[SHELLS];
+#pragma unroll
+    for (int sh = FILL ? 0 : SHELLS - 1; sh < SHELLS; ++sh) {
+        const float lo2 = FILL && sh > 0 ? D.nbr_thr2[sh - 1] : -1.0f, hi2 = D.nbr_thr2[sh];
         for (int i0 = 0; i0 < ncand; i0 += 64) {
             const int i = i0 + lane;
             int b0 = 0, len = 0;
@@ -138,13 +142,17 @@ __global__ __launch_bounds__(BK_WG) void nbr_kernel(const FwDesc *fw, int nfw, c
                     at = src[b0 + j];
                     const float r2 = length2(D.Af, (float)(int32_t)(x[0] - at.x), (float)(int32_t)(x[1] - at.y),
                                              (float)(int32_t)(x[2] - at.z));
-                    in = FILL ? r2 > shell[sh] && r2 <= shell[sh + 1] : r2 <= D.nbr_thr2;
+                    in = r2 > lo2 && r2 <= hi2;
                 }
                 const uint64_t m = __builtin_amdgcn_ballot_w64(in);
                 if (FILL && in) nbr_atoms[at0 + total + __popcll(m & ((1ull << lane) - 1ull))] = at;
                 total += __popcll(m);
             }
         }
+        end[sh] = (int)at0 + total;
+    }
+    static_assert(NBR_RADII == 3, "a cell's start and ends are an int4");
+    if (FILL && lane == 0) nbr_range[D.cg_off + c] = make_int4((int)at0, end[2], end[3], end[4]);
     if (!FILL && lane == 0) nbr_start[D.cg_off + c] = total;
     if (!FILL && sum && lane == 0 && total) atomicAdd(sum, (unsigned long long)total);
     // the slot past a framework's last cell: no atoms
@@ -158,16 +166,17 @@ hipError_t scan_counts(int *counts, int n, void *tmp, size_t *tmp_bytes, hipStre
 }
 
 hipError_t launch_nbr(bool fill, const FwDesc *fw, int nfw, const int *cell_fw_off, int ncells, const int *cell_start,
-                      int *nbr_start, const uint4 *corefx, uint4 *nbr_atoms, unsigned long long *sum, hipStream_t st)
+                      int *nbr_start, const uint4 *corefx, uint4 *nbr_atoms, int4 *nbr_range, unsigned long long *sum,
+                      hipStream_t st)
 {
     if (ncells <= 0) return hipSuccess;
     const dim3 grid((unsigned)((ncells + BK_WG / 64 - 1) / (BK_WG / 64))), block(BK_WG);
     if (fill)
         hipLaunchKernelGGL(nbr_kernel<true>, grid, block, 0, st, fw, nfw, cell_fw_off, ncells, cell_start, nbr_start,
-                           corefx, nbr_atoms, sum);
+                           corefx, nbr_atoms, nbr_range, sum);
     else
         hipLaunchKernelGGL(nbr_kernel<false>, grid, block, 0, st, fw, nfw, cell_fw_off, ncells, cell_start, nbr_start,
-                           corefx, nbr_atoms, sum);
+                           corefx, nbr_atoms, nbr_range, sum);
     return hipGetLastError();
 }
 

@@ -8,6 +8,8 @@
 namespace pa {
 
 // Per unique framework (FrameworkBatch's deduplicated per-framework storage).
+constexpr int NBR_RADII = 3;  // radii at which a phase-0 near list can be cut short
+
 struct FwDesc {
     double A[9];       // cell, column-major
     double invA[9];
@@ -19,12 +21,13 @@ struct FwDesc {
     int atom_off, natoms;  // slice of the atom arrays
     int k_off, nk;         // slice of the k tables
     int upper;             // A is upper triangular (cell_matrix's form)
-    int cg_off;            // hard-core cell grid: first entry of the framework in cell_start
+    int cg_off;            // hard-core cell grid: first entry of the framework in cell_start and nbr_range
     int cg_nc[3];          // cells per axis (fractional cell edge 1/cg_nc)
     int kn_max[3];         // largest |n_d| of the framework's k-vectors k = 2 pi A^-T n
-    // phase-0 near lists: each hard-core cell lists every atom within nbr_r (Å) of any point of it,
-    // found by its distance to the cell's centre (nbr_thr2, Å^2) among the cells within nbr_reach
-    float nbr_r, nbr_thr2;
+    // phase-0 near lists: each hard-core cell lists every atom within nbr_r[2] (Å) of any point of it, found
+    // by its distance to the cell's centre among the cells within nbr_reach. In shells of squared
+    // distance nbr_thr2 (Å^2): those up to number 2 + i hold the atoms within nbr_r[i] of any point
+    float nbr_r[NBR_RADII], nbr_thr2[2 + NBR_RADII];
     int nbr_reach[3];
 };
 
@@ -88,11 +91,7 @@ struct BinSys {
     float rlist2;   // (max cutoff + guest radius + bin circumradius + margin)^2, Å^2
     float alt[3];   // an atom with |fractional offset| >= alt[i] on axis i also gets the image
                     // across the cell boundary on that axis (alt >= 0.5: never)
-    int hc_on;      // phase 0 runs: 1 with the cells' near lists, 2 when the largest rejection radius
-                    // exceeds theirs and the insertions they pass go through the full stencil too
-    uint32_t hc_rf[3];  // largest rejection radius over the perpendicular width, 32-bit fixed point
-                        // and rounded up: a site's hard-core partners lie within +-hc_rf[d];
-                        // all ones: that range (plus one cell) reaches around the axis
+    int hc_end;     // phase 0 runs over the cells' near lists up to this end of nbr_range (1..NBR_RADII); 0: no phase 0
     // radial classes of the neighbour list: class 0 holds the atoms closer than cls_d0 to the bin
     // centre, classes 1..BIN_NCLS-1 split [cls_d0, sqrt(rlist2)] into shells of width 1/cls_inv_w
     float cls_d0, cls_inv_w;
@@ -158,15 +157,10 @@ struct BinnedArgs {
     int *extra_passes;         // max over bins of (passes - 1) of this call's energy launches
     int zero_passes;           // nonzero on the call's first chunk: bin_zero_kernel clears it
     GuestDev guest;
-    // hard-core rejection (phase 0): atoms of each framework sorted by grid cell
-    const uint4 *corefx;       // fixed-point x, y, z and compact type, by cell
-    const int *cell_start;     // per framework: cg_nc[0]*cg_nc[1]*cg_nc[2] + 1 offsets
-    const int *nbr_start;      // same layout: each cell's range of nbr_atoms
-    const uint4 *nbr_atoms;    // per cell, the atoms near it (as corefx), nearest to its centre first
-    int full_stencil;          // some system has hc_on == 2: bin_reject_kernel runs
+    // hard-core rejection (phase 0)
+    const int4 *nbr_range;     // per hard-core cell: start of its list in nbr_atoms, and its end for each of nbr_r
+    const uint4 *nbr_atoms;    // per cell, the atoms near it (fixed point and compact type), nearest to its centre first
     const float *rho2;         // nsys x NS x ntypes_c rejection radii^2 (Å^2), rounded down
-    int *cand;                 // chunk-relative insertions left for the full phase-0 stencil
-    int *ncand;                // their count
 };
 
 // Gradient launches (widom_grad.hip): the weighted-insertion list, its per-insertion sites and

@@ -221,7 +221,7 @@ struct pa_batch {
     std::vector<int4> kn_h;    // n of every k-vector of k64_h
     std::vector<double2> S64_h;
     std::vector<int> atype_h;
-    pa::DevAlloc d_corefx, d_coreidx, d_cell_start, d_rho2, d_cand, d_ncand, d_nbr_start, d_nbr_atoms, d_passes;
+    pa::DevAlloc d_corefx, d_coreidx, d_rho2, d_nbr_range, d_nbr_atoms, d_passes;
     pa::DevAlloc d_binfx, d_bintype;  // the atoms in Morton order, as d_nearf, for the mixed path's list build
     // FP64 paths: lists of the atoms near a point, if near_ready (batch_kernels.hip)
     pa::DevAlloc d_nearf, d_near_desc, d_near_start, d_near_ent, d_rho2_64;

@@ -39,7 +39,8 @@ hipError_t grad_select(const double *dU, const int64_t *seg, int nsys, const dou
 hipError_t launch_grad_recip(const GradArgs &a, const double4 *k64, const int4 *rblk, int nrblk, hipStream_t st);
 hipError_t launch_sk(const double4 *atoms, int natoms, const int4 *kreq, int nreq, double2 *out, hipStream_t st);
 hipError_t launch_nbr(bool fill, const FwDesc *fw, int nfw, const int *cell_fw_off, int ncells, const int *cell_start,
-                      int *nbr_start, const uint4 *corefx, uint4 *nbr_atoms, unsigned long long *sum, hipStream_t st);
+                      int *nbr_start, const uint4 *corefx, uint4 *nbr_atoms, int4 *nbr_range, unsigned long long *sum,
+                      hipStream_t st);
 bool near_bins(const pa_batch *b, NearBuild &a, std::vector<NearDesc> &nd, std::vector<int> &bin_fw, std::vector<int> &run_off);
 hipError_t launch_near_runs(const NearBuild &a, hipStream_t st);
 hipError_t launch_near_build(bool fill, const NearBuild &a, hipStream_t st);
@@ -350,11 +351,12 @@ double lj_pair(double r2, double sg, double ep)
     return 4.0 * ep * (x * x - x);
 }
 
-// Edge (Å) of the hard-core grid cells of phase 0, and the temperature (K) whose rejection radii the
-// cells' near lists hold: the radii fall slowly with temperature (as T^-1/12), so lists for 77 K
-// serve every temperature above it and are a tenth longer than room temperature needs.
+// Edge (Å) of the hard-core grid cells of phase 0, and the temperatures (K) whose rejection radii their near
+// lists are cut at. The radii fall slowly as it gets warmer (as (B_s + 749 kT)^-1/12): lists that hold
+// those of 0 K serve every temperature, and a call takes the shells that its own radii need: those of 273 K
+// for adsorption near room temperature, those of 77 K for the cryogenic standard (nitrogen, argon).
 constexpr double HC_CELL = 1.2;
-constexpr double HC_LIST_T = 77.0;
+constexpr double HC_LIST_T[NBR_RADII] = {273.0, 77.0, 0.0};
 
 // pair_energy (src/reject.jl:22): LJ plus K erfc(alpha r)/r with the pair series.
 double pair_energy_h(double r, double sg, double ep, double K, double alpha)
@@ -564,21 +566,23 @@ int add_atoms(BatchTables &T, FwDesc &D, const double *frac, const double *cart,
     return PA_OK;
 }
 
-// The largest phase-0 rejection radius at HC_LIST_T, per framework.
+// The largest phase-0 rejection radius at each of HC_LIST_T, per framework.
 std::vector<double> near_list_radii(const pa_batch *b)
 {
-    std::vector<double> r(b->nfw, -1.0), rho2((size_t)b->nsites * b->ntypes_c);
+    std::vector<double> r((size_t)b->nfw * NBR_RADII, -1.0), rho2((size_t)b->nsites * b->ntypes_c);
     for (int s = 0; s < b->nsys; ++s) {
-        const int u = b->fw_of[s];
-        if (r[u] >= 0.0) continue;
-        double rmax2 = 0.0;
-        if (rejection_radii(b, s, KB * HC_LIST_T, (double)FLT_EPSILON, rho2.data(), &rmax2)) rmax2 = 0.0;
-        r[u] = std::sqrt(rmax2) * (1.0 + 1e-6);
+        double *ru = &r[(size_t)b->fw_of[s] * NBR_RADII];
+        if (ru[0] >= 0.0) continue;
+        for (int i = 0; i < NBR_RADII; ++i) {
+            double rmax2 = 0.0;
+            if (rejection_radii(b, s, KB * HC_LIST_T[i], (double)FLT_EPSILON, rho2.data(), &rmax2)) rmax2 = 0.0;
+            ru[i] = std::max(i ? ru[i - 1] : 0.0, std::sqrt(rmax2) * (1.0 + 1e-6));
+        }
     }
     return r;
 }
 
-// Radius, distance threshold and cell reach of every framework's phase-0 near lists for the radii r.
+// Radii, distance thresholds and cell reach of every framework's phase-0 near lists for the radii r.
 // Returns a bound on their entries: an atom is in the lists of the cells whose centres lie within thr of
 // it, and those cells lie in the sphere of thr and their circumradius.
 double set_near_radii(pa_batch *b, const std::vector<double> &r)
@@ -595,9 +599,15 @@ double set_near_radii(pa_batch *b, const std::vector<double> &r)
                 matvec(D.A, f, v);
                 rc = std::max(rc, norm3(v));
             }
-        const double thr = (r[u] + rc) * (1.0 + 1.0e-5) + 1.0e-3;  // FP32 distances on the device
-        D.nbr_r = std::nextafter((float)r[u], 0.0f);
-        D.nbr_thr2 = (float)(thr * thr);
+        double thr = 0.0;
+        for (int i = 0; i < NBR_RADII; ++i) {
+            const double R = r[(size_t)u * NBR_RADII + i];
+            thr = (R + rc) * (1.0 + 1.0e-5) + 1.0e-3;  // FP32 distances on the device
+            D.nbr_r[i] = std::nextafter((float)R, 0.0f);
+            D.nbr_thr2[2 + i] = (float)(thr * thr);
+        }
+        D.nbr_thr2[0] = 0.36f * D.nbr_thr2[2];
+        D.nbr_thr2[1] = 0.64f * D.nbr_thr2[2];
         for (int d = 0; d < 3; ++d) {
             D.nbr_reach[d] = std::max(1, (int)std::ceil(thr * D.cg_nc[d] / h.perp[d] + 0.5));
             cells *= D.cg_nc[d];
@@ -634,7 +644,6 @@ int upload_batch(pa_batch *b, const BatchTables &T)
     HIP_TRY(upload(b->d_binfx, T.binfx));
     HIP_TRY(upload(b->d_bintype, T.bintype));
     HIP_TRY(upload(b->d_coreidx, T.coreidx));
-    HIP_TRY(upload(b->d_cell_start, T.cell_start));
     HIP_TRY(upload(b->d_nearf, T.nearf));
     HIP_TRY(b->d_rho2_64.ensure(sizeof(double) * (size_t)b->nsys * b->nsites * b->ntypes_c));
     {
@@ -646,22 +655,25 @@ int upload_batch(pa_batch *b, const BatchTables &T)
         const size_t bin_fw_n = ints.size();
         ints.insert(ints.end(), run_off.begin(), run_off.end());
         ints.insert(ints.end(), T.cell_fw_off.begin(), T.cell_fw_off.end());
-        DevAlloc d_ints, d_run, tmp;
+        const size_t cell_fw_n = T.cell_fw_off.size();
+        ints.insert(ints.end(), T.cell_start.begin(), T.cell_start.end());
+        DevAlloc d_ints, d_run, d_start, tmp;
         HIP_TRY(upload(d_ints, ints));
         const int *cell_fw_off = d_ints.as<int>() + bin_fw_n + run_off.size();
         const int n = (int)T.cell_start.size(), ncells = T.cell_fw_off.back();
-        HIP_TRY(b->d_nbr_start.ensure(sizeof(int) * std::max(n, 1)));
-        int *start = b->d_nbr_start.as<int>(), total[2] = {0, 0};
+        HIP_TRY(d_start.ensure(sizeof(int) * std::max(n, 1)));
+        HIP_TRY(b->d_nbr_range.ensure(sizeof(int4) * std::max(n, 1)));
+        int *start = d_start.as<int>(), total[2] = {0, 0};
         auto nbr = [&](bool fill, uint4 *out, unsigned long long *sum) {
-            return launch_nbr(fill, b->d_fw.as<FwDesc>(), b->nfw, cell_fw_off, ncells, b->d_cell_start.as<int>(), start,
-                              b->d_corefx.as<uint4>(), out, sum, b->stream);
+            return launch_nbr(fill, b->d_fw.as<FwDesc>(), b->nfw, cell_fw_off, ncells, cell_fw_off + cell_fw_n, start,
+                              b->d_corefx.as<uint4>(), out, b->d_nbr_range.as<int4>(), sum, b->stream);
         };
         size_t bytes = 0;
         HIP_TRY(scan_counts(start, std::max(n, nb.nbins + 1), nullptr, &bytes, b->stream));
         HIP_TRY(tmp.ensure(bytes));
         // The phase-0 lists' offsets have 31 bits. Where a bound does not settle that (from some ten million
-        // atoms on) the entries are counted, and only lists that really exceed it get smaller radii,
-        // with which phase 0 has to go through the full stencil too.
+        // atoms on) the entries are counted, and only lists that really exceed it get smaller radii:
+        // phase 0 then rejects within those and the energy kernel evaluates the others.
         std::vector<double> r = near_list_radii(b);
         DevAlloc d_sum;
         for (double scale = 1.0;; scale *= 0.8) {
@@ -1465,7 +1477,7 @@ static double bin_scale_rule(const pa_batch *b, const std::vector<double> &n)
 
 // The default cuts a range of n insertions into equal chunks of at most 2^24 (a short last chunk would run
 // the energy kernel on a fraction of the device; each launch ends on a tail of unevenly
-// sized bins, so fewer launches are faster: 52 B of scratch per insertion, 0.9 GB at 2^24);
+// sized bins, so fewer launches are faster: 48 B of scratch per insertion, 0.8 GB at 2^24);
 // an explicit chunk is taken as given.
 static int64_t chunk_size(int64_t n, int64_t chunk)
 {
@@ -1623,8 +1635,7 @@ static int run_energies(pa_batch *b, const std::vector<int64_t> &seg, int64_t gb
         const double d0 = std::max(0.0, rcmax - rb - b->r_guest - 0.05);
         B.cls_d0 = (float)d0;
         B.cls_inv_w = (float)((binned_nclasses() - 1) / std::max(R - d0, 1e-3));
-        B.hc_on = 0;
-        B.hc_rf[0] = B.hc_rf[1] = B.hc_rf[2] = 0u;
+        B.hc_end = 0;
         for (int d = 0; d < 3; ++d) B.alt[d] = (float)std::max(0.0, 1.0 - R / h.perp[d]);
         B.bin_base = base[s];
         base[s + 1] = base[s] + (int)nb;
@@ -1633,7 +1644,6 @@ static int run_energies(pa_batch *b, const std::vector<int64_t> &seg, int64_t gb
     // phase-0 rejection radii for this kT (src/widom.jl:202-253): margin = (theta + 2) kT + safety
     // + B_s - c_s with the FP32 rounding allowance of the mixed path's pair terms
     std::vector<float> rho2((size_t)nsys * b->nsites * b->ntypes_c, 0.0f);
-    bool full_stencil = false;
     if (kT > 0.0) {
         const int NS = b->nsites, NTC = b->ntypes_c;
         if (b->rr_kT != kT) {
@@ -1650,28 +1660,22 @@ static int run_energies(pa_batch *b, const std::vector<int64_t> &seg, int64_t gb
         }
         for (int s = 0; s < nsys; ++s) {
             const double *r2s = b->rr_r2.data() + (size_t)s * NS * NTC;
-            const double rmax2 = b->rr_max2[s];
+            const double rmax = std::sqrt(b->rr_max2[s]);
+            const FwDesc &D = b->desc[b->fw_of[s]];
+            // the lists hold the radii of every temperature unless a batch has too many atoms for them
+            const double rlist2 = (double)D.nbr_r[NBR_RADII - 1] * D.nbr_r[NBR_RADII - 1];
             for (size_t i = 0; i < (size_t)NS * NTC; ++i) {
                 // FP32 radius rounded down with a 1e-5 relative allowance for the device's FP32
                 // distance
-                const double r2 = r2s[i];
+                const double r2 = std::min(r2s[i], rlist2);
                 float f = (float)(r2 * (1.0 - 1.0e-5));
                 if ((double)f > r2 * (1.0 - 1.0e-5)) f = std::nextafter(f, 0.0f);
                 rho2[(size_t)s * NS * NTC + i] = f;
             }
-            const FwHost &h = b->info[b->fw_of[s]];
-            const FwDesc &D = b->desc[b->fw_of[s]];
-            if (rmax2 > 0.0) {
-                bins[s].hc_on = std::sqrt(rmax2) <= (double)D.nbr_r ? 1 : 2;
-                full_stencil = full_stencil || bins[s].hc_on == 2;
-                for (int d = 0; d < 3; ++d) {
-                    bins[s].hc_rf[d] = (uint32_t)std::min(4294967295.0,
-                                                          std::ceil(std::sqrt(rmax2) / h.perp[d] * 4294967296.0) + 2.0);
-                    // +-hc_rf plus one cell reaching around the axis: every cell, marked by the
-                    // all-ones value so that the kernels need no division
-                    const uint64_t rf = bins[s].hc_rf[d], nc = (uint64_t)D.cg_nc[d];
-                    if (2 * rf + ((uint64_t)1 << 32) / nc >= ((uint64_t)1 << 32)) bins[s].hc_rf[d] = 0xFFFFFFFFu;
-                }
+            if (rmax > 0.0) {
+                int e = 1;
+                while (e < NBR_RADII && rmax > (double)D.nbr_r[e - 1]) ++e;
+                bins[s].hc_end = e;
             }
         }
     }
@@ -1722,10 +1726,6 @@ static int run_energies(pa_batch *b, const std::vector<int64_t> &seg, int64_t gb
     A.order = (int *)p;
     SCR_TRY(b, scr.take(b->d_rank, sizeof(int) * chunk_n, &p));
     A.rank = (int *)p;
-    SCR_TRY(b, scr.take(b->d_cand, sizeof(int) * chunk_n, &p));
-    A.cand = (int *)p;
-    SCR_TRY(b, scr.take(b->d_ncand, sizeof(int), &p));
-    A.ncand = (int *)p;
     SCR_TRY(b, scr.take(b->d_passes, sizeof(int), &p));
     A.extra_passes = (int *)p;
     b->passes_recorded = scr.base == nullptr;  // a fixed region's counter is not kept after the call
@@ -1751,12 +1751,9 @@ static int run_energies(pa_batch *b, const std::vector<int64_t> &seg, int64_t gb
     A.rc_max2f = std::max(A.rc_lj2f, A.rc_ew2f);
     A.listcap = listcap;
     A.guest = b->gdev;
-    A.corefx = b->d_corefx.as<uint4>();
-    A.cell_start = b->d_cell_start.as<int>();
-    A.nbr_start = b->d_nbr_start.as<int>();
+    A.nbr_range = b->d_nbr_range.as<int4>();
     A.nbr_atoms = b->d_nbr_atoms.as<uint4>();
     A.rho2 = d_rho2;
-    A.full_stencil = full_stencil;
     for (int64_t g0 = gb; g0 < ge; g0 += CH) {
         A.g0 = g0;
         A.g1 = std::min(ge, g0 + CH);

@@ -79,80 +79,16 @@ __device__ inline void wave_lds_fence()
     __builtin_amdgcn_wave_barrier();
 }
 
-// Grid cells, along one axis with nc cells, that hold the coordinates within +-rf (32-bit fixed
-// point) of x: `cnt` cells from `start` upwards, wrapping. Atoms are binned as (x nc) >> 32. An
-// interval that reaches around the axis (2 rf + 2^32 / nc >= 2^32, decided once per system on the
-// host) comes as rf = all ones and covers every cell.
-__device__ inline void cell_range(uint32_t x, uint32_t rf, int nc, int &start, int &cnt)
-{
-    if (rf == 0xFFFFFFFFu) {
-        start = 0;
-        cnt = nc;
-        return;
-    }
-    const int lo = (int)(((uint64_t)(uint32_t)(x - rf) * (uint64_t)nc) >> 32);
-    const int hi = (int)(((uint64_t)(uint32_t)(x + rf) * (uint64_t)nc) >> 32);
-    const int span = hi >= lo ? hi - lo : hi - lo + nc;
-    start = lo;
-    cnt = min(span + 1, nc);
-}
-
-// Phase-0 test of one insertion (src/widom.jl:99-151): true when some site lies closer than
-// rho_at to an atom of type t (the radii guarantee exp(-dU/kT) == 0.0 in FP64). The atoms come
-// from the hard-core grid cells that hold coordinates within the largest radius of the site,
-// +-rf[d] along each axis (the radius over the perpendicular width bounds the fractional
-// offset), with the exact fixed-point minimum image. Atoms are sorted by cell with c0 fastest,
-// so the stencil's cells of one (c1, c2) row are one contiguous atom range (two when the row
-// wraps): one dependent cell_start lookup per row.
-template <int NS>
-__device__ inline bool stencil_hit(const BinnedArgs &a, const FwDesc &F, int s, const uint32_t (*sp)[3],
-                                   const uint32_t rf[3])
-{
-    const int *cs = a.cell_start + F.cg_off;
-    const uint4 *cat = a.corefx + F.atom_off;
-    const float *rho = a.rho2 + (size_t)s * NS * a.ntypes_c;
-    const int nc[3] = {F.cg_nc[0], F.cg_nc[1], F.cg_nc[2]};
-    int cnt[3], start[3];
-    bool hit = false;
-    for (int t = 0; t < NS && !hit; ++t) {
-        for (int d = 0; d < 3; ++d) cell_range(sp[t][d], rf[d], nc[d], start[d], cnt[d]);
-        // wrapped indices: start + i < 2 nc, so one conditional subtraction replaces the modulo
-        const int a0 = start[0], a1 = start[0] + cnt[0];
-        const int e0 = a1 < nc[0] ? a1 : nc[0], w1 = a1 > nc[0] ? a1 - nc[0] : 0;
-        for (int i2 = 0; i2 < cnt[2] && !hit; ++i2) {
-            int c2 = start[2] + i2;
-            c2 = c2 >= nc[2] ? c2 - nc[2] : c2;
-            for (int i1 = 0; i1 < cnt[1] && !hit; ++i1) {
-                int c1 = start[1] + i1;
-                c1 = c1 >= nc[1] ? c1 - nc[1] : c1;
-                const int row = nc[0] * (c1 + nc[1] * c2);
-                const int j0 = cs[row + a0], j1 = cs[row + e0];
-                const int k0 = cs[row], k1 = cs[row + w1];
-                const int n1 = j1 - j0, ntot = n1 + (k1 - k0);
-                for (int q = 0; q < ntot; ++q) {
-                    const uint4 at = cat[q < n1 ? j0 + q : k0 + (q - n1)];
-                    const float dx = (float)(int32_t)(sp[t][0] - at.x);
-                    const float dy = (float)(int32_t)(sp[t][1] - at.y);
-                    const float dz = (float)(int32_t)(sp[t][2] - at.z);
-                    const float ex = F.Af[0] * dx + F.Af[3] * dy + F.Af[6] * dz;
-                    const float ey = F.Af[1] * dx + F.Af[4] * dy + F.Af[7] * dz;
-                    const float ez = F.Af[2] * dx + F.Af[5] * dy + F.Af[8] * dz;
-                    if (ex * ex + ey * ey + ez * ez < rho[t * a.ntypes_c + (int)at.w]) hit = true;
-                }
-            }
-        }
-    }
-    return hit;
-}
-
-// Pose, bin and phase 0 of every insertion of the chunk. Each site's hard-core cell lists the
-// atoms within the rejection radii of any point of it, nearest first: one contiguous range per
-// site decides. With the atoms of the 27 cells around it instead, half of the insertions into a
-// porous framework went to a second kernel's wider stencil, by a list whose one atomic counter
-// cost 8 ns a wavefront: 1e6 insertions of CO2 into the 2,160-atom hexagonal cell took 199 us here
-// and 148 us there, 63-101 us now (RUBTAK 3x3x3, whose radii fitted the 27 cells, 72 -> 91 us).
-// Only below the temperature that the lists were built for does an insertion that passes go on
-// to bin_reject_kernel.
+// Pose, bin and phase 0 of every insertion of the chunk (src/widom.jl:99-151): an insertion is rejected when
+// some site lies closer than rho_at to an atom of type t (the radii guarantee exp(-dU/kT) == 0.0 in
+// FP64). Each site's hard-core cell lists the atoms within the rejection radii of any point of it,
+// nearest first: one contiguous range per site decides, up to the shell that the call's own
+// radii reach (hc_end). With the atoms of the 27 cells around it instead, half of the insertions into a
+// porous framework went to a second kernel's wider stencil, by a list with one atomic counter: 1e6
+// insertions of CO2 into the 2,160-atom hexagonal cell took 200 us here and 122 us there, 87 us now
+// (RUBTAK 3x3x3, whose radii fitted the 27 cells, 102 + 5 -> 118 us). With lists that ended at the radii of
+// 77 K, colder calls went through that stencil with every insertion that passed: RUBTAK at
+// 50 K 1.51 ms a call, 1.28 now.
 template <int NS>
 __global__ __launch_bounds__(256) void bin_pose_kernel(BinnedArgs a)
 {
@@ -181,9 +117,7 @@ __global__ __launch_bounds__(256) void bin_pose_kernel(BinnedArgs a)
     const int by = min(B.nb[1] - 1, (int)(f[1] * B.nb[1]));
     const int bz = min(B.nb[2] - 1, (int)(f[2] * B.nb[2]));
     const int key = B.bin_base + bx + B.nb[0] * (by + B.nb[1] * bz);
-    bool pending = false;
-    if (B.hc_on) {
-        const int *nbs = a.nbr_start + F.cg_off;
+    if (B.hc_end) {
         const float *rho = a.rho2 + (size_t)s * NS * a.ntypes_c;
         int j0[NS], j1[NS];
 #pragma unroll
@@ -192,8 +126,9 @@ __global__ __launch_bounds__(256) void bin_pose_kernel(BinnedArgs a)
             const int h1 = (int)(((uint64_t)sp[t][1] * (uint64_t)F.cg_nc[1]) >> 32);
             const int h2 = (int)(((uint64_t)sp[t][2] * (uint64_t)F.cg_nc[2]) >> 32);
             const int c = h0 + F.cg_nc[0] * (h1 + F.cg_nc[1] * h2);
-            j0[t] = nbs[c];
-            j1[t] = nbs[c + 1];
+            const int4 range = a.nbr_range[F.cg_off + c];
+            j0[t] = range.x;
+            j1[t] = B.hc_end == 1 ? range.y : B.hc_end == 2 ? range.z : range.w;
         }
         bool hit = false;
 #pragma unroll
@@ -216,47 +151,9 @@ __global__ __launch_bounds__(256) void bin_pose_kernel(BinnedArgs a)
             a.dU[g - a.out_base] = INFINITY;
             return;
         }
-        pending = B.hc_on == 2;
     }
     a.key[g - a.g0] = key;
-    if (!pending) {
-        a.rank[g - a.g0] = atomicAdd(&a.bin_count[key], 1);
-        return;
-    }
-    // wavefront-aggregated append to the candidate list
-    const uint64_t m = __ballot(1);
-    const int lane = (int)(threadIdx.x & 63);
-    const int leader = __ffsll((long long)m) - 1;
-    int base = 0;
-    if (lane == leader) base = atomicAdd(a.ncand, __popcll(m));
-    base = __shfl(base, leader, 64);
-    a.cand[base + __popcll(m & ((1ull << lane) - 1ull))] = (int)(g - a.g0);
-}
-
-// Phase 0 on the full stencil for the candidates the near stencil left (grid-stride over the
-// device-side candidate count): rejected -> key -1 and dU = +inf, else counted in its bin.
-template <int NS>
-__global__ __launch_bounds__(256) void bin_reject_kernel(BinnedArgs a)
-{
-    const int n = *a.ncand;
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-        const int rel = a.cand[i];
-        const int64_t g = a.g0 + rel;
-        const int s = find_sys64(a.seg, a.nsys, g);
-        const FwDesc &F = a.fw[a.fw_of[s]];
-        const BinSys B = a.bins[s];
-        const uint32_t *sf = a.sitefx + (size_t)rel * 3 * NS;
-        uint32_t sp[NS][3];
-#pragma unroll
-        for (int t = 0; t < NS; ++t)
-            for (int d = 0; d < 3; ++d) sp[t][d] = sf[3 * t + d];
-        if (stencil_hit<NS>(a, F, s, sp, B.hc_rf)) {
-            a.key[rel] = -1;
-            a.dU[g - a.out_base] = INFINITY;
-        } else {
-            a.rank[rel] = atomicAdd(&a.bin_count[a.key[rel]], 1);
-        }
-    }
+    a.rank[g - a.g0] = atomicAdd(&a.bin_count[key], 1);
 }
 
 // Launch order of the energy kernel for a grid of at most BIN_ORDER_MAX bins, and the exclusive
@@ -324,7 +221,6 @@ __global__ __launch_bounds__(256) void bin_zero_kernel(BinnedArgs a)
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i <= a.nbins) a.bin_count[i] = 0;
     if (a.bin_perm && a.nbins > BIN_ORDER_MAX && i < a.nbins) a.bin_iota[i] = i;  // the radix sort's values
-    if (i == 0) *a.ncand = 0;
     if (i == 0 && a.zero_passes) *a.extra_passes = 0;
 }
 
@@ -871,10 +767,6 @@ static hipError_t launch_binned_ns(const BinnedArgs &a, bool upper, hipStream_t 
     const int64_t n = a.g1 - a.g0;
     const dim3 g256((unsigned)((n + 255) / 256)), b256(256);
     hipLaunchKernelGGL((bin_pose_kernel<NS>), g256, b256, 0, st, a);
-    if (a.full_stencil) {
-        const dim3 gr((unsigned)std::min<int64_t>((n + 255) / 256, 2048));
-        hipLaunchKernelGGL((bin_reject_kernel<NS>), gr, b256, 0, st, a);
-    }
     return hipGetLastError();
 }
 

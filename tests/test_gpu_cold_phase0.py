@@ -1,5 +1,6 @@
-"""Phase 0 below the temperature that the cells' near lists are built for (77 K), where insertions that the
-lists pass go through the full stencil too (MI355X). Bars as in test_gpu_reject.py: the device
+"""Phase 0 from the coldest call to the warmest (MI355X): the cells' lists hold the rejection radii of 0 K and
+are cut short at those of 77 and 273 K, and calls at and beside those temperatures take one part or
+the other. Bars as in test_gpu_reject.py: the device
 rejects nothing that the oracle's brute-force check does not, and two-phase and single-phase mixed
 results are the same."""
 import numpy as np
@@ -13,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 
 def _system(cell, guest):
-    """hex: cells of 1.2 Å; long: 64 cells of 3.2 Å on one axis (the stencil's cap)."""
+    """hex: cells of 1.2 Å; long: 64 cells of 3.2 Å on one axis (their cap)."""
     ff = synth.synthetic_forcefield(12.0, guest=guest)
     g = synth.co2_guest(ff) if guest == "co2" else synth.ch4_guest(ff)
     if cell == "hex":
@@ -23,7 +24,7 @@ def _system(cell, guest):
     return fw, ff, g, pa.EwaldParams(12.0, 1e-6)
 
 
-@pytest.mark.parametrize("T", [20.0, 50.0, 76.0])
+@pytest.mark.parametrize("T", [1.0, 20.0, 76.0, 77.0, 78.0, 272.0, 273.0, 274.0, 500.0])
 @pytest.mark.parametrize("cell,guest", [("hex", "co2"), ("hex", "ch4"), ("long", "ch4"), ("long", "co2")])
 def test_cold_flags_and_results(cell, guest, T):
     fw, ff, g, ew = _system(cell, guest)
@@ -37,7 +38,9 @@ def test_cold_flags_and_results(cell, guest, T):
     print(f"{cell} {guest} {T} K: device rejects {dev.sum()}, oracle {ref.sum()} of {n}, at 298 K {warm.sum()}", flush=True)
     assert not np.any(dev & ~ref) and dev.sum() >= 0.97 * ref.sum()
     # radii shrink as it gets warmer
-    assert not np.any(warm & ~dev)
+    assert not np.any(warm & ~dev if T < 298.15 else dev & ~warm)
+    if T < 5.0:  # weights overflow Float64
+        return
     kw = dict(T=T, ninsert=50_000, seed=5, nblocks=4)
     assert pa.widom(b, g, **kw) == pa.widom(b, g, **kw, single_phase=True)
     f64 = pa.widom(b, g, **kw, precision="f64")
