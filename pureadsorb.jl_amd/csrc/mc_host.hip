@@ -294,8 +294,6 @@ McArgs base_mc(pa_state *st)
     McArgs a{};
     a.fw = b->d_fw.as<FwDesc>();
     a.fw_of = b->d_fw_of.as<int>();
-    a.atom64 = b->d_atom64.as<double4>();
-    a.atype = b->d_atype.as<int>();
     a.near = near_lists(b);
     a.upper = b->upper_all ? 1 : 0;
     a.kr = k_runs(st);

@@ -22,7 +22,6 @@
 
 namespace pa {
 
-constexpr int MC_RING = 256;           // per-wavefront ring of in-cutoff pairs: up to 63 pending and 3 x 64 new
 constexpr int MC_BATCH = 64;           // attempts whose random part is drawn at once
 
 // Minimum-image squared distance between two points of the cell, minimum_image's operations.
@@ -106,8 +105,7 @@ __global__ __launch_bounds__(SPEC *GNW * 64) void mc_chain_kernel(McArgs a)
 #pragma clang fp contract(off)
     constexpr int GW = 64 * GNW, WG = SPEC * GW, NW = SPEC * GNW;  // work-items and wavefronts
     __shared__ double red[2][NW];
-    __shared__ double ring_r2[NW][MC_RING], ring_qq[NW][MC_RING];
-    __shared__ int ring_code[NW][MC_RING];
+    __shared__ PairRing rings[NW];
     // the round's attempts: type, slot, bin of the new pose's near list, log of the acceptance
     // uniform, cached host energy of the slot, proposed pose, and the sites of the old (0) and the
     // new (1) pose
@@ -423,35 +421,7 @@ __global__ __launch_bounds__(SPEC *GNW * 64) void mc_chain_kernel(McArgs a)
             }
         // real space: the (site, site) pairs inside the cutoff go through the wavefront's ring in
         // LDS and are evaluated 64 at a time, so LJ + erfc run on full wavefronts
-        const double nan = __builtin_nan("");
-        double *qr2 = ring_r2[wid], *qqq = ring_qq[wid];
-        int *qcode = ring_code[wid];
-        unsigned head = 0, tail = 0;
-        auto drain = [&](unsigned cnt, auto &&eval) {
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            if ((unsigned)lane < cnt) {
-                const unsigned i = (head + lane) & (MC_RING - 1);
-                eval(qr2[i], qqq[i], qcode[i]);
-            }
-            head += cnt;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        };
-        auto push = [&](bool in, double x, double y, int code) {
-            const uint64_t mask = __builtin_amdgcn_ballot_w64(in);
-            if (in) {
-                const unsigned below = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
-                                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-                const unsigned i = (tail + below) & (MC_RING - 1);
-                qr2[i] = x;
-                qqq[i] = y;
-                qcode[i] = code;
-            }
-            tail += (unsigned)__popcll(mask);
-        };
+        PairQueue Q(rings[wid], lane);
         // (1) host-guest, the new pose: minimum images in fractional coordinates
         hsum = 0.0;
         auto host_pair = [&](double r2, double qq, int code) {
@@ -459,48 +429,19 @@ __global__ __launch_bounds__(SPEC *GNW * 64) void mc_chain_kernel(McArgs a)
             hsum += cw_pair(r2, p.x, p.y, qq, alpha, a.rc_lj2, a.rc_ew2);
         };
         if (has_new) {
-            const double4 *af = a.near.atomf + F.atom_off;
-            const int bin = __builtin_amdgcn_readfirstlane(at_bin[gi]);
-            const int e0 = a.near.start[bin], ne = a.near.start[bin + 1] - e0;
-            const uint32_t *ent = a.near.ent + e0;
             double f[NS][3], A[9];
 #pragma unroll
             for (int s = 0; s < NS; ++s)
                 for (int d = 0; d < 3; ++d) f[s][d] = at_frac[gi][1][s][d];
             for (int i = 0; i < 9; ++i) A[i] = cA[i];
-            // the next entry and its atom are loaded while the current one is evaluated; a lane
-            // past the list's end takes a NaN position
-            uint32_t en = gt < ne ? ent[gt] : 0u;
-            double4 hn = gt < ne ? af[en & NEAR_INDEX] : make_double4(nan, nan, nan, 0.0);
-#pragma unroll 1
-            for (int jb = gw * 64; jb < ne; jb += GW) {
-                const double4 h = hn;
-                const int ht = (int)(en >> NEAR_TYPE_SHIFT), j = jb + lane + GW;
-                hn = make_double4(nan, nan, nan, 0.0);
-                if (j < ne) {
-                    en = ent[j];
-                    hn = af[en & NEAR_INDEX];
-                }
-                const double qh = KE * h.w;
-                double r2[NS];
-#pragma unroll
-                for (int s = 0; s < NS; ++s) r2[s] = cw_r2_t<UPPER>(A, f[s][0] - h.x, f[s][1] - h.y, f[s][2] - h.z);
-                // three sites at a time, then whole wavefronts of pairs
-#pragma unroll
-                for (int s0 = 0; s0 < NS; s0 += 3) {
-#pragma unroll
-                    for (int s = s0; s < (s0 + 3 < NS ? s0 + 3 : NS); ++s)
-                        push(r2[s] < a.rc_max2, r2[s], g_q[s] * qh, s * a.ntypes_c + ht);
-#pragma unroll 1
-                    while (tail - head >= 64) drain(64, host_pair);
-                }
-            }
-            drain(tail - head, host_pair);
+            near_scan<NS, UPPER>(a.near, F.atom_off, A, __builtin_amdgcn_readfirstlane(at_bin[gi]), f, g_q, a.ntypes_c,
+                                 a.rc_max2, nullptr, Q, host_pair, gw, GNW);
         }
         // (2) guest-guest: the sites of the new pose (added) and of the old one (taken away by a
         // move, counted by a deletion) against every site of the other live guests. Both poses'
         // terms of a (site, other site) pair are taken in one lane: where guests overlap they are
         // large and nearly cancel.
+        const double nan = __builtin_nan("");
         double gsum = 0.0;
         const double sg_old = type <= MOVE_REINSERTION ? -1.0 : 1.0;
         auto guest_pair = [&](double r2n, double r2o, int code) {
@@ -521,13 +462,13 @@ __global__ __launch_bounds__(SPEC *GNW * 64) void mc_chain_kernel(McArgs a)
                 for (int sa = s0; sa < (s0 + 3 < NS ? s0 + 3 : NS); ++sa) {
                     const double r2n = has_new ? mi_r2<UPPER>(cA, cI, at_site[gi][1][sa], pb) : nan;
                     const double r2o = has_old ? mi_r2<UPPER>(cA, cI, at_site[gi][0][sa], pb) : nan;
-                    push(r2n < a.rc_max2 || r2o < a.rc_max2, r2n, r2o, sa * NS + sb);
+                    Q.push(r2n < a.rc_max2 || r2o < a.rc_max2, r2n, r2o, sa * NS + sb);
                 }
 #pragma unroll 1
-                while (tail - head >= 64) drain(64, guest_pair);
+                while (Q.pending() >= 64) Q.drain(64, guest_pair);
             }
         }
-        drain(tail - head, guest_pair);
+        Q.drain(Q.pending(), guest_pair);
         osum = type == MOVE_DELETION ? -gsum : gsum;
     };
 
@@ -743,7 +684,7 @@ hipError_t launch_mc(const McArgs &a, hipStream_t st)
         spec = exchange ? 4 : 2;
         gnw = exchange ? 4 : 8;
         // LDS: tables, sixteen rings of 20-byte pairs, some 8 KB of draws and records
-        if (spec * tab + pairs + (size_t)16 * MC_RING * 20 + 8 * 1024 > 160 * 1024) spec = 1, gnw = 4;
+        if (spec * tab + pairs + 16 * sizeof(PairRing) + 8 * 1024 > 160 * 1024) spec = 1, gnw = 4;
     }
     const size_t lds = spec * tab + pairs;
     switch (ns * 2 + (a.upper ? 1 : 0)) {

@@ -103,7 +103,7 @@ __global__ __launch_bounds__(64 * CW_NW, (NS <= 3 ? 4 : 1)) void chain_widom_ker
             e += cw_pair(r2, p.x * p.x, 4.0 * p.y, qq, alpha, a.rc_lj2, a.rc_ew2);
         };
         // (1) host-guest real space
-        near_scan<NS, UPPER>(a.near, F, bin, f, G.q, a.ntypes_c, a.rc_max2, nullptr, Q, eval);
+        near_scan<NS, UPPER>(a.near, F.atom_off, F.A, bin, f, G.q, a.ntypes_c, a.rc_max2, nullptr, Q, eval);
         // (2) guest-guest real space
         const double4 *gpos = S.pos + slot * S.nslots + gr0, *gquat = S.quat + slot * S.nslots + gr0;
 #pragma unroll 1

@@ -217,11 +217,6 @@ __device__ inline double cw_r2_t(const double A[9], double f0, double f1, double
     return __builtin_fma(m0, m0, __builtin_fma(m1, m1, m2 * m2));
 }
 
-__device__ inline double cw_r2(const double A[9], double f0, double f1, double f2)
-{
-    return cw_r2_t<false>(A, f0, f1, f2);
-}
-
 // 1/x and 1/sqrt(x) of a positive normal x: the hardware's approximation (about 2^-24) and two
 // Newton steps with fused residuals, which leave at most an ulp or two. The compiler's own FP64
 // division and square root add the scaling and fix-up for zeros, subnormals and infinities that
@@ -283,7 +278,8 @@ __device__ inline double poly_even_odd(double x, const P &c)
     return __builtin_fma(o, x, e);
 }
 
-// exp(x) for x in [-700, 1]: x = n ln2 + r with |r| <= ln2 / 2, the Taylor series of exp(r) to
+// exp(x) for x in [-700, 1]: x = n ln2 + r with |r| <= ln2 / 2 (Cody-Waite: ln2 in two parts, so that n
+// times the first is exact), the Taylor series of exp(r) to
 // r^13 (remainder below 5e-18 of the value), scaled by 2^n.
 __device__ inline double exp64_small(double x, PairCoefPtr C)
 {
@@ -513,27 +509,27 @@ __device__ inline int near_bin(const NearDesc &D, const double f[3])
 }
 
 // One wavefront's host-guest pairs inside the cutoff, from the near list of `bin`: the guest's sites
-// at fractional coordinates f, pairs queued as (r^2, KE q_site q_atom, site * ntypes_c + type) and
-// evaluated by `eval`. With rho2 (squared radii by the same code) the first 64 entries, which hold
+// at fractional coordinates f in the cell A, pairs queued as (r^2, KE q_site q_atom, site * ntypes_c + type) and
+// evaluated by `eval`. Several wavefronts share a list as the w-th of nw. With rho2 (squared radii by the same code) the first 64 entries, which hold
 // the atoms close to the bin, are tested first: true if a site lies inside one, with nothing
 // more evaluated.
 template <int NS, bool UPPER, class E>
-__device__ inline bool near_scan(const NearLists &L, const FwDesc &F, int bin, const double (&f)[NS][3],
+__device__ inline bool near_scan(const NearLists &L, int atom_off, const double *A, int bin, const double (&f)[NS][3],
                                  const double *q, int ntypes_c, double rc_max2, const double *rho2, PairQueue &Q,
-                                 E &&eval)
+                                 E &&eval, int w = 0, int nw = 1)
 {
     const double nan = __builtin_nan("");
-    const double4 *af = L.atomf + F.atom_off;
-    const int e0 = L.start[bin], ne = L.start[bin + 1] - e0, lane = Q.lane;
+    const double4 *af = L.atomf + atom_off;
+    const int e0 = L.start[bin], ne = L.start[bin + 1] - e0, lane = Q.lane, j0 = w * 64 + lane;
     const uint32_t *ent = L.ent + e0;
     // the next entry and its atom are loaded while the current one is evaluated; a lane past the
     // list's end takes a NaN position, which is inside nothing
-    uint32_t en = lane < ne ? ent[lane] : 0u;
-    double4 hn = lane < ne ? af[en & NEAR_INDEX] : make_double4(nan, nan, nan, 0.0);
+    uint32_t en = j0 < ne ? ent[j0] : 0u;
+    double4 hn = j0 < ne ? af[en & NEAR_INDEX] : make_double4(nan, nan, nan, 0.0);
 #pragma unroll 1
-    for (int jb = 0; jb < ne; jb += 64) {
+    for (int jb = w * 64; jb < ne; jb += nw * 64) {
         const double4 h = hn;
-        const int ht = (int)(en >> NEAR_TYPE_SHIFT), j = jb + lane + 64;
+        const int ht = (int)(en >> NEAR_TYPE_SHIFT), j = jb + lane + nw * 64;
         hn = make_double4(nan, nan, nan, 0.0);
         if (j < ne) {
             en = ent[j];
@@ -541,7 +537,7 @@ __device__ inline bool near_scan(const NearLists &L, const FwDesc &F, int bin, c
         }
         double r2[NS];
 #pragma unroll
-        for (int s = 0; s < NS; ++s) r2[s] = cw_r2_t<UPPER>(F.A, f[s][0] - h.x, f[s][1] - h.y, f[s][2] - h.z);
+        for (int s = 0; s < NS; ++s) r2[s] = cw_r2_t<UPPER>(A, f[s][0] - h.x, f[s][1] - h.y, f[s][2] - h.z);
         if (rho2 && jb == 0) {
             bool hit = false;
 #pragma unroll
@@ -586,8 +582,6 @@ struct McArgs {
     // framework tables: the FP64 layout with every k-vector (FULLK batch)
     const FwDesc *fw;
     const int *fw_of;
-    const double4 *atom64;
-    const int *atype;
     NearLists near;             // the framework atoms near a pose
     KRuns kr;                   // the k-vectors; Sk is stored in their order
     int ktab_w;                 // max over frameworks of kn_max[0] + kn_max[1] + kn_max[2] + 3

@@ -154,7 +154,7 @@ __global__ __launch_bounds__(64 * WN_WAVES, 4) void widom_near_kernel(WidomArgs 
         double e = 0.0;
         const double alpha = F.alpha, rc_ew2 = CHARGED ? a.rc_ew2 : 0.0;
         const bool out = near_scan<NS, UPPER>(
-            L, F, bin, f, a.guest.q, a.ntypes_c, fmax(a.rc_lj2, rc_ew2),
+            L, F.atom_off, F.A, bin, f, a.guest.q, a.ntypes_c, fmax(a.rc_lj2, rc_ew2),
             rho2 ? rho2 + (size_t)s * NS * a.ntypes_c : nullptr, Q, [&](double r2, double qq, int code) {
                 const double2 p = a.pair64[code];
                 e += cw_pair(r2, p.x * p.x, 4.0 * p.y, qq, alpha, a.rc_lj2, rc_ew2);
