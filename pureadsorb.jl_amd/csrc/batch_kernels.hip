@@ -119,12 +119,8 @@ __global__ __launch_bounds__(BK_WG) void nbr_kernel(const FwDesc *fw, int nfw, c
     const int *cs = cell_start + D.cg_off;
     const uint4 *src = corefx + D.atom_off;
     constexpr int SHELLS = 2 + NBR_RADII;
-    int total = 0;
-    const int64_t at0 = FILL ? nbr_start[D.cg_off + c] : 0;
-    int end[SHELLS];
-#pragma unroll
-    for (int sh = FILL ? 0 : SHELLS - 1; sh < SHELLS; ++sh) {
-        const float lo2 = FILL && sh > 0 ? D.nbr_thr2[sh - 1] : -1.0f, hi2 = D.nbr_thr2[sh];
+    // calls take(atom, its squared distance) for every atom of the cells in reach, one a lane
+    auto each_atom = [&](auto &&take) {
         for (int i0 = 0; i0 < ncand; i0 += 64) {
             const int i = i0 + lane;
             int b0 = 0, len = 0;
@@ -136,23 +132,48 @@ __global__ __launch_bounds__(BK_WG) void nbr_kernel(const FwDesc *fw, int nfw, c
                 len = cs[cc + 1] - b0;
             }
             for (int j = 0; __builtin_amdgcn_ballot_w64(j < len); ++j) {
-                bool in = false;
                 uint4 at = make_uint4(0u, 0u, 0u, 0u);
+                float r2 = INFINITY;
                 if (j < len) {
                     at = src[b0 + j];
-                    const float r2 = length2(D.Af, (float)(int32_t)(x[0] - at.x), (float)(int32_t)(x[1] - at.y),
-                                             (float)(int32_t)(x[2] - at.z));
-                    in = r2 > lo2 && r2 <= hi2;
+                    r2 = length2(D.Af, (float)(int32_t)(x[0] - at.x), (float)(int32_t)(x[1] - at.y),
+                                 (float)(int32_t)(x[2] - at.z));
                 }
-                const uint64_t m = __builtin_amdgcn_ballot_w64(in);
-                if (FILL && in) nbr_atoms[at0 + total + __popcll(m & ((1ull << lane) - 1ull))] = at;
-                total += __popcll(m);
+                take(at, r2);
             }
         }
-        end[sh] = (int)at0 + total;
+    };
+    auto atoms = [&](float r2, int sh) {  // the lanes whose atom is no farther than shell sh
+        return __builtin_amdgcn_ballot_w64(r2 <= D.nbr_thr2[sh]);
+    };
+    int total = 0;
+    if (!FILL) {
+        each_atom([&](const uint4 &, float r2) { total += __popcll(atoms(r2, SHELLS - 1)); });
+    } else {
+        // the shells' sizes, then the atoms into all of them at once
+        const int at0 = nbr_start[D.cg_off + c];
+        int end[SHELLS], pos[SHELLS];
+#pragma unroll
+        for (int sh = 0; sh < SHELLS; ++sh) end[sh] = at0;
+        each_atom([&](const uint4 &, float r2) {
+#pragma unroll
+            for (int sh = 0; sh < SHELLS; ++sh) end[sh] += __popcll(atoms(r2, sh));
+        });
+#pragma unroll
+        for (int sh = 0; sh < SHELLS; ++sh) pos[sh] = sh ? end[sh - 1] : at0;
+        each_atom([&](const uint4 &at, float r2) {
+            uint64_t inner = 0;
+#pragma unroll
+            for (int sh = 0; sh < SHELLS; ++sh) {
+                const uint64_t within = atoms(r2, sh), m = within & ~inner;
+                if ((m >> lane) & 1) nbr_atoms[pos[sh] + __popcll(m & ((1ull << lane) - 1ull))] = at;
+                pos[sh] += __popcll(m);
+                inner = within;
+            }
+        });
+        static_assert(NBR_RADII == 3, "a cell's start and ends are an int4");
+        if (lane == 0) nbr_range[D.cg_off + c] = make_int4(at0, end[2], end[3], end[4]);
     }
-    static_assert(NBR_RADII == 3, "a cell's start and ends are an int4");
-    if (FILL && lane == 0) nbr_range[D.cg_off + c] = make_int4((int)at0, end[2], end[3], end[4]);
     if (!FILL && lane == 0) nbr_start[D.cg_off + c] = total;
     if (!FILL && sum && lane == 0 && total) atomicAdd(sum, (unsigned long long)total);
     // the slot past a framework's last cell: no atoms
@@ -287,40 +308,41 @@ __global__ __launch_bounds__(256) void near_kernel(NearBuild a)
     const double R = __builtin_sqrt(D.r2);
     const double4 *run = a.run + a.run_off[u];
     const int nrun = a.run_off[u + 1] - a.run_off[u];
-    int total = 0;
-    const int at0 = FILL ? a.start[b] : 0;
-    // filled in two sweeps: the atoms close to the bin come first, so that a caller that tests for
-    // overlaps finds them among the first entries
-    for (int cls = 0; cls < (FILL ? 2 : 1); ++cls)
-        for (int q0 = 0; q0 < nrun; q0 += 64) {
-            // 64 runs at once, one per lane: whether an atom of the run can be within R. A run wider than
-            // the 27 images are sure to cover (an offset of up to a whole cell) is taken as it is.
-            bool cand = false;
-            if (q0 + lane < nrun) {
-                const double4 c = run[q0 + lane];
-                const double lim = R + c.w, k = lim / R * (1.0 + 1.0e-9);
-                const double r0 = D.reach[0] * k, r1 = D.reach[1] * k, r2 = D.reach[2] * k;
-                cand = fmax(r0, fmax(r1, r2)) > 1.0 ||
-                       image_dist2(F, c.x - c0, c.y - c1, c.z - c2, r0, r1, r2) <= lim * lim * (1.0 + 1.0e-9);
-            }
-            for (uint64_t todo = __builtin_amdgcn_ballot_w64(cand); todo; todo &= todo - 1) {
-                const int j = (q0 + __builtin_ctzll(todo)) * 64 + lane;
-                bool in = false;
-                if (j < F.natoms) {
-                    const double4 h = a.atomf[F.atom_off + j];
-                    const double best = image_dist2(F, h.x - c0, h.y - c1, h.z - c2, D.reach[0], D.reach[1], D.reach[2]);
-                    in = best <= D.r2 && (!FILL || (best <= D.close2) == (cls == 0));
-                }
-                const uint64_t mask = __builtin_amdgcn_ballot_w64(in);
-                if (FILL && in) {
-                    const int below = __popcll(mask & ((1ull << lane) - 1ull));
-                    a.ent[at0 + total + below] = (uint32_t)j | ((uint32_t)a.atype[F.atom_off + j] << NEAR_TYPE_SHIFT);
-                }
-                total += __popcll(mask);
-            }
+    // the atoms close to the bin come first, so that a caller that tests for overlaps finds them among
+    // the first entries: where the next one of either kind goes, or how many there are
+    int close = FILL ? a.start[b] : 0, others = FILL ? close + a.close[b] : 0;
+    for (int q0 = 0; q0 < nrun; q0 += 64) {
+        // 64 runs at once, one per lane: whether an atom of the run can be within R. A run wider than
+        // the 27 images are sure to cover (an offset of up to a whole cell) is taken as it is.
+        bool cand = false;
+        if (q0 + lane < nrun) {
+            const double4 c = run[q0 + lane];
+            const double lim = R + c.w, k = lim / R * (1.0 + 1.0e-9);
+            const double r0 = D.reach[0] * k, r1 = D.reach[1] * k, r2 = D.reach[2] * k;
+            cand = fmax(r0, fmax(r1, r2)) > 1.0 ||
+                   image_dist2(F, c.x - c0, c.y - c1, c.z - c2, r0, r1, r2) <= lim * lim * (1.0 + 1.0e-9);
         }
+        for (uint64_t todo = __builtin_amdgcn_ballot_w64(cand); todo; todo &= todo - 1) {
+            const int j = (q0 + __builtin_ctzll(todo)) * 64 + lane;
+            double best = INFINITY;
+            if (j < F.natoms) {
+                const double4 h = a.atomf[F.atom_off + j];
+                best = image_dist2(F, h.x - c0, h.y - c1, h.z - c2, D.reach[0], D.reach[1], D.reach[2]);
+            }
+            const bool in = best <= D.r2;
+            const uint64_t mask = __builtin_amdgcn_ballot_w64(in), near = __builtin_amdgcn_ballot_w64(in && best <= D.close2);
+            if (FILL && in) {
+                const uint64_t below = (1ull << lane) - 1ull;
+                const int at = (near >> lane) & 1 ? close + __popcll(near & below) : others + __popcll(mask & ~near & below);
+                a.ent[at] = (uint32_t)j | ((uint32_t)a.atype[F.atom_off + j] << NEAR_TYPE_SHIFT);
+            }
+            close += __popcll(near);
+            others += __popcll(mask & ~near);
+        }
+    }
     if (!FILL && lane == 0) {
-        a.start[b] = total;
+        a.close[b] = close;
+        a.start[b] = close + others;
         if (b + 1 == a.nbins) a.start[b + 1] = 0;  // the slot past the last bin
     }
 }

@@ -494,6 +494,7 @@ struct NearBuild {
     const int *atype;          // in the same order
     double4 *run;              // per run of 64 atoms: centre (fractional), radius (Å)
     int *start;                // nbins + 1: counts (first pass), then offsets
+    int *close;                // nbins: the atoms within close2 among them (first pass)
     uint32_t *ent;             // entries (second pass)
 };
 

@@ -694,7 +694,8 @@ int upload_batch(pa_batch *b, const BatchTables &T)
         if (near) {
             HIP_TRY(upload(b->d_near_desc, nd));
             HIP_TRY(b->d_near_start.ensure(sizeof(int) * ((size_t)nb.nbins + 1)));
-            HIP_TRY(d_run.ensure(sizeof(double4) * (size_t)std::max(nb.nruns, 1)));
+            const size_t run_bytes = sizeof(double4) * (size_t)nb.nruns;
+            HIP_TRY(d_run.ensure(run_bytes + sizeof(int) * (size_t)nb.nbins));
             nb.fw = b->d_fw.as<FwDesc>();
             nb.nd = b->d_near_desc.as<NearDesc>();
             nb.bin_fw = d_ints.as<int>();
@@ -702,6 +703,7 @@ int upload_batch(pa_batch *b, const BatchTables &T)
             nb.atomf = b->d_nearf.as<double4>();
             nb.atype = b->d_bintype.as<int>();
             nb.run = d_run.as<double4>();
+            nb.close = (int *)(d_run.as<char>() + run_bytes);
             nb.start = b->d_near_start.as<int>();
             HIP_TRY(launch_near_runs(nb, b->stream));
             HIP_TRY(launch_near_build(false, nb, b->stream));
