@@ -506,9 +506,10 @@ int add_atoms(BatchTables &T, FwDesc &D, const double *frac, const double *cart,
         std::memcpy(&qb, &qf, 4);
         T.atomfx.push_back(make_uint4(to_fixed(f[0]), to_fixed(f[1]), to_fixed(f[2]), qb));
     }
-    // the mixed path's list build and the FP64 paths' lists read the atoms in Morton order of their fixed-point coordinates
-    // (the top 10 bits per axis, ties by index): a wavefront's 64 atoms then lie close together,
-    // so an image across a cell boundary is either needed by some of them or skipped by all
+    // the mixed path's list build and the FP64 paths' lists read the atoms in Morton order of their
+    // fixed-point coordinates (the top 10 bits per axis, ties by index): a wavefront's 64 atoms then
+    // lie close together, so an image across a cell boundary is either needed by some of them or
+    // skipped by all
     {
         auto spread = [](uint32_t v) {  // the low 10 bits to every third bit
             v = (v | (v << 16)) & 0x030000FF;
@@ -1447,10 +1448,12 @@ constexpr double BIN_TARGET_INSERTIONS = 64.0;
 // with survivors n exp(-15 A^3 density) and B = 4700, C = 450 instruction slots, and 2,048 bins fill
 // and balance the chip. The nearest step to the systems' mean is taken, so that pinning what
 // pa_batch_bin_scale reports repeats a call bit for bit.
-// Widom calls, rule / best of 1, 1.25, 1.5 (us): RUBTAK 1e6 1286 / 1295, 3e5 536 / 541; hexagonal
-// 80-atom cell 1e6 884 / 884, 40-atom cell 1e6 885 / 866; 32 frameworks x 1e5 3254 / 3265. It replaced
-// timing seven multipliers twice on a batch's first long call: that call's 26.0 (RUBTAK 1e6) and
-// 71 ms (32 frameworks) are 1.9 and 4.6 ms now, at the same multipliers up to one step.
+// Widom calls, rule / best of the steps (us): RUBTAK 1e6 1220 / 1212, 5e5 715 / 695, 4e5 622 / 590;
+// hexagonal 80-atom cell 1e6 874 / 850, 40-atom cell 1e6 838 / 807. Over guests of 1 to 6 sites, 12 frameworks and
+// batches and 2.7e5 to 5e6 insertions: 1.023 on average, 1.18 at worst (six sites at 0.09 atoms per Å^3,
+// where hardly one in a hundred survives); the exponent and the constants are CO2's. It replaced
+// timing seven multipliers twice on a batch's first long call: that call's 25.6 (RUBTAK 1e6) and
+// 70 ms (32 frameworks) are 1.7 and 4.1 ms now, at the same multipliers up to one step.
 static const double BIN_SCALE_STEPS[] = {0.75, 1.0, 1.25, 1.5, 1.75, 2.0, 2.5};
 constexpr int64_t BIN_SCALE_LONG = (int64_t)1 << 18;
 static inline double bin_edge_unit(double V, double n)

@@ -215,7 +215,7 @@ __global__ __launch_bounds__(BIN_ORDER_WG) void bin_order_kernel(BinnedArgs a)
     for (int i = tid; i < nb; i += BIN_ORDER_WG) a.bin_perm[atomicAdd(&cursor[order_class(cs[i + 1] - cs[i])], 1)] = i;
 }
 
-// Clears the bin counts (nbins + 1) and the candidate counter of one chunk in one launch.
+// Clears the bin counts (nbins + 1) of one chunk.
 __global__ __launch_bounds__(256) void bin_zero_kernel(BinnedArgs a)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
